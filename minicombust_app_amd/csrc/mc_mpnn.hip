@@ -236,24 +236,66 @@ __global__ void __launch_bounds__(256) k_mm_tn(int n, const float *X1, int ld1, 
     }
 }
 
-// Sum the block partials (fixed order) into the gradient vector: element
-// (k, m) of the KP x MM product goes to wsplit destinations (m < msplit:
-// g[off1 + k * msplit + m], else g[off2 + k * msplit + m - msplit]) for k < K;
-// the column-sum row goes to g[offb + m] when offb >= 0.
-__global__ void k_tn_reduce(const float *partial, int nblocks, int KP, int MM, int K, int msplit, int off1, int off2,
-                            int offb, float *g)
+// Sums the rows of partial[nblocks][C] into the gradient vector, column i to
+// g[dst(i)] (dst(i) < 0: not kept).  A workgroup takes RC adjacent columns
+// with 1024 / RC rows in flight (one row's 8 floats are 32 contiguous bytes),
+// each thread adds its rows in ascending order in FP64 and the row lanes meet
+// in a fixed tree.  One thread per column over all rows, the earlier form, was
+// a serial chain of dependent loads: at 221,184 cells 3.5 ms for the edge
+// weights' 13,824 rows and 53 us for a product's 216, 70% of a gradient; here
+// 23 us and 7 us (the whole gradient 19.6 -> 5.7 ms).
+constexpr int RC = 8, RLANES = 1024 / RC;
+template <class Dst>
+__global__ void __launch_bounds__(1024) k_col_reduce(const float *partial, int nblocks, int C, Dst dst, float *g)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (KP + 1) * MM) return;
-    const int k = i / MM, m = i % MM;
-    if (k < KP && k >= K) return;
-    if (k == KP && offb < 0) return;
-    float s = 0.f;
-    for (int b = 0; b < nblocks; b++) s += partial[(size_t)b * (KP + 1) * MM + i];
-    if (k == KP) g[offb + m] = s;
-    else if (m < msplit) g[off1 + k * msplit + m] = s;
-    else g[off2 + k * msplit + (m - msplit)] = s;
+    __shared__ double acc[RLANES][RC];
+    const int col = threadIdx.x % RC, lane = threadIdx.x / RC;
+    const int i = blockIdx.x * RC + col;
+    double s = 0.0;
+    if (i < C) {
+        int b = lane;
+        for (; b + 3 * RLANES < nblocks; b += 4 * RLANES) {
+            const float v0 = partial[(size_t)b * C + i], v1 = partial[(size_t)(b + RLANES) * C + i];
+            const float v2 = partial[(size_t)(b + 2 * RLANES) * C + i], v3 = partial[(size_t)(b + 3 * RLANES) * C + i];
+            s += (double)v0; s += (double)v1; s += (double)v2; s += (double)v3;
+        }
+        for (; b < nblocks; b += RLANES) s += (double)partial[(size_t)b * C + i];
+    }
+    acc[lane][col] = s;
+    for (int h = RLANES / 2; h > 0; h >>= 1) {
+        __syncthreads();
+        if (lane < h) acc[lane][col] += acc[lane + h][col];
+    }
+    if (lane == 0 && i < C) {
+        const int d = dst(i);
+        if (d >= 0) g[d] = (float)acc[0][col];
+    }
 }
+
+template <class Dst>
+static void col_reduce(hipStream_t s, const float *partial, int nblocks, int C, const Dst &dst, float *g)
+{
+    hipLaunchKernelGGL(k_col_reduce<Dst>, dim3(div_up(C, RC)), dim3(1024), 0, s, partial, nblocks, C, dst, g);
+}
+
+// Element (k, m) of a KP x MM product: m < msplit: off1 + k * msplit + m, else
+// off2 + k * msplit + m - msplit, for k < K; the column-sum row KP: offb + m
+// (not kept when offb < 0).
+struct TnDst {
+    int KP, MM, K, msplit, off1, off2, offb;
+    __device__ int operator()(int i) const
+    {
+        const int k = i / MM, m = i % MM;
+        if (k == KP) return offb < 0 ? -1 : offb + m;
+        if (k >= K) return -1;
+        return m < msplit ? off1 + k * msplit + m : off2 + k * msplit + (m - msplit);
+    }
+};
+// two runs of columns: i < n0 to off0 + i, the rest to off1 + i - n0
+struct RunsDst {
+    int n0, off0, off1;
+    __device__ int operator()(int i) const { return i < n0 ? off0 + i : off1 + i - n0; }
+};
 
 // ------------------------------------------------------------ edges --
 // s_i = sum_j relu(P_i + Q_j + e_ij we + b1); 16 threads per node, 4 channels each
@@ -340,16 +382,6 @@ __global__ void __launch_bounds__(256) k_edge_bwd(int n, const float *PQ, const 
     }
 }
 
-// sum over blocks of the (we, b1) partials into the gradient
-__global__ void k_edge_reduce(const float *partial, int nblocks, int off_we, int off_b1, float *g)
-{
-    const int i = threadIdx.x;   // 128 threads
-    if (i >= 2 * MH) return;
-    float s = 0.f;
-    for (int b = 0; b < nblocks; b++) s += partial[(size_t)b * 2 * MH + i];
-    g[(i < MH) ? off_we + i : off_b1 + i - MH] = s;
-}
-
 // ------------------------------------------------- decoder and loss --
 // y = h wdec + bdec for 64 rows per workgroup: the rows are staged through LDS
 // with coalesced loads, then each row is summed in column order
@@ -407,15 +439,6 @@ __global__ void __launch_bounds__(256) k_decode_bwd(int n, const float *Hf, cons
         for (int q = 0; q < 16; q++) t += s1[q * 16];
         out[MH] = t;
     }
-}
-
-__global__ void k_decode_reduce(const float *partial, int nblocks, float *g)
-{
-    const int i = threadIdx.x;   // MH + 1 threads
-    if (i > MH) return;
-    float s = 0.f;
-    for (int b = 0; b < nblocks; b++) s += partial[(size_t)b * (MH + 1) + i];
-    g[(i < MH) ? OFF_WDEC + i : OFF_BDEC] = s;
 }
 
 // block partials of sum(y)
@@ -1057,8 +1080,7 @@ static void tn(Ctx *c, const float *X1, int ld1, const float *X2, int ld2, const
     const int nb = div_up(n, TN_ROWS);
     hipLaunchKernelGGL((k_mm_tn<K1, K2, KP, MM>), dim3(nb), dim3(256), 0, c->stream, n, X1, ld1, X2, ld2, D, ldd,
                        rowscale, m->partial);
-    hipLaunchKernelGGL(k_tn_reduce, dim3(div_up((KP + 1) * MM, 256)), dim3(256), 0, c->stream, m->partial, nb, KP, MM,
-                       K, msplit, off1, off2, offb, m->g);
+    col_reduce(c->stream, m->partial, nb, (KP + 1) * MM, TnDst{KP, MM, K, msplit, off1, off2, offb}, m->g);
 }
 
 // loss (into sc[4]) and dy for target t
@@ -1082,7 +1104,7 @@ static int backward(Ctx *c, const float *f, const float *e)
     MC_HIP(c, hipMemsetAsync(m->g, 0, NPARAMS * sizeof(float), c->stream));
     const int nb16 = div_up((int64_t)n * 16, 256);
     hipLaunchKernelGGL(k_decode_bwd, dim3(nb16), blk, 0, c->stream, n, m->H[ML], W, m->dy, m->dH, m->partial);
-    hipLaunchKernelGGL(k_decode_reduce, dim3(1), dim3(128), 0, c->stream, m->partial, nb16, m->g);
+    col_reduce(c->stream, m->partial, nb16, MH + 1, RunsDst{MH, OFF_WDEC, OFF_BDEC}, m->g);
     for (int l = ML - 1; l >= 0; l--) {
         const int base = OFF_L0 + l * LSZ;
         const float *Wl = W + base;
@@ -1107,8 +1129,7 @@ static int backward(Ctx *c, const float *f, const float *e)
         // edges
         hipLaunchKernelGGL(k_edge_bwd, dim3(nb16), blk, 0, c->stream, n, m->PQ[l], m->nbr, m->rev, e, Wl + L_WE,
                            Wl + L_B1, m->dS, m->dPQ, m->partial);
-        hipLaunchKernelGGL(k_edge_reduce, dim3(1), dim3(128), 0, c->stream, m->partial, nb16, base + L_WE,
-                           base + L_B1, m->g);
+        col_reduce(c->stream, m->partial, nb16, 2 * MH, RunsDst{MH, base + L_WE, base + L_B1}, m->g);
         // [P | Q] = h [Wa | Wb]
         tn<MH, 0, MH, 2 * MH>(c, m->H[l], MH, nullptr, 0, m->dPQ, 2 * MH, nullptr, MH, MH, base + L_WA, base + L_WB,
                               -1);
