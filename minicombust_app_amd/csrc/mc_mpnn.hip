@@ -57,11 +57,10 @@ constexpr int P_ABT = 0, P_W2T = P_ABT + 2 * MH * MH, P_N1T = P_W2T + MH * MH, P
               P_N2R = P_N1R + 2 * MH * MH, PSZ = P_N2R + MH * MH;
 constexpr int P_ENCT = ML * PSZ, PTOTAL = P_ENCT + MH * 16;
 
-constexpr int TN_ROWS = 1024;   // rows per block of a weight-gradient product
-
 typedef unsigned short bf16_t;
 typedef short short4v __attribute__((ext_vector_type(4)));
 typedef float float4v __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 struct Mpnn {
     int n = 0;
@@ -174,65 +173,124 @@ __global__ void __launch_bounds__(256) k_mm(int n, const float *X1, int ld1, con
     }
 }
 
-// Block partial of G = [X1 | X2]^T D (KP x MM) over rows [b*TN_ROWS, ...),
-// plus row KP = column sums of D (weighted by rowscale when given):
+// Block partial of G = [X1 | X2]^T D (KP x MM) over the block's rows, plus row
+// KP = column sums of D (weighted by rowscale when given):
 // partial[b][(KP + 1) * MM].  MFMA with the row index as the reduction
 // dimension: A[k][r] = X[r][k], B[r][m] = D[r][m].
+// Bound by reading X and D once (FP32).  32 rows at a time go to LDS as BF16
+// in transposed order (column-major, a row pair per word), so every fragment
+// of v_mfma_f32_16x16x32_bf16 (8 consecutive rows of one column) is one
+// 16-byte LDS read and each value leaves memory once; the next 32 rows'
+// 16-byte loads are in flight behind the products.  The earlier kernel took
+// each fragment's rows from memory one float at a time, for every tile again,
+// with one workgroup per 1,024 rows (216 at 221,184 cells, under one per CU).
+// Per product there: 64 x 64 191 -> 24 us, 64 x 128 364 -> 59 us, 128 x 64 315 -> 44 us.
+constexpr int TN_BLOCKS = 1024;     // most workgroups of a product (four per CU)
+constexpr int TN_MIN_ROWS = 128;    // fewest rows per workgroup
+static int tn_blocks(int n) { return std::max(1, std::min(TN_BLOCKS, div_up(n, TN_MIN_ROWS))); }
+
+constexpr int TN_STR = 20;          // words per LDS column: 16 row pairs, padded to stay 16-byte aligned
+
 template <int K1, int K2, int KP, int MM>
 __global__ void __launch_bounds__(256) k_mm_tn(int n, const float *X1, int ld1, const float *X2, int ld2,
                                               const float *D, int ldd, const float *rowscale, float *partial)
 {
-    constexpr int TI = KP / 16, TJ = MM / 16, T = TI * TJ, TPW = (T + 3) / 4;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r0 = blockIdx.x * TN_ROWS, r1 = min(n, r0 + TN_ROWS);
+    static_assert(K1 % 4 == 0 && K2 % 4 == 0 && K1 + K2 <= KP && KP % 16 == 0 && MM % 64 == 0, "shape");
+    constexpr int TI = KP / 16, TJ = MM / 16, T = TI * TJ, TPW = T / 4;
+    constexpr int XG = KP / 4, DG = MM / 4;                  // 4-column groups
+    constexpr int XI = (16 * XG + 255) / 256, DI = 16 * DG / 256;   // (row pair, group) items per thread
+    static_assert(T % 4 == 0 && 256 % DG == 0, "tiles");
+    __shared__ __align__(16) unsigned xs[KP * TN_STR];
+    __shared__ __align__(16) unsigned ds[MM * TN_STR];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nsteps = (n + 31) / 32, per = (nsteps + (int)gridDim.x - 1) / (int)gridDim.x;
+    const int r0 = min(n, (int)blockIdx.x * per * 32), r1 = min(n, r0 + per * 32);
     float *out = partial + (size_t)blockIdx.x * (KP + 1) * MM;
     float4v acc[TPW];
 #pragma unroll
     for (int u = 0; u < TPW; u++) acc[u] = float4v{0.f, 0.f, 0.f, 0.f};
-    const int kq = 4 * (lane >> 4);
-    for (int rr = r0; rr < r1; rr += 16) {
+    float4 cs = make_float4(0.f, 0.f, 0.f, 0.f);   // column sums of this thread's D items (one column group)
+    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 xv[XI][2], dv[DI][2];
+    auto load = [&](int rr) {
+#pragma unroll
+        for (int q = 0; q < XI; q++) {
+            const int it = tid + 256 * q, k = 4 * (it % XG), rp = it / XG;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int r = rr + 2 * rp + h;
+                xv[q][h] = z4;
+                if (rp < 16 && r < r1) {
+                    if (k < K1) xv[q][h] = *(const float4 *)(X1 + (size_t)r * ld1 + k);
+                    else if (k < K1 + K2) xv[q][h] = *(const float4 *)(X2 + (size_t)r * ld2 + (k - K1));
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < DI; q++) {
+            const int it = tid + 256 * q, m = 4 * (it % DG), rp = it / DG;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int r = rr + 2 * rp + h;
+                dv[q][h] = z4;
+                if (r < r1) {
+                    dv[q][h] = *(const float4 *)(D + (size_t)r * ldd + m);
+                    const float sc = rowscale ? rowscale[r] : 1.f;
+                    cs.x += dv[q][h].x * sc; cs.y += dv[q][h].y * sc;
+                    cs.z += dv[q][h].z * sc; cs.w += dv[q][h].w * sc;
+                }
+            }
+        }
+    };
+    auto put = [&](unsigned *t, int col, int rp, const float4 &lo, const float4 &hi) {
+        t[(col + 0) * TN_STR + rp] = (unsigned)to_bf16(lo.x) | ((unsigned)to_bf16(hi.x) << 16);
+        t[(col + 1) * TN_STR + rp] = (unsigned)to_bf16(lo.y) | ((unsigned)to_bf16(hi.y) << 16);
+        t[(col + 2) * TN_STR + rp] = (unsigned)to_bf16(lo.z) | ((unsigned)to_bf16(hi.z) << 16);
+        t[(col + 3) * TN_STR + rp] = (unsigned)to_bf16(lo.w) | ((unsigned)to_bf16(hi.w) << 16);
+    };
+    if (r0 < r1) load(r0);
+    for (int rr = r0; rr < r1; rr += 32) {
+        __syncthreads();   // the previous step's fragments have been read
+#pragma unroll
+        for (int q = 0; q < XI; q++) {
+            const int it = tid + 256 * q;
+            if (it / XG < 16) put(xs, 4 * (it % XG), it / XG, xv[q][0], xv[q][1]);
+        }
+#pragma unroll
+        for (int q = 0; q < DI; q++) {
+            const int it = tid + 256 * q;
+            put(ds, 4 * (it % DG), it / DG, dv[q][0], dv[q][1]);
+        }
+        __syncthreads();
+        if (rr + 32 < r1) load(rr + 32);
+        const int fo = (lane & 15) * TN_STR + 4 * (lane >> 4);   // this lane's column and 8-row run in a tile
 #pragma unroll
         for (int u = 0; u < TPW; u++) {
             const int tile = wave + 4 * u;
-            if (tile >= T) break;
             const int ti = tile / TJ, tj = tile % TJ;
-            const int kcol = ti * 16 + (lane & 15), mcol = tj * 16 + (lane & 15);
-            short4v a, b;
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const int r = rr + kq + t;
-                float xv = 0.f, dv = 0.f;
-                if (r < r1) {
-                    if (kcol < K1) xv = X1[(size_t)r * ld1 + kcol];
-                    else if (kcol < K1 + K2) xv = X2[(size_t)r * ld2 + (kcol - K1)];
-                    dv = D[(size_t)r * ldd + mcol];
-                }
-                a[t] = (short)to_bf16(xv);
-                b[t] = (short)to_bf16(dv);
-            }
-            acc[u] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[u], 0, 0, 0);
+            const bf16x8 a = *(const bf16x8 *)(xs + ti * 16 * TN_STR + fo);
+            const bf16x8 b = *(const bf16x8 *)(ds + tj * 16 * TN_STR + fo);
+            acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[u], 0, 0, 0);
         }
     }
 #pragma unroll
     for (int u = 0; u < TPW; u++) {
         const int tile = wave + 4 * u;
-        if (tile >= T) break;
         const int ti = tile / TJ, tj = tile % TJ;
 #pragma unroll
-        for (int t = 0; t < 4; t++) out[(size_t)(ti * 16 + kq + t) * MM + tj * 16 + (lane & 15)] = acc[u][t];
+        for (int t = 0; t < 4; t++)
+            out[(size_t)(ti * 16 + 4 * (lane >> 4) + t) * MM + tj * 16 + (lane & 15)] = acc[u][t];
     }
-    // column sums in FP32
-    __shared__ float cs[256];
-    constexpr int PER = 256 / MM;
-    const int col = threadIdx.x % MM, part = threadIdx.x / MM;
-    float s = 0.f;
-    for (int r = r0 + part; r < r1; r += PER) s += D[(size_t)r * ldd + col] * (rowscale ? rowscale[r] : 1.f);
-    cs[threadIdx.x] = s;
+    // column sums: the threads of one column group meet in LDS, added in thread order
     __syncthreads();
-    if (threadIdx.x < MM) {
-        float t = 0.f;
-        for (int p = 0; p < PER; p++) t += cs[p * MM + threadIdx.x];
-        out[(size_t)KP * MM + threadIdx.x] = t;
+    float4 *c4 = (float4 *)ds;
+    static_assert(MM * TN_STR * 4 >= 256 * 16, "column sums in the D tile");
+    c4[tid] = cs;
+    __syncthreads();
+    if (tid < DG) {
+        float4 t = z4;
+        for (int p = tid; p < 256; p += DG) { t.x += c4[p].x; t.y += c4[p].y; t.z += c4[p].z; t.w += c4[p].w; }
+        *(float4 *)(out + (size_t)KP * MM + 4 * tid) = t;
     }
 }
 
@@ -509,7 +567,6 @@ __global__ void k_adam(int np, float *w, const float *g, float *m, float *v, flo
 // writes 128 bytes.  Cells go in the assembly kernels' brick order, each
 // XCD's workgroups over one contiguous range of bricks, so a neighbour's
 // activations were read shortly before by the same L2.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // channel at fragment position (ks, g, t) of a 64-channel vector
 __host__ __device__ constexpr int frag_ch(int ks, int g, int t) { return 16 * (2 * ks + (t >> 2)) + 4 * g + (t & 3); }
@@ -987,8 +1044,8 @@ static int ensure_train(Ctx *c)
     }
     MC_TRY(dalloc(c, &m->dH, N * MH)); MC_TRY(dalloc(c, &m->dH2, N * MH)); MC_TRY(dalloc(c, &m->dU, N * MH));
     MC_TRY(dalloc(c, &m->dHA, N * 2 * MH)); MC_TRY(dalloc(c, &m->dS, N * MH)); MC_TRY(dalloc(c, &m->dPQ, N * 2 * MH));
-    const int64_t nb = div_up(N, TN_ROWS);
-    m->partial_cap = std::max<int64_t>(nb * (2 * MH + 1) * 2 * MH, div_up(N * 16, 256) * (2 * MH + 1));
+    // a block partial of the largest products: (2 MH + 1) x MH and (MH + 1) x 2 MH
+    m->partial_cap = std::max<int64_t>((int64_t)tn_blocks((int)N) * (2 * MH + 2) * MH, div_up(N * 16, 256) * 2 * MH);
     MC_TRY(dalloc(c, &m->partial, m->partial_cap));
     m->train_bufs = true;
     return MC_OK;
@@ -1077,7 +1134,7 @@ static void tn(Ctx *c, const float *X1, int ld1, const float *X2, int ld2, const
 {
     Mpnn *m = M(c);
     const int n = m->n;
-    const int nb = div_up(n, TN_ROWS);
+    const int nb = tn_blocks(n);
     hipLaunchKernelGGL((k_mm_tn<K1, K2, KP, MM>), dim3(nb), dim3(256), 0, c->stream, n, X1, ld1, X2, ld2, D, ldd,
                        rowscale, m->partial);
     col_reduce(c->stream, m->partial, nb, (KP + 1) * MM, TnDst{KP, MM, K, msplit, off1, off2, offb}, m->g);
