@@ -76,7 +76,7 @@ struct Mpnn {
     float *deg = nullptr;
     float *f = nullptr, *e = nullptr, *y = nullptr, *dy = nullptr;
     float *H[ML + 1] = {}, *PQ[ML] = {}, *S[ML] = {}, *A[ML] = {}, *U[ML] = {};
-    float *dH = nullptr, *dH2 = nullptr, *dU = nullptr, *dHA = nullptr, *dS = nullptr, *dPQ = nullptr;
+    float *dH = nullptr, *dH2 = nullptr, *dU = nullptr, *dA = nullptr, *dS = nullptr, *dPQ = nullptr;
     float *partial = nullptr;     // block partial products
     int64_t partial_cap = 0;
     double *sc = nullptr;         // device scalars: mean b, s_b, s_d, mean V, loss, ...
@@ -116,59 +116,112 @@ __global__ void k_pack_rows(bf16_t *dst, int ld, int koff, const float *src, int
 }
 
 // ----------------------------------------------------- MFMA products --
-enum { EPI_BIAS = 1, EPI_RELU = 2, EPI_RESID = 4, EPI_MASK = 8, EPI_ROWSCALE = 16 };
+enum { EPI_BIAS = 1, EPI_RELU = 2, EPI_RESID = 4, EPI_MASK = 8, EPI_ROWSCALE = 16, EPI_ADD1 = 32 };
 
 // Y[n x M] = epi([X1 | X2] B): X1 n x K1 (leading dim ld1), X2 n x K2 (ld2),
-// B given as Bt[m * KP + k] (BF16).  One wave computes 16 rows x M columns
-// with M/16 accumulators of v_mfma_f32_16x16x16_bf16:
-//   A fragment: lane l holds A[l % 16][4 (l / 16) + t], t = 0..3
-//   B fragment: lane l holds B[4 (l / 16) + t][l % 16]
-//   result:     lane l holds C[4 (l / 16) + t][l % 16]
+// B given as Bt[m * KP + k] (BF16).  Bound by reading X and writing Y (FP32)
+// once.  The transposed product Y^T = B^T X^T on v_mfma_f32_16x16x32_bf16, so
+// that a lane ends with four adjacent columns of one row (16-byte stores,
+// residual and mask loads):
+//   A fragment: lane l holds Bt[16 j + l % 16][8 (l / 16) + t], t = 0..7
+//   B fragment: lane l holds X[l % 16][8 (l / 16) + t]
+//   result:     lane l holds Y[l % 16][16 j + 4 (l / 16) + t], t = 0..3
+// A wave keeps the weights' fragments in registers over all its 16-row tiles
+// (fetched per tile they were twice the bytes of the tile's own rows) and has
+// the next tile's rows in flight behind the products.
 // Epilogue order: v = acc (+ R) (+ bias * rowscale) (relu) (zero where mask <= 0).
+// EPI_ADD1: columns < M / 2 are added to Y1 (n x M / 2, dense) and not stored in Y.
+// At 221,184 rows, before (K = 16, weights per tile, 4-byte stores) and now:
+// 64 -> 128 72 -> 37 us, 128 -> 64 79 -> 46-53 us, 64 -> 64 38-59 -> 22-37 us.
+constexpr int MM_BLOCKS = 1024;   // most workgroups of a product (four per CU)
+static int mm_blocks(int n) { return std::max(1, std::min(MM_BLOCKS, div_up(n, 64))); }
+
 template <int K1, int K2, int KP, int MM, int EPI>
 __global__ void __launch_bounds__(256) k_mm(int n, const float *X1, int ld1, const float *X2, int ld2,
                                            const bf16_t *Bt, const float *bias, const float *rowscale,
-                                           const float *R, int ldr, const float *mask, int ldm, float *Y, int ldy)
+                                           const float *R, int ldr, const float *mask, int ldm, float *Y, int ldy,
+                                           float *Y1)
 {
-    static_assert(KP % 16 == 0 && MM % 16 == 0 && K1 % 4 == 0 && K2 % 4 == 0 && K1 + K2 <= KP, "shape");
+    static_assert(KP % 16 == 0 && MM % 32 == 0 && K1 % 4 == 0 && K2 % 4 == 0 && K1 + K2 <= KP, "shape");
+    constexpr int KS = (KP + 31) / 32, NJ = MM / 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int row0 = (blockIdx.x * 4 + wave) * 16;
-    if (row0 >= n) return;
-    const int ar = row0 + (lane & 15);
-    const int kq = 4 * (lane >> 4);
-    float4v acc[MM / 16];
+    const int r16 = lane & 15, g = lane >> 4;
+    bf16x8 wf[NJ][KS];
 #pragma unroll
-    for (int j = 0; j < MM / 16; j++) acc[j] = float4v{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NJ; j++)
 #pragma unroll
-    for (int kk = 0; kk < KP / 16; kk++) {
-        const int k = kk * 16 + kq;
-        float4 xv = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (ar < n) {
-            if (k < K1) xv = *(const float4 *)(X1 + (size_t)ar * ld1 + k);
-            else if (k < K1 + K2) xv = *(const float4 *)(X2 + (size_t)ar * ld2 + (k - K1));
+        for (int ks = 0; ks < KS; ks++) {
+            const int k = ks * 32 + 8 * g;
+            bf16x8 z;
+#pragma unroll
+            for (int t = 0; t < 8; t++) z[t] = (__bf16)0.0f;
+            wf[j][ks] = (k < KP) ? *(const bf16x8 *)(Bt + (size_t)(j * 16 + r16) * KP + k) : z;
         }
-        short4v a;
-        a[0] = (short)to_bf16(xv.x); a[1] = (short)to_bf16(xv.y);
-        a[2] = (short)to_bf16(xv.z); a[3] = (short)to_bf16(xv.w);
+    const int ntiles = (n + 15) / 16, stride = 4 * (int)gridDim.x;
+    float4 xv[KS][2];
+    auto load = [&](int tile) {
+        const int row = tile * 16 + r16;
 #pragma unroll
-        for (int j = 0; j < MM / 16; j++) {
-            const short4v b = *(const short4v *)(Bt + (size_t)(j * 16 + (lane & 15)) * KP + k);
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[j], 0, 0, 0);
+        for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int k = ks * 32 + 8 * g + 4 * h;
+                xv[ks][h] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (row < n) {
+                    if (k < K1) xv[ks][h] = *(const float4 *)(X1 + (size_t)row * ld1 + k);
+                    else if (k < K1 + K2) xv[ks][h] = *(const float4 *)(X2 + (size_t)row * ld2 + (k - K1));
+                }
+            }
+    };
+    int tile = (int)blockIdx.x * 4 + wave;
+    if (tile < ntiles) load(tile);
+    for (; tile < ntiles; tile += stride) {
+        bf16x8 xb[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const float4 lo = xv[ks][0], hi = xv[ks][1];
+            xb[ks][0] = (__bf16)lo.x; xb[ks][1] = (__bf16)lo.y; xb[ks][2] = (__bf16)lo.z; xb[ks][3] = (__bf16)lo.w;
+            xb[ks][4] = (__bf16)hi.x; xb[ks][5] = (__bf16)hi.y; xb[ks][6] = (__bf16)hi.z; xb[ks][7] = (__bf16)hi.w;
         }
-    }
+        if (tile + stride < ntiles) load(tile + stride);
+        const int row = tile * 16 + r16;
 #pragma unroll
-    for (int j = 0; j < MM / 16; j++) {
-        const int col = j * 16 + (lane & 15);
+        for (int j = 0; j < NJ; j++) {
+            float4v acc = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int row = row0 + kq + t;
+            for (int ks = 0; ks < KS; ks++)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][ks], xb[ks], acc, 0, 0, 0);
             if (row >= n) continue;
-            float v = acc[j][t];
-            if (EPI & EPI_RESID) v = R[(size_t)row * ldr + col] + v;
-            if (EPI & EPI_BIAS) v += (EPI & EPI_ROWSCALE) ? bias[col] * rowscale[row] : bias[col];
-            if (EPI & EPI_RELU) v = fmaxf(v, 0.f);
-            if (EPI & EPI_MASK) v = (mask[(size_t)row * ldm + col] > 0.f) ? v : 0.f;
-            Y[(size_t)row * ldy + col] = v;
+            const int col = j * 16 + 4 * g;
+            float4 v = make_float4(acc[0], acc[1], acc[2], acc[3]);
+            if constexpr (EPI & EPI_RESID) {
+                const float4 q = *(const float4 *)(R + (size_t)row * ldr + col);
+                v.x = q.x + v.x; v.y = q.y + v.y; v.z = q.z + v.z; v.w = q.w + v.w;
+            }
+            if constexpr (EPI & EPI_BIAS) {
+                const float4 q = *(const float4 *)(bias + col);
+                const float sc = (EPI & EPI_ROWSCALE) ? rowscale[row] : 1.f;
+                v.x += q.x * sc; v.y += q.y * sc; v.z += q.z * sc; v.w += q.w * sc;
+            }
+            if constexpr (EPI & EPI_RELU) {
+                v.x = fmaxf(v.x, 0.f); v.y = fmaxf(v.y, 0.f); v.z = fmaxf(v.z, 0.f); v.w = fmaxf(v.w, 0.f);
+            }
+            if constexpr (EPI & EPI_MASK) {
+                const float4 q = *(const float4 *)(mask + (size_t)row * ldm + col);
+                v.x = q.x > 0.f ? v.x : 0.f; v.y = q.y > 0.f ? v.y : 0.f;
+                v.z = q.z > 0.f ? v.z : 0.f; v.w = q.w > 0.f ? v.w : 0.f;
+            }
+            if constexpr (EPI & EPI_ADD1) {
+                if (j < NJ / 2) {
+                    float4 *d = (float4 *)(Y1 + (size_t)row * (MM / 2) + col);
+                    const float4 q = *d;
+                    *d = make_float4(q.x + v.x, q.y + v.y, q.z + v.z, q.w + v.w);
+                } else {
+                    *(float4 *)(Y + (size_t)row * ldy + col - MM / 2) = v;
+                }
+            } else {
+                *(float4 *)(Y + (size_t)row * ldy + col) = v;
+            }
         }
     }
 }
@@ -523,15 +576,6 @@ __global__ void __launch_bounds__(256) k_loss(int n, const float *y, const float
         acc[0] += (double)d * (double)d;
     }
     block_partials<1>(acc, partials, blockIdx.x, gridDim.x);
-}
-
-// residual add of a column block: dst[i][c] += src[i * lds + c]
-__global__ void k_add_block(int n, float *dst, const float *src, int lds)
-{
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n * MH) return;
-    const int i = idx / MH, c = idx % MH;
-    dst[idx] += src[(size_t)i * lds + c];
 }
 
 // Adam (Kingma & Ba), FP32 master weights
@@ -1043,7 +1087,7 @@ static int ensure_train(Ctx *c)
         MC_TRY(dalloc(c, &m->A[l], N * MH)); MC_TRY(dalloc(c, &m->U[l], N * MH));
     }
     MC_TRY(dalloc(c, &m->dH, N * MH)); MC_TRY(dalloc(c, &m->dH2, N * MH)); MC_TRY(dalloc(c, &m->dU, N * MH));
-    MC_TRY(dalloc(c, &m->dHA, N * 2 * MH)); MC_TRY(dalloc(c, &m->dS, N * MH)); MC_TRY(dalloc(c, &m->dPQ, N * 2 * MH));
+    MC_TRY(dalloc(c, &m->dA, N * MH)); MC_TRY(dalloc(c, &m->dS, N * MH)); MC_TRY(dalloc(c, &m->dPQ, N * 2 * MH));
     // a block partial of the largest products: (2 MH + 1) x MH and (MH + 1) x 2 MH
     m->partial_cap = std::max<int64_t>((int64_t)tn_blocks((int)N) * (2 * MH + 2) * MH, div_up(N * 16, 256) * 2 * MH);
     MC_TRY(dalloc(c, &m->partial, m->partial_cap));
@@ -1057,29 +1101,29 @@ static void forward_train(Ctx *c, const float *f, const float *e)
 {
     Mpnn *m = M(c);
     const int n = m->n;
-    const dim3 gmm(div_up(n, 64)), blk(256);
+    const dim3 gmm(mm_blocks(n)), blk(256);
     const float *W = m->w;
     hipLaunchKernelGGL((k_mm<MFIN, 0, 16, MH, EPI_BIAS | EPI_RELU>), gmm, blk, 0, c->stream, n, f, MFIN,
                        (const float *)nullptr, 0, m->wb + P_ENCT, W + OFF_BENC, (const float *)nullptr,
-                       (const float *)nullptr, 0, (const float *)nullptr, 0, m->H[0], MH);
+                       (const float *)nullptr, 0, (const float *)nullptr, 0, m->H[0], MH, (float *)nullptr);
     for (int l = 0; l < ML; l++) {
         const float *Wl = W + OFF_L0 + l * LSZ;
         const bf16_t *Pk = m->wb + l * PSZ;
         float *hin = m->H[l], *hout = m->H[l + 1];
         hipLaunchKernelGGL((k_mm<MH, 0, MH, 2 * MH, 0>), gmm, blk, 0, c->stream, n, hin, MH, (const float *)nullptr, 0,
                            Pk + P_ABT, (const float *)nullptr, (const float *)nullptr, (const float *)nullptr, 0,
-                           (const float *)nullptr, 0, m->PQ[l], 2 * MH);
+                           (const float *)nullptr, 0, m->PQ[l], 2 * MH, (float *)nullptr);
         hipLaunchKernelGGL(k_edge_fwd, dim3(div_up((int64_t)n * 16, 256)), blk, 0, c->stream, n, m->PQ[l], m->nbr, e,
                            Wl + L_WE, Wl + L_B1, m->S[l]);
         hipLaunchKernelGGL((k_mm<MH, 0, MH, MH, EPI_BIAS | EPI_ROWSCALE>), gmm, blk, 0, c->stream, n, m->S[l], MH,
                            (const float *)nullptr, 0, Pk + P_W2T, Wl + L_B2, m->deg, (const float *)nullptr, 0,
-                           (const float *)nullptr, 0, m->A[l], MH);
+                           (const float *)nullptr, 0, m->A[l], MH, (float *)nullptr);
         hipLaunchKernelGGL((k_mm<MH, MH, 2 * MH, MH, EPI_BIAS | EPI_RELU>), gmm, blk, 0, c->stream, n, hin, MH, m->A[l],
                            MH, Pk + P_N1T, Wl + L_BN1, (const float *)nullptr, (const float *)nullptr, 0,
-                           (const float *)nullptr, 0, m->U[l], MH);
+                           (const float *)nullptr, 0, m->U[l], MH, (float *)nullptr);
         hipLaunchKernelGGL((k_mm<MH, 0, MH, MH, EPI_RESID | EPI_BIAS>), gmm, blk, 0, c->stream, n, m->U[l], MH,
                            (const float *)nullptr, 0, Pk + P_N2T, Wl + L_BN2, (const float *)nullptr, hin, MH,
-                           (const float *)nullptr, 0, hout, MH);
+                           (const float *)nullptr, 0, hout, MH, (float *)nullptr);
     }
     hipLaunchKernelGGL(k_decode, dim3(div_up(n, 64)), blk, 0, c->stream, n, m->H[ML], W, m->y);
 }
@@ -1156,7 +1200,7 @@ static int backward(Ctx *c, const float *f, const float *e)
 {
     Mpnn *m = M(c);
     const int n = m->n;
-    const dim3 gmm(div_up(n, 64)), blk(256);
+    const dim3 gmm(mm_blocks(n)), blk(256);
     const float *W = m->w;
     MC_HIP(c, hipMemsetAsync(m->g, 0, NPARAMS * sizeof(float), c->stream));
     const int nb16 = div_up((int64_t)n * 16, 256);
@@ -1170,19 +1214,20 @@ static int backward(Ctx *c, const float *f, const float *e)
         tn<MH, 0, MH, MH>(c, m->U[l], MH, nullptr, 0, m->dH, MH, nullptr, MH, MH, base + L_WN2, 0, base + L_BN2);
         hipLaunchKernelGGL((k_mm<MH, 0, MH, MH, EPI_MASK>), gmm, blk, 0, c->stream, n, m->dH, MH,
                            (const float *)nullptr, 0, Pk + P_N2R, (const float *)nullptr, (const float *)nullptr,
-                           (const float *)nullptr, 0, m->U[l], MH, m->dU, MH);
+                           (const float *)nullptr, 0, m->U[l], MH, m->dU, MH, (float *)nullptr);
         // u = relu([h, a] Wn1 + bn1)
         tn<MH, MH, 2 * MH, MH>(c, m->H[l], MH, m->A[l], MH, m->dU, MH, nullptr, 2 * MH, MH, base + L_WN1, 0,
                                base + L_BN1);
-        hipLaunchKernelGGL((k_mm<MH, 0, MH, 2 * MH, 0>), gmm, blk, 0, c->stream, n, m->dU, MH, (const float *)nullptr,
-                           0, Pk + P_N1R, (const float *)nullptr, (const float *)nullptr, (const float *)nullptr, 0,
-                           (const float *)nullptr, 0, m->dHA, 2 * MH);
+        // the h half of d[h, a] joins dH (h' = h + ...), the a half is kept
+        hipLaunchKernelGGL((k_mm<MH, 0, MH, 2 * MH, EPI_ADD1>), gmm, blk, 0, c->stream, n, m->dU, MH,
+                           (const float *)nullptr, 0, Pk + P_N1R, (const float *)nullptr, (const float *)nullptr,
+                           (const float *)nullptr, 0, (const float *)nullptr, 0, m->dA, MH, m->dH);
         // a = s W2 + deg b2
-        tn<MH, 0, MH, MH>(c, m->S[l], MH, nullptr, 0, m->dHA + MH, 2 * MH, m->deg, MH, MH, base + L_W2, 0,
+        tn<MH, 0, MH, MH>(c, m->S[l], MH, nullptr, 0, m->dA, MH, m->deg, MH, MH, base + L_W2, 0,
                           base + L_B2);
-        hipLaunchKernelGGL((k_mm<MH, 0, MH, MH, 0>), gmm, blk, 0, c->stream, n, m->dHA + MH, 2 * MH,
+        hipLaunchKernelGGL((k_mm<MH, 0, MH, MH, 0>), gmm, blk, 0, c->stream, n, m->dA, MH,
                            (const float *)nullptr, 0, Pk + P_W2R, (const float *)nullptr, (const float *)nullptr,
-                           (const float *)nullptr, 0, (const float *)nullptr, 0, m->dS, MH);
+                           (const float *)nullptr, 0, (const float *)nullptr, 0, m->dS, MH, (float *)nullptr);
         // edges
         hipLaunchKernelGGL(k_edge_bwd, dim3(nb16), blk, 0, c->stream, n, m->PQ[l], m->nbr, m->rev, e, Wl + L_WE,
                            Wl + L_B1, m->dS, m->dPQ, m->partial);
@@ -1190,16 +1235,14 @@ static int backward(Ctx *c, const float *f, const float *e)
         // [P | Q] = h [Wa | Wb]
         tn<MH, 0, MH, 2 * MH>(c, m->H[l], MH, nullptr, 0, m->dPQ, 2 * MH, nullptr, MH, MH, base + L_WA, base + L_WB,
                               -1);
-        hipLaunchKernelGGL(k_add_block, dim3(div_up((int64_t)n * MH, 256)), blk, 0, c->stream, n, m->dH, m->dHA,
-                           2 * MH);
         if (l > 0) {
             hipLaunchKernelGGL((k_mm<2 * MH, 0, 2 * MH, MH, EPI_RESID>), gmm, blk, 0, c->stream, n, m->dPQ, 2 * MH,
                                (const float *)nullptr, 0, Pk + P_ABR, (const float *)nullptr, (const float *)nullptr,
-                               m->dH, MH, (const float *)nullptr, 0, m->dH2, MH);
+                               m->dH, MH, (const float *)nullptr, 0, m->dH2, MH, (float *)nullptr);
         } else {   // into the encoder: mask by its ReLU
             hipLaunchKernelGGL((k_mm<2 * MH, 0, 2 * MH, MH, EPI_RESID | EPI_MASK>), gmm, blk, 0, c->stream, n, m->dPQ,
                                2 * MH, (const float *)nullptr, 0, Pk + P_ABR, (const float *)nullptr,
-                               (const float *)nullptr, m->dH, MH, m->H[0], MH, m->dH2, MH);
+                               (const float *)nullptr, m->dH, MH, m->H[0], MH, m->dH2, MH, (float *)nullptr);
         }
         std::swap(m->dH, m->dH2);
     }
