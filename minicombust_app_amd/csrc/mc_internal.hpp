@@ -64,6 +64,11 @@ struct AmgLevel {
     // V-cycle's smoothing sweeps and residual
     _Float16 *hoff = nullptr;
     float *diag32 = nullptr;
+    // box level (bx > 0: bx x by x bz cells, x fastest, 7 diagonals): the next
+    // level halves the directions whose shift is 1 (rounded up), so aggregates,
+    // members and the Galerkin sums are arithmetic and need no index arrays
+    int bx = 0, by = 0, bz = 0;
+    int sx = 0, sy = 0, sz = 0;
     // aggregation to the next level
     int nc = 0;
     int *agg = nullptr;                       // [n] aggregate id
@@ -157,6 +162,7 @@ struct Ctx {
     int fine_nd = 0;               // diagonal copy of the fine pattern (0: CSR kernels)
     int fine_off[DIA_MAX] = {};
     int *fine_map = nullptr;
+    int box_nx = 0, box_ny = 0, box_nz = 0;   // the pattern is a box's 7-point coupling (0: it is not)
     double *A_dia = nullptr;       // momentum / scalar matrix in diagonal storage; with a diagonal
                                    // pattern the assembly kernels write it directly (A_vals unused)
     double *A_dia2 = nullptr;      // the same for the temperature matrix (A_vals2)

@@ -1,0 +1,55 @@
+"""GPU tests of the pressure solve's box hierarchy (halved box levels, taken by
+solves to 1e-9 and below without the limiter) at sizes whose lengths leave
+remainders: odd at the fine level, odd further down, one level only, levels
+that fit the single-workgroup tail and levels that do not.
+
+The residual is formed by numpy from the library's own matrix.  Its bound: the
+solve stops at 1e-10 of the right-hand side by the PCG's recursion (FP64) or
+by the refinement's FP64 residual; the recursion leaves the true residual by
+rounding alone, some hundred units of 1e-16 over these iteration counts, so 1 %
+on top of 1e-10 holds both."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from minicombust_app_amd import mcflow as mc
+from tests.helpers import assert_bits
+
+pytestmark = pytest.mark.gpu
+
+
+def _context(m, psolve, **kw):
+    g = mc.Context(m, mode=mc.MODE_SIMPLE, psolve=psolve, p_rtol=1e-10, **kw)
+    rng = np.random.default_rng(m)
+    g.set(mc.ARR_AU, np.concatenate([10.0 * np.exp(0.5 * rng.standard_normal(g.N)), np.zeros(6)]))
+    g.pressure_assemble()
+    b = rng.standard_normal(g.N)
+    return g, b - b.mean()
+
+
+@pytest.mark.parametrize("psolve", [mc.PSOLVE_FP64, mc.PSOLVE_MIXED])
+@pytest.mark.parametrize("m", [3, 5, 7, 9, 11, 17, 21, 32])
+def test_box_hierarchy_solves(m, psolve):
+    print("box hierarchy m=%d psolve=%d" % (m, psolve), flush=True)
+    g, b = _context(m, psolve)
+    with g:
+        A = sp.csr_matrix((g.get(mc.ARR_PA_VALS), g.get(mc.ARR_COL), g.get(mc.ARR_ROW_PTR)), shape=(g.N, g.N))
+        x, st = g.solve_pressure(b)
+        assert st.converged
+        assert np.linalg.norm(b - A @ x) <= 1.01e-10 * np.linalg.norm(b)
+        assert abs(x.mean()) <= 1e-12 * np.abs(x).max()
+
+
+@pytest.mark.parametrize("psolve", [mc.PSOLVE_FP64, mc.PSOLVE_MIXED])
+@pytest.mark.parametrize("m", [9, 11, 17, 23])
+def test_box_tail_is_the_same_cycle(m, psolve):
+    print("box tail m=%d psolve=%d" % (m, psolve), flush=True)
+    out = {}
+    for tail in (0, 1):
+        g, b = _context(m, psolve, amg_tail=tail)
+        with g:
+            x, st = g.solve_pressure(b)
+            assert st.converged
+            out[tail] = (x.copy(), st.iterations)
+    assert out[0][1] == out[1][1]
+    assert_bits(out[1][0], out[0][0], "pressure correction, tail vs per-pass launches")
