@@ -618,11 +618,28 @@ __global__ void __launch_bounds__(256) k_outlet_sums(Geo g, const int *bfaces, i
     const int b = blockIdx.x;
     const int i0 = b * chunk, i1 = min(Fb, i0 + chunk);
     double v[3] = {0.0, 0.0, 0.0};
-    for (int i = i0 + (int)threadIdx.x; i < i1; i += 256) {
-        const int f = bfaces[i];
-        const int bt = g.btype[g.fc1[f] - g.N];
-        if (bt == INLET) v[0] += mflux[f];
-        else if (bt == OUTLET) { v[1] += mflux[f]; v[2] += g.farea[f]; }
+    // eight faces per trip: their three dependent loads (face, side, flux and
+    // area) are three round trips a trip, not a face; each thread adds its
+    // faces in ascending order as before (14 -> 7 us at modifier 20)
+    for (int ib = i0 + (int)threadIdx.x; ib < i1; ib += 8 * 256) {
+        int f[8], bt[8];
+        double mf[8], ar[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) f[q] = ib + 256 * q < i1 ? bfaces[ib + 256 * q] : -1;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const int ff = f[q] < 0 ? 0 : f[q];
+            bt[q] = f[q] < 0 ? -1 : g.fc1[ff] - g.N;
+            mf[q] = mflux[ff];
+            ar[q] = g.farea[ff];
+        }
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            if (bt[q] < 0) continue;
+            const int t = g.btype[bt[q]];
+            if (t == INLET) v[0] += mf[q];
+            else if (t == OUTLET) { v[1] += mf[q]; v[2] += ar[q]; }
+        }
     }
     block_partials<3>(v, partials, b, gridDim.x);
 }
@@ -1755,20 +1772,28 @@ __global__ void __launch_bounds__(256) k_neg_count(int n, const double *v, int r
 // in place: counts -> exclusive offsets; *total = the sum
 __global__ void __launch_bounds__(1024) k_neg_scan(int nb, int *bcount, int *total)
 {
-    __shared__ int part[1024];
+    // waves scan their own sums by lane exchange, wave 0 the 16 wave totals (one
+    // thread over all 1,024 sums took 10 us)
+    __shared__ int wtot[16];
     const int t = threadIdx.x, per = (nb + 1023) / 1024;
+    const int lane = t & 63, wave = t >> 6;
     const int i0 = min(nb, t * per), i1 = min(nb, i0 + per);
     int s = 0;
     for (int i = i0; i < i1; i++) s += bcount[i];
-    part[t] = s;
-    __syncthreads();
-    if (t == 0) {
-        int run = 0;
-        for (int k = 0; k < 1024; k++) { const int x = part[k]; part[k] = run; run += x; }
-        *total = run;
+    int inc = s;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(inc, d, 64);
+        if (lane >= d) inc += o;
     }
+    if (lane == 63) wtot[wave] = inc;
     __syncthreads();
-    int run = part[t];
+    int before = 0, all = 0;
+    for (int w = 0; w < 16; w++) {
+        if (w < wave) before += wtot[w];
+        all += wtot[w];
+    }
+    if (t == 0) *total = all;
+    int run = before + inc - s;
     for (int i = i0; i < i1; i++) { const int x = bcount[i]; bcount[i] = run; run += x; }
 }
 

@@ -368,32 +368,69 @@ inline CellWalk cell_walk(const Ctx *c)
     return w;
 }
 
-// Block-wide sum of NV values over W waves (blockDim.x == 64 W), result valid
-// in thread 0; the wave sums are added in wave order.
-template <int NV, int W = 4>
-__device__ __forceinline__ void block_sum(double (&v)[NV], double *lds /* NV*W */)
+// Sums over the lanes of a wave, every lane receiving it: the pairs (i, i ^ 32),
+// then (i, i ^ 16), ... of a shuffle tree, exchanged in the vector unit
+// (permlane swaps between the halves and rows, rotations within a row of 16)
+// rather than through LDS: a double's exchange is two moves where a shuffle is
+// two LDS round trips, and the finishing kernels' 9 and 12 sums are chains of
+// six of them.
+__device__ __forceinline__ double wave_sum(double x)
 {
+    {
+        const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(x), __double2loint(x), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(x), __double2hiint(x), false, false);
+        x = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+    }
+    {
+        const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(x), __double2loint(x), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(x), __double2hiint(x), false, false);
+        x = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+    }
+#define MC_ROW_ROR(n)                                                                                   \
+    x += __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x120 + n, 0xf, 0xf, false), \
+                          __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x120 + n, 0xf, 0xf, false))
+    MC_ROW_ROR(8);
+    MC_ROW_ROR(4);
+    MC_ROW_ROR(2);
+    MC_ROW_ROR(1);
+#undef MC_ROW_ROR
+    return x;
+}
+
+// The same over groups of eight lanes (pairs i ^ 1, i ^ 2, i ^ 4; the last as a
+// mirror of the eight, whose quads are uniform by then).
+__device__ __forceinline__ double lane8_sum(double x)
+{
+#define MC_DPP(ctrl)                                                                                  \
+    x += __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), ctrl, 0xf, 0xf, false), \
+                          __builtin_amdgcn_update_dpp(0, __double2loint(x), ctrl, 0xf, 0xf, false))
+    MC_DPP(0xB1);    // quad_perm 1 0 3 2
+    MC_DPP(0x4E);    // quad_perm 2 3 0 1
+    MC_DPP(0x141);   // row_half_mirror
+#undef MC_DPP
+    return x;
+}
+
+// Block-wide sums of NV values over W waves (blockDim.x == 64 W), the wave
+// sums of a value added in wave order by the thread of its number: thread k's
+// return value is total k (k < NV).
+template <int NV, int W>
+__device__ __forceinline__ double block_sums(const double (&v)[NV], double *lds /* NV*W */)
+{
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
     for (int k = 0; k < NV; k++) {
-        double x = v[k];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-        v[k] = x;
-    }
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane == 0) {
-#pragma unroll
-        for (int k = 0; k < NV; k++) lds[k * W + wid] = v[k];
+        const double x = wave_sum(v[k]);
+        if (lane == 0) lds[k * W + wid] = x;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int k = 0; k < NV; k++) {
-            double s = lds[k * W];
-            for (int w = 1; w < W; w++) s += lds[k * W + w];
-            v[k] = s;
-        }
+    double s = 0.0;
+    if (threadIdx.x < NV) {
+        const double *p = lds + threadIdx.x * W;
+        s = p[0];
+        for (int w = 1; w < W; w++) s += p[w];
     }
+    return s;
 }
 
 // Deterministic two-kernel reduction.  Each block of the producing kernel
@@ -407,36 +444,60 @@ template <int NV>
 __device__ __forceinline__ void block_partials(double (&v)[NV], double *partials, int bid, int nblocks)
 {
     __shared__ double lds[NV * 4];
-    block_sum<NV>(v, lds);
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int k = 0; k < NV; k++) partials[(size_t)k * nblocks + bid] = v[k];
-    }
+    const double s = block_sums<NV, 4>(v, lds);
+    if (threadIdx.x < NV) partials[(size_t)threadIdx.x * nblocks + bid] = s;
 }
 
 // Fixed-order sum of the partials of `nblocks` blocks (one block of
-// FINISH_THREADS threads); the totals are valid in thread 0.
+// FINISH_THREADS threads); the totals are valid in thread 0.  One block, a
+// chain of memory round trips: the loads of all values are in flight together
+// (one value after another, the twelve of a four-system BiCGStab step took a
+// round trip each: 16 us for 63 blocks, 5.7 us now).
 constexpr int FINISH_THREADS = 1024;
 template <int NV>
 __device__ __forceinline__ void sum_partials(const double *partials, int nblocks, double (&v)[NV])
 {
-    __shared__ double lds[NV * (FINISH_THREADS / 64)];
+    constexpr int W = FINISH_THREADS / 64, step = FINISH_THREADS;
+    __shared__ double lds[NV * W], tot[NV];
+    if (nblocks <= step) {
+        const bool in = (int)threadIdx.x < nblocks;
 #pragma unroll
-    for (int k = 0; k < NV; k++) {
-        const double *pk = partials + (size_t)k * nblocks;
-        double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-        const int step = blockDim.x;
-        int i = threadIdx.x;
-        for (; i + 3 * step < nblocks; i += 4 * step) {
-            s0 += pk[i];
-            s1 += pk[i + step];
-            s2 += pk[i + 2 * step];
-            s3 += pk[i + 3 * step];
+        for (int k = 0; k < NV; k++) v[k] = in ? 0.0 + partials[(size_t)k * nblocks + threadIdx.x] : 0.0;
+    } else {
+        // values in groups of G, four of a value's partials per trip
+        constexpr int G = NV < 4 ? NV : 4;
+        for (int k0 = 0; k0 < NV; k0 += G) {
+            double s[G][4];
+#pragma unroll
+            for (int g = 0; g < G; g++) s[g][0] = s[g][1] = s[g][2] = s[g][3] = 0.0;
+            int i = threadIdx.x;
+            for (; i + 3 * step < nblocks; i += 4 * step)
+#pragma unroll
+                for (int g = 0; g < G; g++) {
+                    const double *pk = partials + (size_t)(k0 + g < NV ? k0 + g : k0) * nblocks;
+                    s[g][0] += pk[i];
+                    s[g][1] += pk[i + step];
+                    s[g][2] += pk[i + 2 * step];
+                    s[g][3] += pk[i + 3 * step];
+                }
+            for (; i < nblocks; i += step)
+#pragma unroll
+                for (int g = 0; g < G; g++)
+                    s[g][0] += partials[(size_t)(k0 + g < NV ? k0 + g : k0) * nblocks + i];
+#pragma unroll
+            for (int g = 0; g < G; g++)
+#pragma unroll
+                for (int k = 0; k < NV; k++)
+                    if (k == k0 + g) v[k] = (s[g][0] + s[g][1]) + (s[g][2] + s[g][3]);
         }
-        for (; i < nblocks; i += step) s0 += pk[i];
-        v[k] = (s0 + s1) + (s2 + s3);
     }
-    block_sum<NV, FINISH_THREADS / 64>(v, lds);
+    const double s = block_sums<NV, W>(v, lds);
+    if (threadIdx.x < NV) tot[threadIdx.x] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int k = 0; k < NV; k++) v[k] = tot[k];
+    }
 }
 
 // Finishing kernel: one block of FINISH_THREADS threads; thread 0 runs epi(totals).

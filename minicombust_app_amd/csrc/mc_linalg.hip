@@ -196,11 +196,7 @@ __device__ __forceinline__ void for_rows(const Mat<T> &A, int r0, int r1, XF X, 
             }
 #pragma unroll
             for (int k = 0; k < NR; k++) {
-                double v = acc[k];
-                v += __shfl_xor(v, 1, 64);
-                v += __shfl_xor(v, 2, 64);
-                v += __shfl_xor(v, 4, 64);
-                acc[k] = v;
+                acc[k] = lane8_sum(acc[k]);
             }
             if (lane8 == 0 && r < r1) f(r, acc);
         }
@@ -1671,9 +1667,7 @@ __global__ void __launch_bounds__(BLOCK) k_resid_restrict(Mat<T> A, int nc, cons
             }
         }
     }
-    s += __shfl_xor(s, 1, 64);
-    s += __shfl_xor(s, 2, 64);
-    s += __shfl_xor(s, 4, 64);
+    s = lane8_sum(s);
     if (lane8 == 0 && I < nc) bc[I] = (T)s;
 }
 
@@ -2138,9 +2132,7 @@ __global__ void __launch_bounds__(BLOCK) k_box_restrict(BoxWalk w, R resid, T *b
         const int x = (X << b.sx) + i, y = (Y << b.sy) + j, z = (Z << b.sz) + k;
         if (x < b.nx && y < b.ny && z < b.nz) s = resid(x + b.nx * (y + b.ny * z));
     }
-    s += __shfl_xor(s, 1, 64);
-    s += __shfl_xor(s, 2, 64);
-    s += __shfl_xor(s, 4, 64);
+    s = lane8_sum(s);
     if (lane8 == 0 && I < b.nc) bc[I] = (T)s;
 }
 
