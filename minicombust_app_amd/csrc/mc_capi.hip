@@ -151,7 +151,8 @@ static int alloc_workspace(Ctx *c)
     MC_TRY(dalloc(c, &c->red, RED_PARTIALS));
     MC_TRY(dalloc(c, &c->dscal, 1024));
     MC_HIP(c, hipMemset(c->dscal, 0, 1024 * sizeof(double)));
-    MC_HIP(c, hipHostMalloc((void **)&c->hscal, 1024 * sizeof(double), hipHostMallocDefault));
+    MC_HIP(c, hipHostMalloc((void **)&c->hscal, 1024 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
+    MC_HIP(c, hipHostGetDevicePointer((void **)&c->hscal_dev, c->hscal, 0));
     memset(c->hscal, 0, 1024 * sizeof(double));
     MC_TRY(flow_workspace(c));
     return MC_OK;

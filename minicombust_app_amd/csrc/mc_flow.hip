@@ -1770,7 +1770,7 @@ __global__ void __launch_bounds__(256) k_neg_count(int n, const double *v, int r
 }
 
 // in place: counts -> exclusive offsets; *total = the sum
-__global__ void __launch_bounds__(1024) k_neg_scan(int nb, int *bcount, int *total)
+__global__ void __launch_bounds__(1024) k_neg_scan(int nb, int *bcount, int *total, Pub pub)
 {
     // waves scan their own sums by lane exchange, wave 0 the 16 wave totals (one
     // thread over all 1,024 sums took 10 us)
@@ -1795,6 +1795,7 @@ __global__ void __launch_bounds__(1024) k_neg_scan(int nb, int *bcount, int *tot
     if (t == 0) *total = all;
     int run = before + inc - s;
     for (int i = i0; i < i1; i++) { const int x = bcount[i]; bcount[i] = run; run += x; }
+    publish(pub);
 }
 
 __global__ void __launch_bounds__(256) k_neg_write(int n, const double *v, int rounds, const int *boff, int *list)
@@ -1888,13 +1889,13 @@ int clip_nonneg(Ctx *c, double *phi, int slot)
         const int nb = div_up(N, 256 * rounds);
         int *bc = (int *)c->red;
         hipLaunchKernelGGL(k_neg_count, dim3(nb), dim3(256), 0, c->stream, N, (const double *)phi, rounds, bc);
-        hipLaunchKernelGGL(k_neg_scan, dim3(1), dim3(1024), 0, c->stream, nb, bc, dcount);
+        hipLaunchKernelGGL(k_neg_scan, dim3(1), dim3(1024), 0, c->stream, nb, bc, dcount,
+                           make_pub(c, dcount, 700, sizeof(double)));
         hipLaunchKernelGGL(k_neg_write, dim3(nb), dim3(256), 0, c->stream, N, (const double *)phi, rounds,
                            (const int *)bc, c->neg_list);
         MC_LAUNCH_CHECK(c);
     }
-    MC_HIP(c, hipMemcpyAsync(hcount, dcount, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    MC_HIP(c, hipStreamSynchronize(c->stream));
+    MC_TRY(wait_pub(c));
     const int K = *hcount;
     c->st.clip_cells += K;
     if (K == 0) return MC_OK;

@@ -673,6 +673,31 @@ struct EpiBiXr {
     }
 };
 
+static_assert(sizeof(KState) % 8 == 0 && sizeof(KState) / 8 <= 500, "published as doubles below the mirror's other slots");
+
+int wait_pub(Ctx *c)
+{
+    const unsigned long long *flag = (const unsigned long long *)(c->hscal + PUB_FLAG);
+    for (unsigned spin = 1;; spin++) {
+        if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == c->pub_seq) return MC_OK;
+        if ((spin & 0x3fff) == 0) {
+            // the stream must still be at work on it: one that has drained or
+            // failed without publishing ends the wait
+            const hipError_t e = hipStreamQuery(c->stream);
+            if (e == hipErrorNotReady) {
+                (void)hipGetLastError();
+                continue;
+            }
+            MC_HIP(c, e);
+            if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == c->pub_seq) return MC_OK;
+            c->err = "a published result did not arrive";
+            return MC_ERR_HIP;
+        }
+    }
+}
+
+// A solver's state copied back and waited for (graph replays, which hold no
+// publication).
 static int poll_done(Ctx *c, KState *ks, KState *host)
 {
     MC_HIP(c, hipMemcpyAsync(host, ks, sizeof(KState), hipMemcpyDeviceToHost, c->stream));
@@ -760,10 +785,12 @@ static int bicgstab_nr(Ctx *c, const double *vals, double *const *b, double *con
                            g.chunk);
             launch_finish<3 * NR>(c->stream, c->red, g.blocks, EpiBiOmega<NR>{ks});
             hipLaunchKernelGGL(k_bi_xr<NR>, dim3(g.blocks), dim3(BLOCK), 0, c->stream, n, W, ks, c->red, g.chunk);
-            launch_finish<2 * NR>(c->stream, c->red, g.blocks, EpiBiXr<NR>{ks});
+            const bool last = j == batch - 1 || it == maxit - 1;
+            launch_finish<2 * NR>(c->stream, c->red, g.blocks, EpiBiXr<NR>{ks},
+                                  last ? make_pub(c, ks, 0, sizeof(KState)) : Pub());
         }
         MC_LAUNCH_CHECK(c);
-        MC_TRY(poll_done(c, ks, hs));
+        MC_TRY(wait_pub(c));
         c->st.host_polls++;
         if (hs->all_done || it >= maxit) break;
         double rn = 0.0;
@@ -869,7 +896,7 @@ __global__ void __launch_bounds__(BLOCK) k_maxabs(int n, const double *v, double
 }
 
 __global__ void __launch_bounds__(BLOCK) k_maxabs_finish(const double *v, const double *partials, int nblocks,
-                                                         double *out)
+                                                         double *out, Pub pub)
 {
     double mm = 0.0;
     for (int i = threadIdx.x; i < nblocks; i += BLOCK) mm = fmax(mm, partials[i]);
@@ -882,6 +909,7 @@ __global__ void __launch_bounds__(BLOCK) k_maxabs_finish(const double *v, const 
         const double p0 = v[0];
         *out = (p0 != p0) ? p0 : ((mm > p0) ? mm : p0);
     }
+    publish(pub);
 }
 
 int reduce_maxabs_pp(Ctx *c, const double *v, double *out_host)
@@ -889,10 +917,10 @@ int reduce_maxabs_pp(Ctx *c, const double *v, double *out_host)
     const Grid g = grid_for(c->N);
     double *d = c->dscal + 520;
     hipLaunchKernelGGL(k_maxabs, dim3(g.blocks), dim3(BLOCK), 0, c->stream, c->N, v, c->red, g.chunk);
-    hipLaunchKernelGGL(k_maxabs_finish, dim3(1), dim3(BLOCK), 0, c->stream, v, c->red, g.blocks, d);
+    hipLaunchKernelGGL(k_maxabs_finish, dim3(1), dim3(BLOCK), 0, c->stream, v, c->red, g.blocks, d,
+                       make_pub(c, d, 520, sizeof(double)));
     MC_LAUNCH_CHECK(c);
-    MC_HIP(c, hipMemcpyAsync(c->hscal + 520, d, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    MC_HIP(c, hipStreamSynchronize(c->stream));
+    MC_TRY(wait_pub(c));
     *out_host = c->hscal[520];
     return MC_OK;
 }
@@ -2840,7 +2868,7 @@ struct EpiPcgXr {
 // and ||r||; every step returns at once when the solve is done.
 template <typename T>
 static int pcg_iteration(Ctx *c, const Mat<T> &A, const Grid &g, PcgVecs<T> w, T *pa, T *pb, KState *ks,
-                         double vbytes)
+                         double vbytes, const Pub &pub = Pub())
 {
     const int n = c->N;
     {
@@ -2855,7 +2883,7 @@ static int pcg_iteration(Ctx *c, const Mat<T> &A, const Grid &g, PcgVecs<T> w, T
     launch_finish<1>(c->stream, c->red, g.blocks, EpiPcgAlpha{ks});
     hipLaunchKernelGGL(k_pcg_xr<T>, dim3(g.blocks), dim3(BLOCK), 0, c->stream, n, w.x, w.r, pb, w.q, ks, c->red,
                        g.chunk);
-    launch_finish<1>(c->stream, c->red, g.blocks, EpiPcgXr{ks});
+    launch_finish<1>(c->stream, c->red, g.blocks, EpiPcgXr{ks}, pub);
     return MC_OK;
 }
 
@@ -2955,12 +2983,14 @@ static int pcg_core(Ctx *c, const T *b, bool project, PcgVecs<T> w, double rtol,
                 MC_TRY(dense_join(c));
                 MC_HIP(c, hipGraphLaunch(ge, c->stream));
             } else {
-                MC_TRY(pcg_iteration<T>(c, A, g, w, pa, pb, ks, vbytes));
+                const bool last = j == batch - 1 || it == maxit - 1;
+                MC_TRY(pcg_iteration<T>(c, A, g, w, pa, pb, ks, vbytes,
+                                        last ? make_pub(c, ks, 0, sizeof(KState)) : Pub()));
             }
             std::swap(pa, pb);
         }
         MC_LAUNCH_CHECK(c);
-        MC_TRY(poll_done(c, ks, hs));
+        MC_TRY(graphs ? poll_done(c, ks, hs) : wait_pub(c));
         c->st.host_polls++;
         if (hs->all_done || it >= maxit) break;
         const double rn = hs->rnorm[0] / std::max(hs->tol[0], 1e-300);
@@ -3110,10 +3140,9 @@ int mixed_ir_solve(Ctx *c, const double *vals, const double *b, double *x, doubl
                 MC_DISPATCH_ND(nd_code(A), (k_ir_resid<ND_>), dim3(g.blocks), dim3(BLOCK), 0, c->stream, A, b, mean, x,
                                r, c->red, g.chunk);
             }
-            launch_finish<1>(c->stream, c->red, g.blocks, EpiSqrt{rn});
+            launch_finish<1>(c->stream, c->red, g.blocks, EpiSqrt{rn}, make_pub(c, rn, 621, sizeof(double)));
             MC_LAUNCH_CHECK(c);
-            MC_HIP(c, hipMemcpyAsync(c->hscal + 621, rn, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-            MC_HIP(c, hipStreamSynchronize(c->stream));
+            MC_TRY(wait_pub(c));
             c->st.host_polls++;
             rnorm = c->hscal[621];
         }
@@ -3332,7 +3361,7 @@ static void defl_launch(Ctx *c, const DeflVecs &v, const double *b, double *x, d
     launch_finish<defl_nv<K>()>(c->stream, c->red, g.blocks, EpiDefl<K>{sc, 1.0 / n});
     hipLaunchKernelGGL(k_defl_start<K>, dim3(g.blocks), dim3(BLOCK), 0, c->stream, n, v, b, (const double *)sc, x, r,
                        c->red, g.chunk);
-    launch_finish<2>(c->stream, c->red, g.blocks, EpiDeflAccept{sc, K});
+    launch_finish<2>(c->stream, c->red, g.blocks, EpiDeflAccept{sc, K}, make_pub(c, sc, 640, (K + 5) * sizeof(double)));
 }
 
 // The start of a loop-1 solve: *used = the start is kept (x = W y, and *ir
@@ -3376,8 +3405,7 @@ static int deflation_start(Ctx *c, const double *b, double *x, bool want_guess, 
     default: defl_launch<5>(c, v, b, x, r, sc); break;
     }
     MC_LAUNCH_CHECK(c);
-    MC_HIP(c, hipMemcpyAsync(c->hscal + 640, sc, (K + 5) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    MC_HIP(c, hipStreamSynchronize(c->stream));
+    MC_TRY(wait_pub(c));
     const double *h = c->hscal + 640;
     *used = h[K + 4] > 0.0;
     *bnorm = h[K + 2];
