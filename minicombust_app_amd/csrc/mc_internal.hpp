@@ -502,6 +502,49 @@ __device__ __forceinline__ void sum_partials(const double *partials, int nblocks
     }
 }
 
+// A finish folded into the kernel that needs its result: every block of 256
+// threads sums the partials itself, in k_finish's order (groups of 64 partials
+// by lane tree, the groups in ascending order), so each block has the totals
+// and no finishing launch stands between producer and consumer.  Every block
+// reads all partials, nblocks^2 x NV x 8 bytes from L2 in all, which up to
+// FOLD_BLOCKS costs less than the launch (about 5 us with its gap on a chain
+// of short kernels) and beyond it more.
+constexpr int FOLD_BLOCKS = 512;
+template <int NV>
+__device__ __forceinline__ void fold_sums(const double *partials, int nblocks, double (&tot)[NV])
+{
+    constexpr int MAXG = FOLD_BLOCKS / 64, Q = MAXG / 4;
+    __shared__ double lds[NV * MAXG], t[NV];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double x[NV][Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        const int i = (wave + 4 * q) * 64 + lane;
+#pragma unroll
+        for (int k = 0; k < NV; k++) x[k][q] = i < nblocks ? 0.0 + partials[(size_t)k * nblocks + i] : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        const int g = wave + 4 * q;
+        if (g * 64 < nblocks)
+#pragma unroll
+            for (int k = 0; k < NV; k++) {
+                const double s = wave_sum(x[k][q]);
+                if (lane == 0) lds[k * MAXG + g] = s;
+            }
+    }
+    __syncthreads();
+    if (threadIdx.x < NV) {
+        const double *p = lds + threadIdx.x * MAXG;
+        double s = p[0];
+        for (int g = 1; g * 64 < nblocks; g++) s += p[g];
+        t[threadIdx.x] = s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NV; k++) tot[k] = t[k];
+}
+
 // Publication of n doubles (a solver's state, a norm) to the pinned host
 // mirror by the kernel that forms them, followed by a sequence number the host
 // spins on (wait_pub): the host goes on a few microseconds after the kernel's

@@ -448,7 +448,7 @@ __global__ void __launch_bounds__(BLOCK) k_bi_init_r0(int n, BiVecs w, double *p
 
 // The criterion stays ||r|| <= rtol ||b|| (PETSc's default test, as with a
 // zero start).  A guess whose residual is not below ||b|| is dropped: that
-// right-hand side restarts from x0 = 0 (k_bi_zero_start), so a warm start
+// right-hand side restarts from x0 = 0 (in the first k_bi_pv), so a warm start
 // never converges later than the zero start would.
 template <int NR>
 struct EpiBiInitX0 {
@@ -477,18 +477,6 @@ struct EpiBiInitX0 {
     }
 };
 
-// x = 0, r = b for the right-hand sides whose guess was dropped (b = 0
-// included: its solution is zero)
-template <int NR>
-__global__ void __launch_bounds__(BLOCK) k_bi_zero_start(int n, BiVecs w, const KState *ks)
-{
-    const int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
-#pragma unroll
-    for (int k = 0; k < NR; k++)
-        if (ks->zero_start[k] || ks->bnorm[k] == 0.0) { w.x[k][i] = 0.0; w.r[k][i] = w.b[k][i]; }
-}
-
 template <int NR>
 struct EpiBiInit {
     KState *ks;
@@ -516,13 +504,28 @@ struct EpiBiInit {
 // v = A p with p formed on the fly ; partials of (r^, v)
 template <int ND, int NR>
 __global__ void __launch_bounds__(BLOCK) k_bi_pv(Mat<double> A, BiVecs w, const KState *ks, double *partials,
-                                                 int chunk)
+                                                 int chunk, int warm)
 {
-    if (ks->all_done) return;
     const int b = xcd_block(blockIdx.x, gridDim.x);
     const int r0 = b * chunk, r1 = min(A.n, r0 + chunk);
-    bool skip[NR], first[NR];
+    bool skip[NR], first[NR], zs[NR];
     double beta[NR], om[NR], dsum[NR];
+    bool any = false;
+#pragma unroll
+    for (int k = 0; k < NR; k++) {
+        // first iteration after a warm start: a right-hand side whose guess
+        // was dropped (b = 0 included: its solution is zero) restarts from
+        // x = 0, r = b, converged or not; p is then read from b, since other
+        // blocks are writing r
+        zs[k] = warm && (ks->zero_start[k] || ks->bnorm[k] == 0.0);
+        any |= zs[k];
+    }
+    if (any)
+        for (int i = r0 + (int)threadIdx.x; i < r1; i += BLOCK)
+#pragma unroll
+            for (int k = 0; k < NR; k++)
+                if (zs[k]) { w.x[k][i] = 0.0; w.r[k][i] = w.b[k][i]; }
+    if (ks->all_done) return;
 #pragma unroll
     for (int k = 0; k < NR; k++) {
         skip[k] = ks->done[k] != 0;
@@ -532,6 +535,7 @@ __global__ void __launch_bounds__(BLOCK) k_bi_pv(Mat<double> A, BiVecs w, const 
         dsum[k] = 0.0;
     }
     auto P = [&](int k, int j) -> double {
+        if (zs[k]) return w.b[k][j];
         if (first[k]) return w.r[k][j];
         return fma(beta[k], fma(-om[k], w.vo[k][j], w.po[k][j]), w.r[k][j]);
     };
@@ -561,18 +565,27 @@ struct EpiBiAlpha {
 
 // t = A s with s = r - alpha v formed on the fly ; partials of (t,s), (t,t), (s,s)
 template <int ND, int NR>
-__global__ void __launch_bounds__(BLOCK) k_bi_st(Mat<double> A, BiVecs w, const KState *ks, double *partials,
-                                                 int chunk)
+__global__ void __launch_bounds__(BLOCK) k_bi_st(Mat<double> A, BiVecs w, KState *ks, const double *fold,
+                                                 double *partials, int chunk)
 {
     if (ks->all_done) return;
     const int b = xcd_block(blockIdx.x, gridDim.x);
     const int r0 = b * chunk, r1 = min(A.n, r0 + chunk);
     bool skip[NR];
     double al[NR], dsum[3 * NR];
+    if (fold) {   // EpiBiAlpha here; no block reads the alpha that block 0 stores for k_bi_xr
+        double v[NR];
+        fold_sums<NR>(fold, gridDim.x, v);
+#pragma unroll
+        for (int k = 0; k < NR; k++) {
+            al[k] = ks->rho[k] / v[k];
+            if (blockIdx.x == 0 && threadIdx.x == 0 && !ks->done[k]) ks->alpha[k] = al[k];
+        }
+    }
 #pragma unroll
     for (int k = 0; k < NR; k++) {
         skip[k] = ks->done[k] != 0;
-        al[k] = ks->alpha[k];
+        if (!fold) al[k] = ks->alpha[k];
         dsum[3 * k] = dsum[3 * k + 1] = dsum[3 * k + 2] = 0.0;
     }
     auto S = [&](int k, int j) -> double { return fma(-al[k], w.v[k][j], w.r[k][j]); };
@@ -610,19 +623,37 @@ struct EpiBiOmega {
 
 // x += alpha p + omega s ; r = s - omega t ; partials of (r,r), (r^,r)
 template <int NR>
-__global__ void __launch_bounds__(BLOCK) k_bi_xr(int n, BiVecs w, const KState *ks, double *partials, int chunk)
+__global__ void __launch_bounds__(BLOCK) k_bi_xr(int n, BiVecs w, KState *ks, const double *fold, double *partials,
+                                                 int chunk)
 {
     if (ks->all_done) return;
     const int b = xcd_block(blockIdx.x, gridDim.x);
     const int i0 = b * chunk, i1 = min(n, i0 + chunk);
     bool skip[NR], half[NR];
     double al[NR], om[NR], acc[2 * NR];
+    if (fold) {   // EpiBiOmega here; what block 0 stores is read by EpiBiXr only
+        double v[3 * NR];
+        fold_sums<3 * NR>(fold, gridDim.x, v);
+#pragma unroll
+        for (int k = 0; k < NR; k++) {
+            const double sn = sqrt(v[3 * k + 2]);
+            half[k] = sn <= ks->tol[k];
+            om[k] = v[3 * k] / v[3 * k + 1];
+            if (blockIdx.x == 0 && threadIdx.x == 0 && !ks->done[k]) {
+                ks->sn[k] = sn;
+                ks->half[k] = half[k] ? 1 : 0;
+                if (!half[k]) ks->omega[k] = om[k];
+            }
+        }
+    }
 #pragma unroll
     for (int k = 0; k < NR; k++) {
         skip[k] = ks->done[k] != 0;
-        half[k] = ks->half[k] != 0;
         al[k] = ks->alpha[k];
-        om[k] = ks->omega[k];
+        if (!fold) {
+            half[k] = ks->half[k] != 0;
+            om[k] = ks->omega[k];
+        }
         acc[2 * k] = acc[2 * k + 1] = 0.0;
     }
     for (int i = i0 + threadIdx.x; i < i1; i += BLOCK) {
@@ -746,17 +777,19 @@ static int bicgstab_nr(Ctx *c, const double *vals, double *const *b, double *con
     KState *ks = (KState *)c->dscal;
     KState *hs = (KState *)c->hscal;
     const Grid g = grid_for(n);
+    // short grids: alpha and omega are formed by their consumers (fold_sums);
+    // a folding kernel reads one half of the partials buffer and writes the other
+    const bool fold = g.blocks <= FOLD_BLOCKS;
+    double *red2 = fold ? c->red + RED_PARTIALS / 2 : c->red;
     if (warm && r0) {
         // the assembly formed r = b - A x0 (same x0, same matrix): it is the r vector
         for (int k = 0; k < NR; k++) w[0].r[k] = w[1].r[k] = r0[k];
         hipLaunchKernelGGL(k_bi_init_r0<NR>, dim3(g.blocks), dim3(BLOCK), 0, c->stream, n, w[0], c->red, g.chunk);
         launch_finish<3 * NR>(c->stream, c->red, g.blocks, EpiBiInitX0<NR>{ks, rtol, maxit});
-        hipLaunchKernelGGL(k_bi_zero_start<NR>, dim3(div_up(n, BLOCK)), dim3(BLOCK), 0, c->stream, n, w[0], ks);
     } else if (warm) {
         MC_DISPATCH_ND(nd_code(A), (k_bi_init_x0<ND_, NR>), dim3(g.blocks), dim3(BLOCK), 0, c->stream, A, w[0], c->red,
                        g.chunk);
         launch_finish<3 * NR>(c->stream, c->red, g.blocks, EpiBiInitX0<NR>{ks, rtol, maxit});
-        hipLaunchKernelGGL(k_bi_zero_start<NR>, dim3(div_up(n, BLOCK)), dim3(BLOCK), 0, c->stream, n, w[0], ks);
     } else {
         hipLaunchKernelGGL(k_bi_init<NR>, dim3(g.blocks), dim3(BLOCK), 0, c->stream, n, w[0], c->red, g.chunk);
         launch_finish<NR>(c->stream, c->red, g.blocks, EpiBiInit<NR>{ks, rtol, maxit});
@@ -778,13 +811,14 @@ static int bicgstab_nr(Ctx *c, const double *vals, double *const *b, double *con
             {
                 KTimer kt(c, MC_KC_BICG, mbytes);
                 MC_DISPATCH_ND(nd_code(A), (k_bi_pv<ND_, NR>), dim3(g.blocks), dim3(BLOCK), 0, c->stream, A, W, ks, c->red,
-                               g.chunk);
+                               g.chunk, warm && it == 0 ? 1 : 0);
             }
-            launch_finish<NR>(c->stream, c->red, g.blocks, EpiBiAlpha<NR>{ks});
-            MC_DISPATCH_ND(nd_code(A), (k_bi_st<ND_, NR>), dim3(g.blocks), dim3(BLOCK), 0, c->stream, A, W, ks, c->red,
-                           g.chunk);
-            launch_finish<3 * NR>(c->stream, c->red, g.blocks, EpiBiOmega<NR>{ks});
-            hipLaunchKernelGGL(k_bi_xr<NR>, dim3(g.blocks), dim3(BLOCK), 0, c->stream, n, W, ks, c->red, g.chunk);
+            if (!fold) launch_finish<NR>(c->stream, c->red, g.blocks, EpiBiAlpha<NR>{ks});
+            MC_DISPATCH_ND(nd_code(A), (k_bi_st<ND_, NR>), dim3(g.blocks), dim3(BLOCK), 0, c->stream, A, W, ks,
+                           fold ? (const double *)c->red : nullptr, red2, g.chunk);
+            if (!fold) launch_finish<3 * NR>(c->stream, red2, g.blocks, EpiBiOmega<NR>{ks});
+            hipLaunchKernelGGL(k_bi_xr<NR>, dim3(g.blocks), dim3(BLOCK), 0, c->stream, n, W, ks,
+                               fold ? (const double *)red2 : nullptr, c->red, g.chunk);
             const bool last = j == batch - 1 || it == maxit - 1;
             launch_finish<2 * NR>(c->stream, c->red, g.blocks, EpiBiXr<NR>{ks},
                                   last ? make_pub(c, ks, 0, sizeof(KState)) : Pub());
@@ -2564,7 +2598,7 @@ static int vcycle(Ctx *c, size_t l, const T *b, T *x, KState *ks, const KState *
         if (ks) {  // one-level hierarchy: no smoothing sweep carries the (r, z) reduction
             const Grid g = grid_for(L.n);
             hipLaunchKernelGGL(k_rz<T>, dim3(g.blocks), dim3(BLOCK), 0, c->stream, L.n, b, x, ks, c->red, g.chunk);
-            launch_finish<1>(c->stream, c->red, g.blocks, EpiRz{ks});
+            if (g.blocks > FOLD_BLOCKS) launch_finish<1>(c->stream, c->red, g.blocks, EpiRz{ks});
         }
         return MC_OK;
     }
@@ -2683,7 +2717,7 @@ static int vcycle(Ctx *c, size_t l, const T *b, T *x, KState *ks, const KState *
                 MC_DISPATCH_ND(nd_code(A), (k_jac<ND_, T>), dim3(g.blocks), dim3(BLOCK), 0, c->stream, A, dinv, b,
                                cur, dst, (T)wts[nu - 1 - s], g.chunk, dotv, c->red, stop);
         }
-        if (dotv) launch_finish<1>(c->stream, c->red, g.blocks, EpiRz{ks});
+        if (dotv && g.blocks > FOLD_BLOCKS) launch_finish<1>(c->stream, c->red, g.blocks, EpiRz{ks});
         oth = cur;
         cur = dst;
     }
@@ -2805,13 +2839,20 @@ struct EpiPcgInit {
 // product reads z + beta p_old at the neighbours, so the p update needs no
 // pass of its own (p_old and p_new are separate buffers).
 template <int ND, typename T>
-__global__ void __launch_bounds__(BLOCK) k_pcg_pq(Mat<T> A, const T *z, const T *pold, T *pnew, T *q,
-                                                  const KState *ks, double *partials, int chunk)
+__global__ void __launch_bounds__(BLOCK) k_pcg_pq(Mat<T> A, const T *z, const T *pold, T *pnew, T *q, KState *ks,
+                                                  const double *fold, double *partials, int chunk)
 {
     if (ks->all_done) return;
     const int bb = xcd_block(blockIdx.x, gridDim.x);
     const int r0 = bb * chunk, r1 = min(A.n, r0 + chunk);
-    const T beta = (T)ks->beta[0];
+    double be = fold ? 0.0 : ks->beta[0];
+    if (fold) {   // EpiRz here, rho_old left to EpiPcgXr: no block reads what block 0 stores
+        double v[1];
+        fold_sums<1>(fold, gridDim.x, v);
+        be = (ks->iters[0] == 0) ? 0.0 : v[0] / ks->rho_old[0];
+        if (blockIdx.x == 0 && threadIdx.x == 0) { ks->rho[0] = v[0]; ks->beta[0] = be; }
+    }
+    const T beta = (T)be;
     double dsum[1] = {0.0};
     for_rows<ND, 1>(A, r0, r1, [&](int, int j) { return (double)(z[j] + beta * pold[j]); },
                     [&](int r, const double (&ax)[1]) {
@@ -2833,12 +2874,18 @@ struct EpiPcgAlpha {
 
 template <typename T>
 __global__ void __launch_bounds__(BLOCK) k_pcg_xr(int n, T *x, T *r, const T *p, const T *q, const KState *ks,
-                                                  double *partials, int chunk)
+                                                  const double *fold, double *partials, int chunk)
 {
     if (ks->all_done) return;
     const int bb = xcd_block(blockIdx.x, gridDim.x);
     const int i0 = bb * chunk, i1 = min(n, i0 + chunk);
-    const T al = (T)ks->alpha[0];
+    double a = fold ? 0.0 : ks->alpha[0];
+    if (fold) {   // EpiPcgAlpha here
+        double v[1];
+        fold_sums<1>(fold, gridDim.x, v);
+        a = ks->rho[0] / v[0];
+    }
+    const T al = (T)a;
     double acc[1] = {0.0};
     for (int i = i0 + threadIdx.x; i < i1; i += BLOCK) {
         x[i] += al * p[i];
@@ -2855,6 +2902,7 @@ struct EpiPcgXr {
     {
         if (ks->all_done) return;
         const double rn = sqrt(v[0]);
+        ks->rho_old[0] = ks->rho[0];
         ks->rnorm[0] = rn;
         ks->iters[0] += 1;
         if (rn <= ks->tol[0]) { ks->done[0] = 1; ks->conv[0] = 1; }
@@ -2871,6 +2919,8 @@ static int pcg_iteration(Ctx *c, const Mat<T> &A, const Grid &g, PcgVecs<T> w, T
                          double vbytes, const Pub &pub = Pub())
 {
     const int n = c->N;
+    const bool fold = g.blocks <= FOLD_BLOCKS;   // rho, beta and alpha formed by their consumers (fold_sums)
+    double *red2 = fold ? c->red + RED_PARTIALS / 2 : c->red;
     {
         KTimer kt(c, MC_KC_VCYCLE, c->profile ? vcycle_bytes<T>(c) : 0.0);
         MC_TRY(vcycle<T>(c, 0, w.r, w.z, ks, ks));
@@ -2878,11 +2928,11 @@ static int pcg_iteration(Ctx *c, const Mat<T> &A, const Grid &g, PcgVecs<T> w, T
     {
         KTimer kt(c, sizeof(T) == 8 ? MC_KC_SPMV64 : MC_KC_SPMV32, vbytes);
         MC_DISPATCH_ND(nd_code(A), (k_pcg_pq<ND_, T>), dim3(g.blocks), dim3(BLOCK), 0, c->stream, A, w.z, pa, pb, w.q,
-                       ks, c->red, g.chunk);
+                       ks, fold ? (const double *)c->red : nullptr, red2, g.chunk);
     }
-    launch_finish<1>(c->stream, c->red, g.blocks, EpiPcgAlpha{ks});
-    hipLaunchKernelGGL(k_pcg_xr<T>, dim3(g.blocks), dim3(BLOCK), 0, c->stream, n, w.x, w.r, pb, w.q, ks, c->red,
-                       g.chunk);
+    if (!fold) launch_finish<1>(c->stream, red2, g.blocks, EpiPcgAlpha{ks});
+    hipLaunchKernelGGL(k_pcg_xr<T>, dim3(g.blocks), dim3(BLOCK), 0, c->stream, n, w.x, w.r, pb, w.q, ks,
+                       fold ? (const double *)red2 : nullptr, c->red, g.chunk);
     launch_finish<1>(c->stream, c->red, g.blocks, EpiPcgXr{ks}, pub);
     return MC_OK;
 }
