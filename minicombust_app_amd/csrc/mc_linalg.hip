@@ -1884,30 +1884,37 @@ template <> float *lv_t<float>(AmgLevel &L) { return L.t32; }
 template <> float *lv_dinv<float>(AmgLevel &L) { return L.dinv32; }
 
 // ------------------------------- V-cycle tail of a matched hierarchy --
-// The levels of at most VT_ROWS rows, and the dense coarsest level, in one
-// workgroup: each launch of vcycle() on those levels becomes a pass of the
-// 1024 threads over the level's rows, the passes separated by barriers, so
-// half a dozen launches of a few microseconds each become one.  Every row is
-// formed by the expressions of the per-pass kernels (k_jac_first2, k_jac,
-// k_resid, k_restrict, k_dense_apply) in the same order, so the result is the
-// same.  Measured at m = 128: a tail from the 1,024-row level saves 0.05 ms per
-// pressure solve; one from the 8,192-row level costs 0.3 ms more than the
-// launches it replaces (one CU's passes over 8K rows are slower).
-constexpr int VT_LEVELS = 4, VT_ROWS = 2048, TAIL_THREADS = 1024;
+// The small levels of a hierarchy from pairwise matching, and the dense
+// coarsest level, in one workgroup of 1024 threads: the six launches of a
+// level (7 to 10 us each with their gaps on a CSR level of any size) become
+// passes separated by barriers.  A pass is bound by one round trip to L2 for
+// the matrix: x and b of every level stay in LDS, CSR row pointers too, and all
+// of a thread's entries are asked for together.  Rows in diagonal storage take
+// a thread each; CSR rows eight lanes, lane l the entries l, l + 8, ..., as in
+// the per-pass kernels.  Every row is formed by those kernels' expressions
+// (k_jac_first2, k_jac, k_resid_restrict_seq / k_resid_restrict, k_jac_prolong,
+// k_dense_apply) in the same order, so the result is the same.
+// Sizes: LDS holds VT_SUM rows in all; a first level beyond VT_ROWS takes
+// longer on one CU than its launches do on all of them.  Measured: modifier 33
+// mixed (13 launches of the two CSR levels below 9,537 rows into one) 47 us per
+// cycle, ten timesteps 92 -> 82 ms.
+constexpr int VT_LEVELS = 4, VT_ROWS = 2304, VT_SUM = 4096, TAIL_THREADS = 1024;
 
 template <typename T>
 struct VtLevel {
-    Mat<T> A;
+    Mat<T> A;                       // dia: 7 diagonals; else CSR
     const T *dinv;
-    T *b, *x, *t;
     const int *agg, *aptr, *amem;   // aggregation to the next level
     int nc;
+    int off, rpo;                   // the level's place in the LDS vectors / row pointers
 };
 
 template <typename T>
 struct VtArgs {
-    VtLevel<T> lv[VT_LEVELS + 1];   // lv[nl]: the dense level (b, x only)
+    VtLevel<T> lv[VT_LEVELS];
     int nl;                             // smoothed levels
+    const T *b;                         // right-hand side and solution of the first
+    T *x;
     const double *inv;                  // dense inverse, transposed
     int nd;                             // dense level size
     int nu;
@@ -1915,127 +1922,182 @@ struct VtArgs {
     double w[8];
 };
 
-template <int ND, typename T, typename XF>
-__device__ __forceinline__ double tail_ax(const Mat<T> &A, int i, XF X)
+// f(i, (A src)_i, D^-1_i) for every row i, by one thread each
+template <bool SYM, typename T, typename F>
+__device__ __forceinline__ void vt_rows(const VtLevel<T> &L, const T *src, const int *rp, F f)
 {
-    constexpr bool SYM = ND < 0;
-    constexpr int NA = SYM ? -ND : ND;
-    double a[NA > 0 ? NA : 1];
-    int j[NA > 0 ? NA : 1];
+    const int n = L.A.n, tid = threadIdx.x;
+    if (L.A.dia) {
+        constexpr int R = (VT_ROWS + TAIL_THREADS - 1) / TAIL_THREADS;
+        double a[R][7];
+        T di[R];
 #pragma unroll
-    for (int d = 0; d < NA; d++) {
-        a[d] = dia_at<SYM>(A, d, i);
-        j[d] = clampi(i + A.off[d], A.n);
+        for (int r = 0; r < R; r++) {
+            if (TAIL_THREADS * r >= n) break;
+            const int i = min(tid + TAIL_THREADS * r, n - 1);
+#pragma unroll
+            for (int d = 0; d < 7; d++) a[r][d] = dia_at<SYM>(L.A, d, i);
+            di[r] = L.dinv[i];
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if (TAIL_THREADS * r >= n) break;
+            const int i = tid + TAIL_THREADS * r;
+            if (i >= n) continue;
+            double acc = 0.0;
+#pragma unroll
+            for (int d = 0; d < 7; d++) acc = fma(a[r][d], (double)src[clampi(i + L.A.off[d], n)], acc);
+            f(i, acc, di[r]);
+        }
+    } else {
+        constexpr int B = 3, E = 3;   // rows in flight, entries per lane fetched ahead
+        const int lane8 = tid & 7, g = tid >> 3;
+        for (int r0 = 0; r0 < n; r0 += 128 * B) {
+            double v[B][E];
+            int c[B][E], beg[B], end[B];
+            T di[B];
+#pragma unroll
+            for (int q = 0; q < B; q++) {
+                const int i = min(r0 + 128 * q + g, n - 1);
+                beg[q] = rp[i];
+                end[q] = rp[i + 1];
+                di[q] = L.dinv[i];
+#pragma unroll
+                for (int e = 0; e < E; e++) {
+                    const int k = beg[q] + lane8 + 8 * e;
+                    const bool in = k < end[q];
+                    const int kk = in ? k : beg[q];
+                    c[q][e] = L.A.col[kk];
+                    v[q][e] = in ? (double)L.A.csr[kk] : 0.0;
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < B; q++) {
+                double acc = 0.0;
+#pragma unroll
+                for (int e = 0; e < E; e++)
+                    if (beg[q] + lane8 + 8 * e < end[q]) acc = fma(v[q][e], (double)src[c[q][e]], acc);
+                for (int k = beg[q] + lane8 + 8 * E; k < end[q]; k += 8)
+                    acc = fma((double)L.A.csr[k], (double)src[L.A.col[k]], acc);
+                acc = lane8_sum(acc);
+                const int i = r0 + 128 * q + g;
+                if (lane8 == 0 && i < n) f(i, acc, di[q]);
+            }
+        }
     }
-    double acc = 0.0;
-#pragma unroll
-    for (int d = 0; d < NA; d++) acc = fma(a[d], X(j[d]), acc);
-    return acc;
 }
 
-template <int ND, typename T>
+template <bool SYM, typename T>
 __global__ void __launch_bounds__(TAIL_THREADS) k_vtail(VtArgs<T> a, const KState *stop)
 {
-    if constexpr (ND != 7 && ND != -7) {
-        return;   // 7-diagonal storage only (the host launches no other)
-    } else {
-        if (stop && stop->all_done) return;
-        __shared__ double bs[DENSE_MAX];
-        __shared__ double part[TAIL_THREADS / DENSE_MAX][DENSE_MAX];
-        const int tid = threadIdx.x;
-        T *curs[VT_LEVELS], *oths[VT_LEVELS];
-        const int nu = a.nu;
-#pragma unroll
-        for (int l = 0; l < VT_LEVELS; l++) {
-            if (l >= a.nl) break;
-            const VtLevel<T> &L = a.lv[l];
-            const int n = L.A.n;
-            T *cur = L.x, *oth = L.t;
-            const T w1 = (T)a.w[0], w2 = (T)a.w[nu >= 2 ? 1 : 0];
-            for (int i = tid; i < n; i += TAIL_THREADS) {
-                if (nu >= 2) {
-                    const double ax = tail_ax<ND>(L.A, i, [&](int jj) { return (double)vc_first(w1, L.dinv[jj], L.b[jj]); });
-                    cur[i] = vc_first2(w1, w2, L.dinv[i], L.b[i], ax);
-                } else {
-                    cur[i] = vc_first(w1, L.dinv[i], L.b[i]);
-                }
-            }
+    if (stop && stop->all_done) return;
+    __shared__ T xs[VT_SUM], bl[VT_SUM], alt[VT_ROWS];
+    __shared__ int rps[VT_SUM + VT_LEVELS];
+    __shared__ double bs[DENSE_MAX];
+    __shared__ T xd[DENSE_MAX];
+    __shared__ double part[TAIL_THREADS / DENSE_MAX][DENSE_MAX];
+    const int tid = threadIdx.x, nu = a.nu;
+    for (int l = 0; l < a.nl; l++)
+        if (!a.lv[l].A.dia)
+            for (int i = tid; i <= a.lv[l].A.n; i += TAIL_THREADS) rps[a.lv[l].rpo + i] = a.lv[l].A.rp[i];
+    for (int i = tid; i < a.lv[0].A.n; i += TAIL_THREADS) bl[i] = a.b[i];
+    __syncthreads();
+    for (int l = 0; l < a.nl; l++) {
+        const VtLevel<T> &L = a.lv[l];
+        const int n = L.A.n;
+        T *x = xs + L.off;
+        const T *b = bl + L.off;
+        const int *rp = rps + L.rpo;
+        const T w1 = (T)a.w[0], w2 = (T)a.w[nu >= 2 ? 1 : 0];
+        for (int i = tid; i < n; i += TAIL_THREADS) x[i] = vc_first(w1, L.dinv[i], b[i]);
+        __syncthreads();
+        T *cur = x, *oth = alt;
+        for (int k = 1; k < nu; k++) {
+            const T omega = (T)a.w[k];
+            if (k == 1)
+                vt_rows<SYM>(L, cur, rp, [&](int i, double ax, T di) { oth[i] = vc_first2(w1, w2, di, b[i], ax); });
+            else
+                vt_rows<SYM>(L, cur, rp, [&](int i, double ax, T di) { oth[i] = vc_jac(cur[i], omega, di, b[i], ax); });
             __syncthreads();
-            for (int s = 2; s < nu; s++) {
-                const T omega = (T)a.w[s];
-                for (int i = tid; i < n; i += TAIL_THREADS) {
-                    const double ax = tail_ax<ND>(L.A, i, [&](int jj) { return (double)cur[jj]; });
-                    oth[i] = vc_jac(cur[i], omega, L.dinv[i], L.b[i], ax);
-                }
-                __syncthreads();
-                T *sw = cur; cur = oth; oth = sw;
-            }
-            T *r = (cur == L.x) ? L.t : L.x;
-            for (int i = tid; i < n; i += TAIL_THREADS)
-                r[i] = (T)((double)L.b[i] - tail_ax<ND>(L.A, i, [&](int jj) { return (double)cur[jj]; }));
+            T *sw = cur; cur = oth; oth = sw;
+        }
+        if (cur != x) {   // x keeps the value; alt is free
+            for (int i = tid; i < n; i += TAIL_THREADS) x[i] = cur[i];
             __syncthreads();
-            T *bc = a.lv[l + 1].b;
+        }
+        const bool dense = l + 1 == a.nl;
+        T *bc = dense ? nullptr : bl + a.lv[l + 1].off;
+        if (L.A.dia) {
+            vt_rows<SYM>(L, x, rp, [&](int i, double ax, T) { alt[i] = (T)((double)b[i] - ax); });
+            __syncthreads();
             for (int I = tid; I < L.nc; I += TAIL_THREADS) {
                 double sum = 0.0;
-                for (int t = L.aptr[I]; t < L.aptr[I + 1]; t++) sum += (double)r[L.amem[t]];
-                bc[I] = (T)sum;
+                for (int t = L.aptr[I]; t < L.aptr[I + 1]; t++) sum += (double)alt[L.amem[t]];
+                if (dense) bs[I] = (double)(T)sum; else bc[I] = (T)sum;
             }
-            __syncthreads();
-            curs[l] = cur;
-            oths[l] = oth;
+        } else {
+            const int lane8 = tid & 7;
+            for (int I0 = 0; I0 < L.nc; I0 += 128) {
+                const int I = I0 + (tid >> 3);
+                double s = 0.0;
+                if (I < L.nc)
+                    for (int t = L.aptr[I]; t < L.aptr[I + 1]; t++) {
+                        const int i = L.amem[t];
+                        double acc = 0.0;
+                        for (int e = rp[i] + lane8; e < rp[i + 1]; e += 8)
+                            acc = fma((double)L.A.csr[e], (double)x[L.A.col[e]], acc);
+                        if (lane8 == 0) s += (double)b[i];
+                        s -= acc;
+                    }
+                s = lane8_sum(s);
+                if (lane8 == 0 && I < L.nc) { if (dense) bs[I] = (double)(T)s; else bc[I] = (T)s; }
+            }
         }
-        {   // dense coarsest level
-            constexpr int PARTS = TAIL_THREADS / DENSE_MAX, PLEN = DENSE_MAX / PARTS;
-            const int nd = a.nd;
-            const T *bd = a.lv[a.nl].b;
-            T *xd = a.lv[a.nl].x;
-            if (tid < nd) bs[tid] = (double)bd[tid];
-            __syncthreads();
-            const int i = tid % DENSE_MAX, p = tid / DENSE_MAX;
-            double sum = 0.0;
-            if (i < nd) {
-                const int j0 = p * PLEN;
+        __syncthreads();
+    }
+    {   // dense coarsest level, as k_dense_apply
+        constexpr int PARTS = TAIL_THREADS / DENSE_MAX, PLEN = DENSE_MAX / PARTS;
+        const int nd = a.nd;
+        const int i = tid % DENSE_MAX, p = tid / DENSE_MAX;
+        double sum = 0.0;
+        if (i < nd) {
+            const int j0 = p * PLEN;
 #pragma unroll
-                for (int jj = 0; jj < PLEN; jj++) {
-                    const int j = j0 + jj;
-                    if (j < nd) sum = fma(a.inv[(size_t)j * nd + i], bs[j], sum);
-                }
+            for (int jj = 0; jj < PLEN; jj++) {
+                const int j = j0 + jj;
+                if (j < nd) sum = fma(a.inv[(size_t)j * nd + i], bs[j], sum);
             }
-            part[p][i] = sum;
-            __syncthreads();
-            if (tid < nd) {
-                double y = 0.0;
-#pragma unroll
-                for (int q = 0; q < PARTS; q++) y += part[q][tid];
-                xd[tid] = (T)y;
-            }
-            __syncthreads();
         }
+        part[p][i] = sum;
+        __syncthreads();
+        if (tid < nd) {
+            double y = 0.0;
 #pragma unroll
-        for (int l = VT_LEVELS - 1; l >= 0; l--) {
-            if (l >= a.nl) continue;
-            const VtLevel<T> &L = a.lv[l];
-            const int n = L.A.n;
-            const T *xc = a.lv[l + 1].x;
-            T *cur = curs[l], *oth = oths[l], *x = L.x, *tmp = L.t;
-            for (int s = 0; s < nu; s++) {
-                const bool first = s == 0, last = s == nu - 1;
-                T *dst = last ? x : oth;
-                if (dst == cur) dst = tmp;
-                const T omega = (T)a.w[nu - 1 - s];
-                auto yv = [&](int jj) -> T { return first ? vc_prolong(cur[jj], a.cs, xc[L.agg[jj]]) : cur[jj]; };
-                for (int i = tid; i < n; i += TAIL_THREADS) {
-                    const double ax = tail_ax<ND>(L.A, i, [&](int jj) { return (double)yv(jj); });
-                    dst[i] = vc_jac(yv(i), omega, L.dinv[i], L.b[i], ax);
-                }
-                __syncthreads();
-                oth = cur;
-                cur = dst;
-            }
-            if (cur != x) {
-                for (int i = tid; i < n; i += TAIL_THREADS) x[i] = cur[i];
-                __syncthreads();
-            }
+            for (int q = 0; q < PARTS; q++) y += part[q][tid];
+            xd[tid] = (T)y;
+        }
+        __syncthreads();
+    }
+    for (int l = a.nl - 1; l >= 0; l--) {
+        const VtLevel<T> &L = a.lv[l];
+        const int n = L.A.n;
+        const T *xc = l + 1 == a.nl ? xd : xs + a.lv[l + 1].off;
+        T *x = xs + L.off;
+        const T *b = bl + L.off;
+        for (int i = tid; i < n; i += TAIL_THREADS) x[i] = vc_prolong(x[i], a.cs, xc[L.agg[i]]);
+        __syncthreads();
+        T *cur = x, *oth = alt;
+        for (int k = 0; k < nu; k++) {
+            const T omega = (T)a.w[nu - 1 - k];
+            vt_rows<SYM>(L, cur, rps + L.rpo,
+                         [&](int i, double ax, T di) { oth[i] = vc_jac(cur[i], omega, di, b[i], ax); });
+            __syncthreads();
+            T *sw = cur; cur = oth; oth = sw;
+        }
+        T *dst = l == 0 ? a.x : x;
+        if (cur != dst) {
+            for (int i = tid; i < n; i += TAIL_THREADS) dst[i] = cur[i];
+            __syncthreads();
         }
     }
 }
@@ -2280,28 +2342,36 @@ __global__ void __launch_bounds__(BLOCK) k_box_jac_prolong_h(BoxProlong<float> p
 }
 
 // ----------------------------------------------------- V-cycle tail --
-// The small box levels and the dense coarsest one in one workgroup of 1024
-// threads.  Bound by the chain of passes, each a handful of values per row:
+// The small levels in seven-diagonal storage (box levels, or matched ones whose
+// aggregates came out regular) and the dense coarsest one in one workgroup of
+// 1024 threads.  Bound by the chain of passes, each a handful of values per row:
 // a row's matrix entries, inverse diagonal, right-hand side and value stay in
 // its thread's registers for the whole cycle (loaded at the start, all in
 // flight together) and only x goes through LDS for the neighbours, so a sweep
-// is six LDS reads and two barriers instead of a launch (or, as in the
-// earlier tail, a round of loads from L2).  Every row is formed by the
+// is seven LDS reads and two barriers instead of a launch (or, as in the
+// earlier tail, a round of loads from L2).  LDS holds x as doubles also in the
+// FP32 cycle: a value is converted once when stored, not by each of its seven
+// readers (FP64 sums; the conversions run at a quarter of the rate).  Every row is formed by the
 // expressions of the per-pass kernels in the same order, so the result is the
 // same (amg_tail = 0 launches them).
-// Rows: up to R0 x 1024 on the first level, 1024 and 512 below.  FP32
-// takes R0 = 8, FP64 4 (more entries than registers beyond).  FP32, levels of
-// 4,225 and 637 rows and a dense 112: 28 us, where the matched hierarchy's CSR
-// levels of these sizes take 13 launches of 7 to 15 us.
+// Rows: up to R0 x 1024 on the first level, 1024 and 512 below.  FP64
+// takes R0 = 4 (more entries than registers beyond), FP32 5: 8,192 rows in
+// eight a thread measured 52 us, its six launches with the tail of the next
+// level 40.  FP64, 1,024 rows and a dense 128: 22 -> 11.8 us; 2,000 and 250
+// rows: 38 -> 18 us.  FP32, 4,225 and 637 rows and a dense 112: 27 us, where
+// the matched hierarchy's CSR levels of these sizes took 13 launches of 7 to
+// 15 us.
 constexpr int TAIL_LEVELS = 3;
-template <typename T> constexpr int tail_rows() { return (sizeof(T) == 4 ? 8 : 4) * TAIL_THREADS; }
+template <typename T> constexpr int tail_rows() { return (sizeof(T) == 4 ? 5 : 4) * TAIL_THREADS; }
 constexpr int tail_cap(int l) { return l <= 1 ? 1024 : 512; }   // rows of level l >= 1
 
 template <typename T>
 struct TailLevel {
-    BoxDims b;
+    BoxDims b;                      // nx = 0: a matched level, its aggregation in the arrays
     Mat<T> A;
     const T *dinv;
+    const int *agg, *aptr, *amem;
+    int nc;
 };
 
 template <typename T>
@@ -2343,29 +2413,29 @@ struct TailRows {
             di[r] = in ? L.dinv[i] : (T)0;
         }
     }
-    __device__ __forceinline__ double ax(const TailLevel<T> &L, const T *s, int r, int i) const
+    __device__ __forceinline__ double ax(const TailLevel<T> &L, const double *s, int r, int i) const
     {
         double acc = 0.0;
 #pragma unroll
         for (int d = 0; d < 7; d++) {
             T av = a[r][d];
             if constexpr (sizeof(T) == 4) asm volatile("" : "+v"(av));   // converted here, not kept as a double
-            acc = fma((double)av, (double)s[clampi(i + L.A.off[d], L.A.n)], acc);
+            acc = fma((double)av, s[clampi(i + L.A.off[d], L.A.n)], acc);
         }
         return acc;
     }
-    __device__ __forceinline__ void put(const TailLevel<T> &L, T *s, const T (&v)[R]) const
+    __device__ __forceinline__ void put(const TailLevel<T> &L, double *s, const T (&v)[R]) const
     {
         const int tid = tail_tid();
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const int i = tid + TAIL_THREADS * r;
-            if (i < L.A.n) s[i] = v[r];
+            if (i < L.A.n) s[i] = (double)v[r];
         }
     }
     // x <- x + omega D^-1 (b - A x), x also in s (which the caller's barrier
     // has made visible); leaves the new x in s
-    __device__ __forceinline__ void sweep(const TailLevel<T> &L, T *s, T omega)
+    __device__ __forceinline__ void sweep(const TailLevel<T> &L, double *s, T omega)
     {
         const int tid = tail_tid();
 #pragma unroll
@@ -2378,7 +2448,7 @@ struct TailRows {
         __syncthreads();
     }
     // pre-smoothing from x = 0, then the residual into s
-    __device__ __forceinline__ void down(const TailLevel<T> &L, T *s, const double *w, int nu)
+    __device__ __forceinline__ void down(const TailLevel<T> &L, double *s, const double *w, int nu)
     {
         const T w1 = (T)w[0], w2 = (T)w[nu >= 2 ? 1 : 0];
 #pragma unroll
@@ -2409,7 +2479,7 @@ struct TailRows {
         __syncthreads();
     }
     // prolongation from the next level's solution xc, post-smoothing
-    __device__ __forceinline__ void up(const TailLevel<T> &L, T *s, const T *xc, T cs, const double *w, int nu)
+    __device__ __forceinline__ void up(const TailLevel<T> &L, double *s, const double *xc, T cs, const double *w, int nu)
     {
         const BoxDims &b_ = L.b;
         const int tid = tail_tid();
@@ -2417,8 +2487,14 @@ struct TailRows {
         for (int r = 0; r < R; r++) {
             const int i = tid + TAIL_THREADS * r;
             if (i < L.A.n) {
-                const int X = i % b_.nx, q = i / b_.nx, Y = q % b_.ny, Z = q / b_.ny;
-                x[r] = vc_prolong(x[r], cs, xc[(X >> b_.sx) + b_.cx * ((Y >> b_.sy) + b_.cy * (Z >> b_.sz))]);
+                int I;
+                if (b_.nx) {
+                    const int X = i % b_.nx, q = i / b_.nx, Y = q % b_.ny, Z = q / b_.ny;
+                    I = (X >> b_.sx) + b_.cx * ((Y >> b_.sy) + b_.cy * (Z >> b_.sz));
+                } else {
+                    I = L.agg[i];
+                }
+                x[r] = vc_prolong(x[r], cs, (T)xc[I]);
             }
         }
         put(L, s, x);
@@ -2427,29 +2503,62 @@ struct TailRows {
     }
 };
 
-// member sum of coarse cell I over residuals s, in k_box_restrict's tree order
-template <typename T>
-__device__ __forceinline__ T tail_restrict(const BoxDims &b, const T *s, int I)
-{
-    const int X = I % b.cx, q = I / b.cx, Y = q % b.cy, Z = q / b.cy;
-    double v[8];
+// The members of coarse row tid, found before the level's sweeps, and the sum
+// of their residuals: a box level's in k_box_restrict's tree order, a matched
+// level's in member order (k_resid_restrict_seq).
+struct TailMembers {
+    unsigned m[4];   // two 16-bit rows each, 0xffff: none
+    template <typename T>
+    __device__ __forceinline__ void load(const TailLevel<T> &L)
+    {
+        const int I = tail_tid();
+        const BoxDims &b = L.b;
 #pragma unroll
-    for (int m = 0; m < 8; m++) {
-        const int i = m & 1, j = (m >> 1) & 1, k = m >> 2;
-        const int x = (X << b.sx) + i, y = (Y << b.sy) + j, z = (Z << b.sz) + k;
-        const bool in = i <= b.sx && j <= b.sy && k <= b.sz && x < b.nx && y < b.ny && z < b.nz;
-        v[m] = in ? (double)s[x + b.nx * (y + b.ny * z)] : 0.0;
+        for (int q = 0; q < 4; q++) m[q] = 0xffffffffu;
+        if (I >= L.nc) return;
+        if (b.nx) {
+            const int X = I % b.cx, q = I / b.cx, Y = q % b.cy, Z = q / b.cy;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const int i = e & 1, j = (e >> 1) & 1, k = e >> 2;
+                const int x = (X << b.sx) + i, y = (Y << b.sy) + j, z = (Z << b.sz) + k;
+                if (i <= b.sx && j <= b.sy && k <= b.sz && x < b.nx && y < b.ny && z < b.nz) put(e, x + b.nx * (y + b.ny * z));
+            }
+        } else {
+            const int t0 = L.aptr[I], cnt = L.aptr[I + 1] - t0;
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (e < cnt) put(e, L.amem[t0 + e]);
+        }
     }
-    return (T)(((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
-}
+    __device__ __forceinline__ void put(int e, int i)
+    {
+        if (e & 1) m[e >> 1] = (m[e >> 1] & 0xffffu) | ((unsigned)i << 16);
+        else m[e >> 1] = (m[e >> 1] & 0xffff0000u) | (unsigned)i;
+    }
+    __device__ __forceinline__ double sum(const double *s, bool tree) const
+    {
+        double v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const unsigned i = (e & 1) ? m[e >> 1] >> 16 : m[e >> 1] & 0xffffu;
+            v[e] = i != 0xffffu ? s[i] : 0.0;
+        }
+        if (tree) return (((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
+        double t = 0.0;
+#pragma unroll
+        for (int e = 0; e < 8; e++) t += v[e];
+        return t;
+    }
+};
 
 template <int R0, bool SYM, typename T>
-__global__ void __launch_bounds__(TAIL_THREADS) k_box_tail(TailArgs<T> a, const KState *stop)
+__global__ void __launch_bounds__(TAIL_THREADS) k_dia_tail(TailArgs<T> a, const KState *stop)
 {
     if (stop && stop->all_done) return;
-    __shared__ T s0[R0 * TAIL_THREADS], s1[tail_cap(1)], s2[tail_cap(2)];
+    __shared__ double s0[R0 * TAIL_THREADS], s1[tail_cap(1)], s2[tail_cap(2)];
     __shared__ double bs[DENSE_MAX];
-    __shared__ T xd[DENSE_MAX];
+    __shared__ double xd[DENSE_MAX];
     __shared__ double part[TAIL_THREADS / DENSE_MAX][DENSE_MAX];
     const int tid = threadIdx.x, nu = a.nu, nl = a.nl;
     TailRows<R0, SYM, T> r0;
@@ -2460,17 +2569,21 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_box_tail(TailArgs<T> a, const 
         const int i = tid + TAIL_THREADS * r;
         r0.b[r] = i < a.lv[0].A.n ? a.b[i] : (T)0;
     }
+    TailMembers mem;   // of the level being left
+    mem.load(a.lv[0]);
     if (nl > 1) r1.load(a.lv[1]);
-    const T *rs = s0;   // the last smoothed level's residuals
+    const double *rs = s0;   // the last smoothed level's residuals
     r0.down(a.lv[0], s0, a.w, nu);
     if (nl > 1) {
-        r1.b[0] = tid < a.lv[1].A.n ? tail_restrict(a.lv[0].b, s0, tid) : (T)0;
+        r1.b[0] = (T)mem.sum(s0, a.lv[0].b.nx != 0);   // (zero beyond the level's rows)
+        mem.load(a.lv[1]);
         r1.down(a.lv[1], s1, a.w, nu);
         rs = s1;
     }
     if (nl > 2) {
         r2.load(a.lv[2]);
-        r2.b[0] = tid < a.lv[2].A.n ? tail_restrict(a.lv[1].b, s1, tid) : (T)0;
+        r2.b[0] = (T)mem.sum(s1, a.lv[1].b.nx != 0);
+        mem.load(a.lv[2]);
         r2.down(a.lv[2], s2, a.w, nu);
         rs = s2;
     }
@@ -2478,7 +2591,7 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_box_tail(TailArgs<T> a, const 
         constexpr int PARTS = TAIL_THREADS / DENSE_MAX, PLEN = DENSE_MAX / PARTS;
         const int nd = a.nd;
         const int i = tid % DENSE_MAX, p = tid / DENSE_MAX;
-        if (tid < nd) bs[tid] = (double)tail_restrict(a.lv[nl - 1].b, rs, tid);
+        if (tid < nd) bs[tid] = (double)(T)mem.sum(rs, a.lv[nl - 1].b.nx != 0);
         __syncthreads();
         double sum = 0.0;
         if (i < nd) {
@@ -2494,7 +2607,7 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_box_tail(TailArgs<T> a, const 
             double y = 0.0;
 #pragma unroll
             for (int q = 0; q < PARTS; q++) y += part[q][tid];
-            xd[tid] = (T)y;
+            xd[tid] = (double)(T)y;
         }
         __syncthreads();
     }
@@ -2516,15 +2629,17 @@ static int tail_launch(Ctx *c, size_t l, const T *b, T *x, int nu, const double 
     const size_t nl = c->amg.size() - 1 - l;
     if (!c->opt.amg_tail || l == 0 || nl == 0 || nl > (size_t)TAIL_LEVELS || nu > 8) return MC_OK;
     for (size_t k = 0; k < nl; k++) {
-        const AmgLevel &L = c->amg[l + k];
-        if (!L.bx || L.n > (k ? tail_cap((int)k) : tail_rows<T>())) return MC_OK;
+        AmgLevel &L = c->amg[l + k];
+        if (nd_code(level_mat<T>(L)) != (sizeof(T) == 8 ? -7 : 7)) return MC_OK;
+        if (L.n > (k ? tail_cap((int)k) : tail_rows<T>()) || L.nc > TAIL_THREADS) return MC_OK;
     }
     TailArgs<T> ta;
     memset(&ta, 0, sizeof(ta));
     ta.nl = (int)nl;
     for (size_t k = 0; k < nl; k++) {
         AmgLevel &L = c->amg[l + k];
-        ta.lv[k].b = box_dims(L);
+        if (L.bx) ta.lv[k].b = box_dims(L);
+        ta.lv[k].agg = L.agg; ta.lv[k].aptr = L.agg_ptr; ta.lv[k].amem = L.agg_members; ta.lv[k].nc = L.nc;
         ta.lv[k].A = level_mat<T>(L);
         ta.lv[k].dinv = lv_dinv<T>(L);
     }
@@ -2536,11 +2651,11 @@ static int tail_launch(Ctx *c, size_t l, const T *b, T *x, int nu, const double 
     constexpr bool SYM = sizeof(T) == 8;   // the FP64 levels keep the upper diagonals
     const dim3 one(1), thr(TAIL_THREADS);
     const int n0 = c->amg[l].n;
-    if (n0 <= TAIL_THREADS) hipLaunchKernelGGL((k_box_tail<1, SYM, T>), one, thr, 0, c->stream, ta, stop);
-    else if (n0 <= 2 * TAIL_THREADS) hipLaunchKernelGGL((k_box_tail<2, SYM, T>), one, thr, 0, c->stream, ta, stop);
-    else if (n0 <= 4 * TAIL_THREADS) hipLaunchKernelGGL((k_box_tail<4, SYM, T>), one, thr, 0, c->stream, ta, stop);
+    if (n0 <= TAIL_THREADS) hipLaunchKernelGGL((k_dia_tail<1, SYM, T>), one, thr, 0, c->stream, ta, stop);
+    else if (n0 <= 2 * TAIL_THREADS) hipLaunchKernelGGL((k_dia_tail<2, SYM, T>), one, thr, 0, c->stream, ta, stop);
+    else if (n0 <= 4 * TAIL_THREADS) hipLaunchKernelGGL((k_dia_tail<4, SYM, T>), one, thr, 0, c->stream, ta, stop);
     else if constexpr (sizeof(T) == 4)
-        hipLaunchKernelGGL((k_box_tail<8, SYM, T>), one, thr, 0, c->stream, ta, stop);
+        hipLaunchKernelGGL((k_dia_tail<5, SYM, T>), one, thr, 0, c->stream, ta, stop);
     MC_LAUNCH_CHECK(c);
     *done = true;
     return MC_OK;
@@ -2562,32 +2677,37 @@ static int vcycle(Ctx *c, size_t l, const T *b, T *x, KState *ks, const KState *
     }
     if (l >= 1 && l + 1 < c->amg.size() && c->opt.amg_tail && !L.bx) {
         // the rest of the cycle in one workgroup when every level left is
-        // small and in diagonal storage of one kind
+        // small and in seven-diagonal or CSR storage
         const size_t nl = c->amg.size() - 1 - l;
-        const int code = nd_code(level_mat<T>(L));
-        bool ok = nl <= (size_t)VT_LEVELS && (code == 7 || code == -7) && nu <= 8 && b == lv_b<T>(L) &&
-                  x == lv_x<T>(L);
-        for (size_t k = l; ok && k + 1 < c->amg.size(); k++)
-            ok = c->amg[k].n <= VT_ROWS && nd_code(level_mat<T>(c->amg[k])) == code;
+        bool ok = nl <= (size_t)VT_LEVELS && nu <= 8 && L.n <= VT_ROWS;
+        int sum = 0;
+        for (size_t k = l; ok && k + 1 < c->amg.size(); k++) {
+            const int code = nd_code(level_mat<T>(c->amg[k]));
+            sum += c->amg[k].n;
+            ok = (code == 0 || code == (sizeof(T) == 8 ? -7 : 7)) && sum <= VT_SUM;
+        }
         if (ok) {
             VtArgs<T> ta;
             memset(&ta, 0, sizeof(ta));
             ta.nl = (int)nl;
+            int off = 0;
             for (size_t k = 0; k < nl; k++) {
                 AmgLevel &Lk = c->amg[l + k];
                 VtLevel<T> &t = ta.lv[k];
                 t.A = level_mat<T>(Lk);
                 t.dinv = lv_dinv<T>(Lk);
-                t.b = lv_b<T>(Lk); t.x = lv_x<T>(Lk); t.t = lv_t<T>(Lk);
                 t.agg = Lk.agg; t.aptr = Lk.agg_ptr; t.amem = Lk.agg_members; t.nc = Lk.nc;
+                t.off = off;
+                t.rpo = off + (int)k;   // n + 1 pointers a level
+                off += Lk.n;
             }
-            AmgLevel &Ld = c->amg.back();
-            ta.lv[nl].b = lv_b<T>(Ld); ta.lv[nl].x = lv_x<T>(Ld);
-            ta.inv = c->amg_dense; ta.nd = Ld.n;
+            ta.b = b; ta.x = x;
+            ta.inv = c->amg_dense; ta.nd = c->amg.back().n;
             ta.nu = nu; ta.cs = (T)c->opt.amg_cscale;
             for (int k = 0; k < 8; k++) ta.w[k] = wts[k];
             MC_TRY(dense_join(c));
-            MC_DISPATCH_ND(code, (k_vtail<ND_, T>), dim3(1), dim3(TAIL_THREADS), 0, c->stream, ta, stop);
+            constexpr bool SYM = sizeof(T) == 8;   // FP64 seven-diagonal levels keep the upper diagonals
+            hipLaunchKernelGGL((k_vtail<SYM, T>), dim3(1), dim3(TAIL_THREADS), 0, c->stream, ta, stop);
             MC_LAUNCH_CHECK(c);
             return MC_OK;
         }

@@ -53,3 +53,24 @@ def test_box_tail_is_the_same_cycle(m, psolve):
             out[tail] = (x.copy(), st.iterations)
     assert out[0][1] == out[1][1]
     assert_bits(out[1][0], out[0][0], "pressure correction, tail vs per-pass launches")
+
+
+@pytest.mark.parametrize("psolve", [mc.PSOLVE_FP64, mc.PSOLVE_MIXED])
+@pytest.mark.parametrize("m", [5, 9, 10, 11, 17, 23, 33, 40])
+def test_matched_tail_is_the_same_cycle(m, psolve):
+    """The hierarchy of looser solves (pairwise matching): levels in diagonal
+    and in CSR storage, with and without the single-workgroup tail."""
+    print("matched tail m=%d psolve=%d" % (m, psolve), flush=True)
+    out = {}
+    for tail in (0, 1):
+        with mc.Context(m, mode=mc.MODE_SIMPLE, psolve=psolve, p_rtol=1e-8, amg_tail=tail) as g:
+            rng = np.random.default_rng(m)
+            x = np.arange(g.N) % (2 * m)
+            g.set(mc.ARR_AU, np.concatenate([10.0 + 3.0 * np.exp(-0.2 * x) + 0.01 * np.sin(np.arange(g.N)), np.zeros(6)]))
+            g.pressure_assemble()
+            b = rng.standard_normal(g.N)
+            sol, st = g.solve_pressure(b - b.mean())
+            assert st.converged
+            out[tail] = (sol.copy(), st.iterations)
+    assert out[0][1] == out[1][1]
+    assert_bits(out[1][0], out[0][0], "pressure correction, tail vs per-pass launches")
