@@ -165,6 +165,7 @@ static int alloc_workspace(Ctx *c)
 static int finish_ctor(Ctx *c)
 {
     MC_TRY(mesh_finish(c));
+    MC_TRY(box_tables(c));
     MC_TRY(alloc_workspace(c));
     MC_TRY(dia_setup_fine(c));
     c->first_pressure = true;
@@ -623,6 +624,7 @@ int mc_array_set(mc_ctx *x, int id, const void *host, int64_t count)
 {
     CTX_OR_FAIL
     c->pa_dia_fresh = false;   // the AMG fine level is refreshed from whatever the arrays now hold
+    if (id >= MC_ARR_FACE_AREA && id <= MC_ARR_CELL_DENSITY) c->box.ok = false;   // the caller's geometry from here on
     ArrDesc d;
     MC_TRY(describe(c, id, d));
     if (!host || count != d.count) { c->err = "array size mismatch (expected " + std::to_string(d.count) + ")"; return MC_ERR_ARG; }

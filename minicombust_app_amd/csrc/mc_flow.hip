@@ -127,6 +127,152 @@ static Sizes sizes_of(const Ctx *c)
     return Sizes{(double)c->N, (double)c->F, (double)(c->F - c->Fb), (double)c->Fb, (double)c->nnz};
 }
 
+// ============================================== generated-box kernels ==
+// The assembly kernels above for a generated box whose geometry is in tables
+// (Ctx::box).  They are bound by the latency of dependent gathers (a cell's
+// face ids and fother codes, then per face the neighbour's values and 7 to 14
+// geometry values) and re-read face geometry from both sides.  Here neighbours
+// and face positions are arithmetic and geometry comes from per-axis tables of
+// a few hundred values, so every field value a cell needs is asked for at once
+// and only field data crosses HBM.  On a face normal to an axis only that
+// component of a normal or of a centre-to-centre vector is nonzero, so only
+// that component of a neighbour's gradient is read: the products left out are
+// signed zeros for finite operands and leave sums that start at +0 unchanged.
+// Faces are visited in ascending reference id as everywhere (low z, y, x of
+// interior faces, then the cell's own in side order with low boundary faces at
+// their sides' places), so the results are the general kernels' bit for bit.
+//
+// m = 128 (4,194,304 cells), general -> box kernels, us: k_grad<11> 570 -> 466,
+// k_grad<1> 120 -> 65, k_momentum 635 -> 390, k_scalar 495 -> 281 (mean of TE
+// and ED), k_scalar_batch<true> beside the ED solve 1200 -> 753, k_mass_faces
+// 487 -> 274, k_mass_rows 274 -> 260, k_flux_correct 282 -> 134,
+// k_cell_correct 145 -> 98.  They move little beyond what they must (momentum:
+// 0.86 GB read and 0.67 written of 0.80 + 0.67) at 3 to 4 TB/s, with up to 44
+// separate streams each.
+struct BoxG {
+    int nx, ny, nz, N, nxny;
+    const double *cc[3], *w[3], *lam[3], *dist[3], *fc[3], *ft[3][3], *vis[3];
+    double zero[3][3], rho;
+    // boundary faces keep the arrays
+    const double *fcx, *fcy, *fcz, *fnx, *fny, *fnz, *farea, *frlc;
+    int btype[6], last_face[6];
+    CellWalk wk;
+};
+
+static bool box_on(const Ctx *c) { return c->box.ok && c->fine_nd == 7; }
+
+static BoxG box_geo(const Ctx *c, int vis = 0)
+{
+    BoxG g;
+    const Ctx::BoxTables &b = c->box;
+    g.nx = b.n[0]; g.ny = b.n[1]; g.nz = b.n[2]; g.N = c->N; g.nxny = g.nx * g.ny;
+    for (int a = 0; a < 3; a++) {
+        g.cc[a] = b.cc[a]; g.w[a] = b.w[a]; g.lam[a] = b.lam[a]; g.dist[a] = b.dist[a]; g.fc[a] = b.fc[a];
+        g.vis[a] = b.vis[vis][a];
+        for (int e = 0; e < 3; e++) { g.ft[a][e] = b.ft[a][e]; g.zero[a][e] = b.zero[a][e]; }
+    }
+    g.rho = b.rho;
+    g.fcx = c->fcx; g.fcy = c->fcy; g.fcz = c->fcz; g.fnx = c->fnx; g.fny = c->fny; g.fnz = c->fnz;
+    g.farea = c->farea; g.frlc = c->frlc;
+    for (int s = 0; s < 6; s++) { g.btype[s] = c->btype[s]; g.last_face[s] = c->last_face[s]; }
+    g.wk = cell_walk(c);
+    return g;
+}
+
+// A cell of the box, its neighbours by side (FRONT -z, BACK +z, LEFT -x, RIGHT
+// +x, DOWN -y, UP +y; the cell itself where there is none) and the storage
+// positions of its faces.
+struct BoxCell {
+    int c, x[3];
+    bool in[6];      // the side's face is interior
+    int nb[6], f[6];
+};
+__device__ __forceinline__ bool box_cell(const BoxG &g, BoxCell &q)
+{
+    q.c = walk_xyz_at(g.wk, xcd_block(blockIdx.x, gridDim.x), threadIdx.x, q.x[0], q.x[1], q.x[2]);
+    if (q.c < 0) return false;
+    const int c = q.c, x = q.x[0], y = q.x[1], z = q.x[2], N = g.N;
+    q.in[0] = z > 0; q.in[1] = z + 1 < g.nz; q.in[2] = x > 0; q.in[3] = x + 1 < g.nx; q.in[4] = y > 0; q.in[5] = y + 1 < g.ny;
+    q.nb[0] = q.in[0] ? c - g.nxny : c; q.nb[1] = q.in[1] ? c + g.nxny : c;
+    q.nb[2] = q.in[2] ? c - 1 : c;      q.nb[3] = q.in[3] ? c + 1 : c;
+    q.nb[4] = q.in[4] ? c - g.nx : c;   q.nb[5] = q.in[5] ? c + g.nx : c;
+    q.f[0] = q.in[0] ? 2 * N + c - g.nxny : 3 * N + g.ny * g.nz + g.nx * g.nz + x + g.nx * y;
+    q.f[1] = 2 * N + c;
+    q.f[2] = q.in[2] ? c - 1 : 3 * N + y + g.ny * z;
+    q.f[3] = c;
+    q.f[4] = q.in[4] ? N + c - g.nx : 3 * N + g.ny * g.nz + x + g.nx * z;
+    q.f[5] = N + c;
+    return true;
+}
+
+template <int S> struct SideTag { static constexpr int side = S, axis = S < 2 ? 2 : S < 4 ? 0 : 1; static constexpr bool high = S & 1; };
+
+// the cell's faces in ascending reference id: fi(SideTag) for interior ones,
+// fb(side) for boundary ones
+template <class FI, class FB>
+__device__ __forceinline__ void box_faces(const BoxCell &q, FI fi, FB fb)
+{
+    if (q.in[0]) fi(SideTag<0>());
+    if (q.in[4]) fi(SideTag<4>());
+    if (q.in[2]) fi(SideTag<2>());
+    if (!q.in[0]) fb(0);
+    if (q.in[1]) fi(SideTag<1>()); else fb(1);
+    if (!q.in[2]) fb(2);
+    if (q.in[3]) fi(SideTag<3>()); else fb(3);
+    if (!q.in[4]) fb(4);
+    if (q.in[5]) fi(SideTag<5>()); else fb(5);
+}
+
+// interior face across a side: weight of cell0, area, distance, viscosity
+struct BoxFace {
+    double l0, l1, area, dist, vis;
+};
+template <class TAG>
+__device__ __forceinline__ BoxFace box_face(const BoxG &g, const BoxCell &q, const double (&area)[3], TAG)
+{
+    constexpr int a = TAG::axis;
+    const int t = TAG::high ? q.x[a] : q.x[a] - 1;
+    BoxFace f;
+    f.l0 = g.lam[a][t];
+    f.l1 = 1.0 - f.l0;
+    f.area = area[a];
+    f.dist = g.dist[a][t];
+    f.vis = g.vis[a][t];
+    return f;
+}
+__device__ __forceinline__ void box_areas(const BoxG &g, const BoxCell &q, double (&area)[3], double &vol)
+{
+    const double w0 = g.w[0][q.x[0]], w1 = g.w[1][q.x[1]], w2 = g.w[2][q.x[2]];
+    area[0] = w1 * w2; area[1] = w2 * w0; area[2] = w0 * w1;
+    vol = w0 * w1 * w2;
+}
+
+// Row of a momentum / scalar matrix: seven diagonals -z -y -x main +x +y +z.
+__device__ __forceinline__ void box_store_row(const BoxG &g, const BoxCell &q, const double (&ff)[6], double diag,
+                                              double *dia)
+{
+    const size_t N = (size_t)g.N;
+    const int c = q.c;
+    if (q.in[0]) st_out(&dia[c], ff[0]);
+    if (q.in[4]) st_out(&dia[N + c], ff[4]);
+    if (q.in[2]) st_out(&dia[2 * N + c], ff[2]);
+    st_out(&dia[3 * N + c], diag);
+    if (q.in[3]) st_out(&dia[4 * N + c], ff[3]);
+    if (q.in[5]) st_out(&dia[5 * N + c], ff[5]);
+    if (q.in[1]) st_out(&dia[6 * N + c], ff[1]);
+}
+// diag - off-diagonals, in the visiting order of the interior faces
+__device__ __forceinline__ double box_minus_off(const BoxCell &q, const double (&ff)[6], double A)
+{
+    if (q.in[0]) A -= ff[0];
+    if (q.in[4]) A -= ff[4];
+    if (q.in[2]) A -= ff[2];
+    if (q.in[1]) A -= ff[1];
+    if (q.in[3]) A -= ff[3];
+    if (q.in[5]) A -= ff[5];
+    return A;
+}
+
 // ========================================================== A4 / A5 ==
 struct GradArgs {
     const double *phi[11];
@@ -270,12 +416,70 @@ __global__ void __launch_bounds__(256) k_limit(Geo g, GradArgs a)
     }
 }
 
+// ---- gradients (k_grad) ----
+template <int NF>
+__global__ void __launch_bounds__(256) k_box_grad(BoxG g, GradArgs a)
+{
+    BoxCell q;
+    if (!box_cell(g, q)) return;
+    const int c = q.c;
+    const dv3 cc = v3(g.cc[0][q.x[0]], g.cc[1][q.x[1]], g.cc[2][q.x[2]]);
+    dv3 dX[6];
+    int at[6];   // the value across the side: the neighbour's, or the side's slot
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+        const int ax = s < 2 ? 2 : s < 4 ? 0 : 1;
+        if (q.in[s]) {
+            const double d = g.cc[ax][(s & 1) ? q.x[ax] + 1 : q.x[ax] - 1] - (ax == 0 ? cc.x : ax == 1 ? cc.y : cc.z);
+            dX[s] = v3(ax == 0 ? d : 0.0, ax == 1 ? d : 0.0, ax == 2 ? d : 0.0);
+            at[s] = q.nb[s];
+        } else {
+            dX[s] = ld3(g.fcx, g.fcy, g.fcz, q.f[s]) - cc;
+            at[s] = g.N + s;
+        }
+    }
+    double a00 = 0.0, a10 = 0.0, a20 = 0.0, a11 = 0.0, a21 = 0.0, a22 = 0.0;
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+        a00 += (dX[s].x * dX[s].x); a10 += (dX[s].x * dX[s].y); a20 += (dX[s].x * dX[s].z);
+        a11 += (dX[s].y * dX[s].y); a21 += (dX[s].y * dX[s].z); a22 += (dX[s].z * dX[s].z);
+    }
+    const double A00 = a00, A01 = a10, A02 = a20, A10 = a10, A11 = a11, A12 = a21, A20 = a20, A21 = a21, A22 = a22;
+    const double det = (A00 * (A11 * A22 - A21 * A12)) - (A01 * (A10 * A22 - A20 * A12)) +
+                       (A02 * (A10 * A21 - A20 * A11));
+    double invdet = 0.0;
+    if (det != 0.0) invdet = 1 / det;
+    const double c00 = (A11 * A22 - A21 * A12), c01 = (A21 * A02 - A01 * A22), c02 = (A01 * A12 - A11 * A02);
+    const double c10 = (A12 * A20 - A10 * A22), c11 = (A00 * A22 - A20 * A02), c12 = (A10 * A02 - A00 * A12);
+    const double c20 = (A10 * A21 - A20 * A11), c21 = (A20 * A01 - A00 * A21), c22 = (A00 * A11 - A10 * A01);
+#pragma unroll
+    for (int k = 0; k < NF; k++) {
+        const double *phi = a.phi[k];
+        const double ph = phi[c];
+        double v[6];
+#pragma unroll
+        for (int s = 0; s < 6; s++) v[s] = phi[at[s]];
+        double bx = 0.0, by = 0.0, bz = 0.0;
+#pragma unroll
+        for (int s = 0; s < 6; s++) {
+            const double d = (!q.in[s] && a.zero_boundary[k]) ? 0.0 : v[s] - ph;
+            bx += (dX[s].x * d); by += (dX[s].y * d); bz += (dX[s].z * d);
+        }
+        const double gx = (bx * invdet * c00) + (by * invdet * c01) + (bz * invdet * c02);
+        const double gy = (bx * invdet * c10) + (by * invdet * c11) + (bz * invdet * c12);
+        const double gz = (bx * invdet * c20) + (by * invdet * c21) + (bz * invdet * c22);
+        st_out(&a.gx[k][c], gx); st_out(&a.gy[k][c], gy); st_out(&a.gz[k][c], gz);
+    }
+}
+
 // k_grad<NF>: per cell phi (8 NF) read, gradients (24 NF) written, centre
 // (24), neighbour list (24); per boundary face cell_faces and fc1 entries (8)
-// and the face centre (24).
+// and the face centre (24).  k_box_grad<NF>: the cell's fields and gradients
+// and the boundary faces' centres.
 static double grad_bytes(Ctx *c, int nf)
 {
     const Sizes z = sizes_of(c);
+    if (box_on(c)) return 32.0 * nf * z.N + 24.0 * z.Fb;
     return (32.0 * nf + 48.0) * z.N + 32.0 * z.Fb;
 }
 
@@ -295,7 +499,9 @@ int grad_multi(Ctx *c, bool limit)
 {
     const GradArgs a = grad11_args(c);
     KTimer kt(c, MC_KC_GRAD, grad_bytes(c, 11));
-    if (limit)
+    if (!limit && box_on(c))
+        hipLaunchKernelGGL(k_box_grad<11>, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, box_geo(c), a);
+    else if (limit)
         hipLaunchKernelGGL((k_grad<11, true>), dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, geo(c), a);
     else
         hipLaunchKernelGGL((k_grad<11, false>), dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, geo(c), a);
@@ -318,7 +524,10 @@ int grad_single(Ctx *c, int field, bool pressure)
     a.gx[0] = c->gx[field]; a.gy[0] = c->gy[field]; a.gz[0] = c->gz[field];
     a.zero_boundary[0] = pressure ? 1 : 0;
     KTimer kt(c, MC_KC_GRAD1, grad_bytes(c, 1));
-    hipLaunchKernelGGL(k_grad<1>, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, geo(c), a);
+    if (box_on(c))
+        hipLaunchKernelGGL(k_box_grad<1>, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, box_geo(c), a);
+    else
+        hipLaunchKernelGGL(k_grad<1>, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, geo(c), a);
     MC_LAUNCH_CHECK(c);
     return MC_OK;
 }
@@ -515,6 +724,151 @@ __global__ void __launch_bounds__(256) k_momentum(Geo g, MomArgs a)
     store_row(g, c, nint, own_nb, own_ff, A, a.vals, a.dia);
 }
 
+// ---- momentum (k_momentum) ----
+__global__ void __launch_bounds__(256) k_box_momentum(BoxG g, MomArgs a)
+{
+    BoxCell q;
+    if (!box_cell(g, q)) return;
+    const int c = q.c, N = g.N;
+    double SU = 0.0, SV = 0.0, SW = 0.0, A = 0.0;
+    double xU = 0.0, xV = 0.0, xW = 0.0;
+    double ff[6];
+    const dv3 gUc = ld3(a.gUx, a.gUy, a.gUz, c), gVc = ld3(a.gVx, a.gVy, a.gVz, c), gWc = ld3(a.gWx, a.gWy, a.gWz, c);
+    const double Uc = a.U[c], Vc = a.V[c], Wc = a.W[c];
+    double mf[6];
+#pragma unroll
+    for (int s = 0; s < 6; s++) mf[s] = a.mflux[q.f[s]];
+    double area[3], vol;
+    box_areas(g, q, area, vol);
+    auto fi = [&](auto tag) {
+        using TAG = decltype(tag);
+        constexpr int s = TAG::side, ax = TAG::axis;
+        const int nb = q.nb[s];
+        const BoxFace f = box_face(g, q, area, tag);
+        // face gradients by weight: cell0 is the cell on a high side
+        auto mix = [&](double own, double oth) {
+            return TAG::high ? own * f.l0 + oth * f.l1 : oth * f.l0 + own * f.l1;
+        };
+        const double VisFace = f.vis * (f.area / f.dist);
+        const double Un = a.U[nb], Vn = a.V[nb], Wn = a.W[nb];
+        double fude, fvde, fwde, fudi, fvdi, fwdi;
+        if constexpr (ax == 0) {
+            const double Ux = mix(gUc.x, a.gUx[nb]), Uy = mix(gUc.y, a.gUy[nb]), Uz = mix(gUc.z, a.gUz[nb]);
+            const double Vx = mix(gVc.x, a.gVx[nb]), Wx = mix(gWc.x, a.gWx[nb]);
+            fude = f.vis * ((Ux + Ux) * f.area);
+            fvde = f.vis * ((Uy + Vx) * f.area);
+            fwde = f.vis * ((Uz + Wx) * f.area);
+            fudi = VisFace * (Ux * f.dist); fvdi = VisFace * (Vx * f.dist); fwdi = VisFace * (Wx * f.dist);
+        } else if constexpr (ax == 1) {
+            const double Uy = mix(gUc.y, a.gUy[nb]), Wy = mix(gWc.y, a.gWy[nb]);
+            const double Vx = mix(gVc.x, a.gVx[nb]), Vy = mix(gVc.y, a.gVy[nb]), Vz = mix(gVc.z, a.gVz[nb]);
+            fude = f.vis * ((Uy + Vx) * f.area);
+            fvde = f.vis * ((Vy + Vy) * f.area);
+            fwde = f.vis * ((Wy + Vz) * f.area);
+            fudi = VisFace * (Uy * f.dist); fvdi = VisFace * (Vy * f.dist); fwdi = VisFace * (Wy * f.dist);
+        } else {
+            const double Uz = mix(gUc.z, a.gUz[nb]), Vz = mix(gVc.z, a.gVz[nb]);
+            const double Wx = mix(gWc.x, a.gWx[nb]), Wy = mix(gWc.y, a.gWy[nb]), Wz = mix(gWc.z, a.gWz[nb]);
+            fude = f.vis * ((Uz + Wx) * f.area);
+            fvde = f.vis * ((Vz + Wy) * f.area);
+            fwde = f.vis * ((Wz + Wz) * f.area);
+            fudi = VisFace * (Uz * f.dist); fvdi = VisFace * (Vz * f.dist); fwdi = VisFace * (Wz * f.dist);
+        }
+        const double ff0 = -VisFace - dmax(mf[s], 0.0);
+        const double ff1 = -VisFace + dmin(mf[s], 0.0);
+        if constexpr (TAG::high) {
+            SU = SU + fude - fudi;
+            SV = SV + fvde - fvdi;
+            SW = SW + fwde - fwdi;
+            ff[s] = ff1;
+            st_out(&a.ff0[q.f[s]], ff0); st_out(&a.ff1[q.f[s]], ff1);
+        } else {
+            SU = SU - fude + fudi;
+            SV = SV - fvde + fvdi;
+            SW = SW - fwde + fwdi;
+            ff[s] = ff0;
+        }
+        xU += ff[s] * Un; xV += ff[s] * Vn; xW += ff[s] * Wn;
+    };
+    auto fb = [&](int side) {
+        const int f = side == 0 ? q.f[0] : side == 1 ? q.f[1] : side == 2 ? q.f[2] : side == 3 ? q.f[3] : side == 4 ? q.f[4] : q.f[5];
+        const int bt = g.btype[side];
+        const dv3 cc = v3(g.cc[0][q.x[0]], g.cc[1][q.x[1]], g.cc[2][q.x[2]]);
+        const dv3 Xpn = ld3(g.fcx, g.fcy, g.fcz, f) - cc;
+        const bool last = (f == g.last_face[side]);
+        if (bt == INLET || bt == OUTLET) {
+            const dv3 dUdXac = gUc, dVdXac = gVc, dWdXac = gWc;
+            double UFace, VFace, WFace, Visac;
+            if (bt == INLET) {
+                UFace = a.vel_x; VFace = a.vel_y; WFace = a.vel_z; Visac = a.inlet_ev;
+            } else {
+                Visac = a.ev; UFace = Uc; VFace = Vc; WFace = Wc;
+            }
+            const double VisFace = Visac * g.frlc[f];
+            const double sx = g.fnx[f], sy = g.fny[f], sz = g.fnz[f];
+            const double fude = Visac * ((dUdXac.x + dUdXac.x) * sx + (dUdXac.y + dVdXac.x) * sy + (dUdXac.z + dWdXac.x) * sz);
+            const double fvde = Visac * ((dUdXac.y + dVdXac.x) * sx + (dVdXac.y + dVdXac.y) * sy + (dVdXac.z + dWdXac.y) * sz);
+            const double fwde = Visac * ((dUdXac.z + dWdXac.x) * sx + (dWdXac.y + dVdXac.z) * sy + (dWdXac.z + dWdXac.z) * sz);
+            const double fudi = VisFace * dot(dUdXac, Xpn);
+            const double fvdi = VisFace * dot(dVdXac, Xpn);
+            const double fwdi = VisFace * dot(dWdXac, Xpn);
+            double m = a.mflux[f];
+            if (bt == OUTLET && m < 0.0) { m = 1e-15; a.mflux[f] = m; }   // FlowSolver.inl:1576-1580
+            const double fbc = -VisFace + dmin(m, 0.0);
+            A = A - fbc;
+            SU = SU - fbc * UFace + fude - fudi;
+            SV = SV - fbc * VFace + fvde - fvdi;
+            SW = SW - fbc * WFace + fwde - fwdi;
+            if (last) { a.U[N + side] = UFace; a.V[N + side] = VFace; a.W[N + side] = WFace; }
+        } else if (bt == WALL) {
+            const double Visac = a.ev;
+            const double coef = Visac * g.frlc[f];
+            const dv3 Up = v3(Uc - 0., Vc - 0., Wc - 0.);
+            const dv3 n = ld3(g.fnx, g.fny, g.fnz, f);
+            const dv3 nh = n / mag(n);
+            const double dp = dot(Up, nh);
+            const dv3 Ut = Up - nh * dp;
+            const double Uvel = fabs(Ut.x) + fabs(Ut.y) + fabs(Ut.z);
+            dv3 force = v3(0.0, 0.0, 0.0);
+            if (Uvel > 0.0) {
+                const double distance_to_face = mag(Xpn);
+                force = (Ut * (g.farea[f] * Visac)) / distance_to_face;
+            }
+            A = A + coef;
+            SU = SU + coef * Uc - force.x;
+            SV = SV + coef * Vc - force.y;
+            SW = SW + coef * Wc - force.z;
+            if (last) { a.U[N + side] = 0.; a.V[N + side] = 0.; a.W[N + side] = 0.; }
+        }
+    };
+    box_faces(q, fi, fb);
+    // buoyancy, pressure gradient, transient (FlowSolver.inl:1689-1721)
+    const double rho = g.rho;
+    const double BodyForce = -0.001 * rho * vol * (a.TEM[c] - a.gas_tem);
+    SU += 0.0 * BodyForce;
+    SV += -9.81 * BodyForce;
+    SW += 0.0 * BodyForce;
+    SU -= a.gPx[c] * vol;
+    SV -= a.gPy[c] * vol;
+    SW -= a.gPz[c] * vol;
+    const double fv = rho * vol * a.rdelta;
+    SU += fv * Uc; SV += fv * Vc; SW += fv * Wc;
+    A += fv;
+    A = box_minus_off(q, ff, A);
+    A *= (1. / a.urf);
+    SU = SU + (1.0 - a.urf) * A * Uc;
+    SV = SV + (1.0 - a.urf) * A * Vc;
+    SW = SW + (1.0 - a.urf) * A * Wc;
+    st_out(&a.AU[c], A);
+    st_out(&a.SU[c], SU); st_out(&a.SV[c], SV); st_out(&a.SW[c], SW);
+    if (a.r0[0]) {
+        st_out(&a.r0[0][c], SU - (A * Uc + xU));
+        st_out(&a.r0[1][c], SV - (A * Vc + xV));
+        st_out(&a.r0[2][c], SW - (A * Wc + xW));
+    }
+    box_store_row(g, q, ff, A, a.dia);
+}
+
 static MomArgs mom_args(Ctx *c)
 {
     MomArgs a;
@@ -548,10 +902,13 @@ static int r0_buffers(Ctx *c)
 // A_U, S_U, S_V, S_W (32) and, warm-started, b - A x0 of the three systems
 // (24) written; per face mass flux, lambda, rlencos, normal (48) read; per
 // interior face ff0, ff1 (16) written; per boundary face centre and area
-// (32) read; the matrix entries (8 nnz) written.
+// (32) read; the matrix entries (8 nnz) written.  k_box_momentum: the same
+// without the cells' and interior faces' geometry, forder and fother.
 static double momentum_bytes(Ctx *c, bool r0)
 {
     const Sizes z = sizes_of(c);
+    if (box_on(c))
+        return (160.0 + (r0 ? 24.0 : 0.0)) * z.N + 8.0 * z.F + 16.0 * z.Fi + 64.0 * z.Fb + 8.0 * z.nnz;
     return (248.0 + (r0 ? 24.0 : 0.0)) * z.N + 48.0 * z.F + 16.0 * z.Fi + 32.0 * z.Fb + 8.0 * z.nnz;
 }
 
@@ -563,7 +920,10 @@ int momentum_assemble(Ctx *c, bool r0)
         for (int k = 0; k < 3; k++) a.r0[k] = c->r0buf[k];
     }
     KTimer kt(c, MC_KC_MOM_ASM, momentum_bytes(c, a.r0[0] != nullptr));
-    hipLaunchKernelGGL(k_momentum, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, geo(c), a);
+    if (box_on(c) && a.dia)
+        hipLaunchKernelGGL(k_box_momentum, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, box_geo(c), a);
+    else
+        hipLaunchKernelGGL(k_momentum, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, geo(c), a);
     MC_LAUNCH_CHECK(c);
     return MC_OK;
 }
@@ -717,24 +1077,38 @@ __device__ __forceinline__ RCCell rc_cell(const Geo &g, const MassArgs &a, int i
     return q;
 }
 
+// A face's own values there.
+struct RCFace {
+    double lambda0, area;
+    dv3 fc, n;
+};
+__device__ __forceinline__ RCFace rc_face(const Geo &g, int f)
+{
+    RCFace r;
+    r.lambda0 = g.flam[f]; r.area = g.farea[f];
+    r.fc = ld3(g.fcx, g.fcy, g.fcz, f);
+    r.n = ld3(g.fnx, g.fny, g.fnz, f);
+    return r;
+}
+
 // Rhie-Chow interior mass flux (FlowSolver.inl:1893-1950); q0, q1: the
 // face's cell0 and cell1.
-__device__ __forceinline__ double rhie_chow(const Geo &g, int f, const RCCell &q0, const RCCell &q1, double &ApV_out)
+__device__ __forceinline__ double rhie_chow(const RCFace &rf, const RCCell &q0, const RCCell &q1, double &ApV_out)
 {
-    const double lambda0 = g.flam[f], lambda1 = 1.0 - lambda0;
+    const double lambda0 = rf.lambda0, lambda1 = 1.0 - lambda0;
     const dv3 dUdXac = q0.gU * lambda0 + q1.gU * lambda1;
     const dv3 dVdXac = q0.gV * lambda0 + q1.gV * lambda1;
     const dv3 dWdXac = q0.gW * lambda0 + q1.gW * lambda1;
     const dv3 cc0 = q0.cc, cc1 = q1.cc;
     const dv3 Xac = cc1 * lambda1 + cc0 * lambda0;
-    const dv3 fc = ld3(g.fcx, g.fcy, g.fcz, f);
+    const dv3 fc = rf.fc;
     const dv3 delta = fc - Xac;
     const double UFace = q1.U * lambda1 + q0.U * lambda0 + dot(dUdXac, delta);
     const double VFace = q1.V * lambda1 + q0.V * lambda0 + dot(dVdXac, delta);
     const double WFace = q1.W * lambda1 + q0.W * lambda0 + dot(dWdXac, delta);
     const double rho0 = q0.rho, rho1 = q1.rho;
     const double densityf = rho0 * lambda0 + rho1 * lambda1;
-    const dv3 n = ld3(g.fnx, g.fny, g.fnz, f);
+    const dv3 n = rf.n;
     double m = densityf * (UFace * n.x + VFace * n.y + WFace * n.z);
     const dv3 nh = n / mag(n);
     const dv3 Xpac = fc - nh * dot(fc - cc0, nh);
@@ -750,7 +1124,7 @@ __device__ __forceinline__ double rhie_chow(const Geo &g, int f, const RCCell &q
     const double ApV1 = (A1 != 0.0) ? 1.0 / A1 : 0.0;
     double ApV = rho0 * ApV0 * lambda0 + rho1 * ApV1 * lambda1;
     const double volume_avg = q0.vol * lambda0 + q1.vol * lambda1;
-    ApV = ApV * g.farea[f] * volume_avg / dot(Xpn2, nh);
+    ApV = ApV * rf.area * volume_avg / dot(Xpn2, nh);
     const double dpx = (gP1.x * lambda1 + gP0.x * lambda0) * Xpn.x;
     const double dpy = (gP1.y * lambda1 + gP0.y * lambda0) * Xpn.y;
     const double dpz = (gP1.z * lambda1 + gP0.z * lambda0) * Xpn.z;
@@ -774,7 +1148,7 @@ __global__ void __launch_bounds__(256) k_mass_faces(Geo g, MassArgs a)
         const int f = cf.f[k];
         const RCCell other = rc_cell(g, a, c1);
         double ApV;
-        const double m = rhie_chow(g, f, own, other, ApV);
+        const double m = rhie_chow(rc_face(g, f), own, other, ApV);
         st_out(&a.mflux[f], m);
         st_out(&a.ff0[f], -ApV); st_out(&a.ff1[f], -ApV);
     }
@@ -850,9 +1224,211 @@ __global__ void __launch_bounds__(256) k_mass_rows(Geo g, MassArgs a)
     }
 }
 
+// ---- Rhie-Chow fluxes (k_mass_faces): the faces towards the next cells ----
+__global__ void __launch_bounds__(256) k_box_mass_faces(BoxG g, MassArgs a)
+{
+    BoxCell q;
+    if (!box_cell(g, q)) return;
+    const int c = q.c;
+    double area[3], vol;
+    box_areas(g, q, area, vol);
+    const dv3 cc = v3(g.cc[0][q.x[0]], g.cc[1][q.x[1]], g.cc[2][q.x[2]]);
+    auto cell = [&](int i, const dv3 &x, double v) {
+        RCCell r;
+        r.gU = ld3(a.gUx, a.gUy, a.gUz, i); r.gV = ld3(a.gVx, a.gVy, a.gVz, i); r.gW = ld3(a.gWx, a.gWy, a.gWz, i);
+        r.gP = ld3(a.gPx, a.gPy, a.gPz, i); r.cc = x;
+        r.U = a.U[i]; r.V = a.V[i]; r.W = a.W[i]; r.P = a.P[i];
+        r.rho = g.rho; r.AU = a.AU[i]; r.vol = v;
+        return r;
+    };
+    const RCCell own = cell(c, cc, vol);
+    auto face = [&](auto tag) {
+        using TAG = decltype(tag);
+        constexpr int ax = TAG::axis, s = TAG::side;
+        const int t = q.x[ax];
+        const double wn = g.w[ax][t + 1];
+        // the neighbour's volume in the order width * height * length
+        const double w0 = ax == 0 ? wn : g.w[0][q.x[0]], w1 = ax == 1 ? wn : g.w[1][q.x[1]], w2 = ax == 2 ? wn : g.w[2][q.x[2]];
+        dv3 xn = cc;
+        const double cn = g.cc[ax][t + 1];
+        if (ax == 0) xn.x = cn; else if (ax == 1) xn.y = cn; else xn.z = cn;
+        const RCCell other = cell(q.nb[s], xn, w0 * w1 * w2);
+        RCFace f;
+        f.lambda0 = g.lam[ax][t];
+        f.fc = v3(ax == 0 ? g.fc[0][t] : g.ft[ax][0][q.x[0]], ax == 1 ? g.fc[1][t] : g.ft[ax][1][q.x[1]],
+                  ax == 2 ? g.fc[2][t] : g.ft[ax][2][q.x[2]]);
+        f.n = v3(ax == 0 ? area[0] : g.zero[ax][0], ax == 1 ? area[1] : g.zero[ax][1], ax == 2 ? area[2] : g.zero[ax][2]);
+        f.area = area[ax];
+        double ApV;
+        const double m = rhie_chow(f, own, other, ApV);
+        st_out(&a.mflux[q.f[s]], m);
+        st_out(&a.ff0[q.f[s]], -ApV); st_out(&a.ff1[q.f[s]], -ApV);
+    };
+    // any order: the faces are independent
+    if (q.in[3]) face(SideTag<3>());
+    if (q.in[5]) face(SideTag<5>());
+    if (q.in[1]) face(SideTag<1>());
+}
+
+// ---- mass balance and pressure rows (k_mass_rows) ----
+__global__ void __launch_bounds__(256) k_box_mass_rows(BoxG g, const int *row_ptr, MassArgs a)
+{
+    BoxCell q;
+    if (!box_cell(g, q)) return;
+    const int c = q.c;
+    double mf[6], v[6];
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+        mf[s] = a.mflux[q.f[s]];
+        v[s] = q.in[s] ? a.ff0[q.f[s]] : 0.0;   // -ApV
+    }
+    double S = 0.0, AV = 0.0;
+    // boundary faces in ascending id: FRONT, BACK, LEFT, RIGHT, DOWN, UP
+#pragma unroll
+    for (int s = 0; s < 6; s++)
+        if (!q.in[s] && g.btype[s] == INLET) S = S - mf[s];
+#pragma unroll
+    for (int s = 0; s < 6; s++)
+        if (!q.in[s] && g.btype[s] == OUTLET) S -= mf[s];
+    if (!a.assemble) { a.SU[c] = S; return; }
+    constexpr int order[6] = {0, 4, 2, 1, 3, 5};
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        const int s = order[k];
+        if (!q.in[s]) continue;
+        if (s & 1) S -= mf[s]; else S += mf[s];
+        AV -= v[s];
+    }
+    a.SU[c] = S;
+    a.AV[c] = AV;
+    if (!a.into_pressure) return;
+    a.Pb[c] = S;
+    {   // CSR: ascending columns -z -y -x main +x +y +z
+        int p = row_ptr[c];
+        if (q.in[0]) a.PAvals[p++] = v[0];
+        if (q.in[4]) a.PAvals[p++] = v[4];
+        if (q.in[2]) a.PAvals[p++] = v[2];
+        a.PAvals[p++] = AV;
+        if (q.in[3]) a.PAvals[p++] = v[3];
+        if (q.in[5]) a.PAvals[p++] = v[5];
+        if (q.in[1]) a.PAvals[p++] = v[1];
+    }
+    if (!a.pdia) return;
+    // the AMG fine level's copies, as k_level_dia writes them
+    const size_t n = (size_t)g.N;
+    constexpr int slot[6] = {0, 6, 2, 4, 1, 5};   // diagonal of each side's neighbour
+    a.pdia[(size_t)(3 - a.pskip) * n + c] = AV;
+    a.pdia32[3 * n + c] = (float)AV;
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+        if (!q.in[s]) continue;
+        a.pdia32[(size_t)slot[s] * n + c] = (float)v[s];
+        if (slot[s] >= a.pskip) a.pdia[(size_t)(slot[s] - a.pskip) * n + c] = v[s];
+    }
+    const double di = (AV != 0.0) ? 1.0 / AV : 0.0;
+    a.pdinv[c] = di;
+    a.pdinv32[c] = (float)di;
+    if (a.phoff) {
+        a.pdiag32[c] = (float)AV;
+#pragma unroll
+        for (int s = 0; s < 6; s++)
+            if (q.in[s]) a.phoff[(size_t)(slot[s] < 3 ? slot[s] : slot[s] - 1) * n + c] = (_Float16)(v[s] / AV);
+    }
+}
+
+// ---- flux and cell corrections (k_flux_correct, k_cell_correct) ----
+__global__ void __launch_bounds__(256) k_box_flux_correct(BoxG g, const double *PP, const double *gPPx,
+                                                          const double *gPPy, const double *gPPz, const double *ff0,
+                                                          double *mflux, double *fcorr)
+{
+    BoxCell q;
+    if (!box_cell(g, q)) return;
+    const int c = q.c;
+    const double P0 = PP[c];
+    const dv3 cc0 = v3(g.cc[0][q.x[0]], g.cc[1][q.x[1]], g.cc[2][q.x[2]]);
+    double area[3], vol;
+    box_areas(g, q, area, vol);
+    auto flush = [](double v) { return fabs(v) < 0.0000000000000003 ? 0.0 : v; };
+    auto face = [&](auto tag) {
+        using TAG = decltype(tag);
+        constexpr int ax = TAG::axis, s = TAG::side;
+        const int t = q.x[ax], c1 = q.nb[s], f = q.f[s];
+        const double fact = ff0[f];
+        double m = mflux[f];
+        m += (fact * (PP[c1] - P0));
+        dv3 cc1 = cc0;
+        const double cn = g.cc[ax][t + 1];
+        if (ax == 0) cc1.x = cn; else if (ax == 1) cc1.y = cn; else cc1.z = cn;
+        const dv3 fc = v3(ax == 0 ? g.fc[0][t] : g.ft[ax][0][q.x[0]], ax == 1 ? g.fc[1][t] : g.ft[ax][1][q.x[1]],
+                          ax == 2 ? g.fc[2][t] : g.ft[ax][2][q.x[2]]);
+        const dv3 n = v3(ax == 0 ? area[0] : g.zero[ax][0], ax == 1 ? area[1] : g.zero[ax][1],
+                         ax == 2 ? area[2] : g.zero[ax][2]);
+        const dv3 nh = n / mag(n);
+        const dv3 Xpac = fc - nh * dot(fc - cc0, nh);
+        const dv3 Xnac = fc - nh * dot(fc - cc1, nh);
+        const dv3 Xn = v3(flush(Xnac.x - cc1.x), flush(Xnac.y - cc1.y), flush(Xnac.z - cc1.z));
+        const dv3 Xp = v3(flush(Xpac.x - cc0.x), flush(Xpac.y - cc0.y), flush(Xpac.z - cc0.z));
+        // offsets of a rounding at most; where all six are flushed the
+        // correction is a signed zero and no gradient is read
+        double fcv = 0.0;
+        if (Xn.x != 0.0 || Xn.y != 0.0 || Xn.z != 0.0 || Xp.x != 0.0 || Xp.y != 0.0 || Xp.z != 0.0) {
+            const dv3 gP0 = ld3(gPPx, gPPy, gPPz, c), gP1 = ld3(gPPx, gPPy, gPPz, c1);
+            const double dpx = gP1.x * Xn.x - gP0.x * Xp.x;
+            const double dpy = gP1.y * Xn.y - gP0.y * Xp.y;
+            const double dpz = gP1.z * Xn.z - gP0.z * Xp.z;
+            fcv = fact * (dpx + dpy + dpz) * 0.8;
+            m += fcv;
+        }
+        st_out(&mflux[f], m);
+        st_out(&fcorr[f], fcv);
+    };
+    if (q.in[3]) face(SideTag<3>());
+    if (q.in[5]) face(SideTag<5>());
+    if (q.in[1]) face(SideTag<1>());
+}
+
+__global__ void __launch_bounds__(256) k_box_cell_correct(BoxG g, const double *fcorr, double *SU, double *P, double *PP,
+                                                          double *Uf, double *Vf, double *Wf, const double *gPPx,
+                                                          const double *gPPy, const double *gPPz, const double *AU,
+                                                          int which)
+{
+    BoxCell q;
+    if (!box_cell(g, q)) return;
+    const int c = q.c;
+    if (c < 6) PP[g.N + c] = 0.0;
+    double fc[6];
+#pragma unroll
+    for (int s = 0; s < 6; s++) fc[s] = q.in[s] ? fcorr[q.f[s]] : 0.0;
+    double S = 0.0;
+    constexpr int order[6] = {0, 4, 2, 1, 3, 5};
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        const int s = order[k];
+        if (!q.in[s]) continue;
+        if (s & 1) S -= fc[s]; else S += fc[s];
+    }
+    SU[c] = S;
+    if (which == 2 || (which == 1 && c == 0)) {
+        double area[3], vol;
+        box_areas(g, q, area, vol);
+        const double Ar = (AU[c] != 0.0) ? 1.0 / AU[c] : 0.0;
+        const double fact = vol * Ar;
+        P[c] += 0.2 * PP[c];
+        Uf[c] -= gPPx[c] * fact;
+        Vf[c] -= gPPy[c] * fact;
+        Wf[c] -= gPPz[c] * fact;
+    }
+    PP[c] = 0.0;
+}
+
 static void launch_mass(Ctx *c, const MassArgs &a)
 {
     const dim3 grid(walk_blocks(cell_walk(c)));
+    if (box_on(c)) {
+        hipLaunchKernelGGL(k_box_mass_faces, grid, dim3(256), 0, c->stream, box_geo(c), a);
+        hipLaunchKernelGGL(k_box_mass_rows, grid, dim3(256), 0, c->stream, box_geo(c), c->row_ptr, a);
+        return;
+    }
     hipLaunchKernelGGL(k_mass_faces, grid, dim3(256), 0, c->stream, geo(c), a);
     hipLaunchKernelGGL(k_mass_rows, grid, dim3(256), 0, c->stream, geo(c), a);
 }
@@ -892,12 +1468,14 @@ int set_up_field(Ctx *c)
 // ff0 (8) read; the CSR values (8 nnz) written; with the AMG fine level's
 // copies also the symmetric FP64 diagonals (8 (N + F_i)), the FP32 ones
 // (4 nnz), both inverse diagonals (12 N), and with the FP16 smoothing copy
-// the FP32 diagonal (4 N) and the FP16 off-diagonals (2 * 2 F_i).
+// the FP32 diagonal (4 N) and the FP16 off-diagonals (2 * 2 F_i).  The box
+// kernels: the same without geometry, forder and fother, with row_ptr (4).
 static double mass_bytes(Ctx *c, const MassArgs &a)
 {
     const Sizes z = sizes_of(c);
-    double b = 224.0 * z.N + 88.0 * z.Fi;                  // k_mass_faces
-    b += 72.0 * z.N + 8.0 * z.F + 8.0 * z.Fi + 8.0 * z.nnz;  // k_mass_rows
+    const bool box = box_on(c);
+    double b = box ? 136.0 * z.N + 24.0 * z.Fi : 224.0 * z.N + 88.0 * z.Fi;          // faces
+    b += (box ? 28.0 : 72.0) * z.N + 8.0 * z.F + 8.0 * z.Fi + 8.0 * z.nnz;           // rows
     if (a.pdia) b += 8.0 * (z.N + z.Fi) + 4.0 * z.nnz + 12.0 * z.N;
     if (a.phoff) b += 4.0 * z.N + 4.0 * z.Fi;
     return b;
@@ -1127,11 +1705,22 @@ int calculate_pressure(Ctx *c)
                 // read; per interior face ff0, mass flux, centre, normal (64)
                 // read and mass flux, correction (16) written
                 KTimer kt(c, MC_KC_CORRECT, 104.0 * c->N + 80.0 * (double)(c->F - c->Fb));
-                hipLaunchKernelGGL(k_flux_correct, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, geo(c),
-                                   c->phi[PP], c->gx[PP], c->gy[PP], c->gz[PP], c->ff0, c->mflux, c->fcorr);
+                if (box_on(c))
+                    hipLaunchKernelGGL(k_box_flux_correct, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream,
+                                       box_geo(c), c->phi[PP], c->gx[PP], c->gy[PP], c->gz[PP], c->ff0, c->mflux,
+                                       c->fcorr);
+                else
+                    hipLaunchKernelGGL(k_flux_correct, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream,
+                                       geo(c), c->phi[PP], c->gx[PP], c->gy[PP], c->gz[PP], c->ff0, c->mflux,
+                                       c->fcorr);
             }
             const int which = simple ? 2 : (c->first_pressure ? 1 : 0);
-            hipLaunchKernelGGL(k_cell_correct, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, geo(c), c->fcorr, c->SU,
+            if (box_on(c))
+                hipLaunchKernelGGL(k_box_cell_correct, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream,
+                                   box_geo(c), c->fcorr, c->SU, c->phi[P], c->phi[PP], c->phi[U], c->phi[V], c->phi[W],
+                                   c->gx[PP], c->gy[PP], c->gz[PP], c->AU, which);
+            else
+                hipLaunchKernelGGL(k_cell_correct, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, geo(c), c->fcorr, c->SU,
                                c->phi[P], c->phi[PP], c->phi[U], c->phi[V], c->phi[W], c->gx[PP], c->gy[PP],
                                c->gz[PP], c->AU, which);
             MC_LAUNCH_CHECK(c);
@@ -1540,6 +2129,324 @@ __global__ void __launch_bounds__(256, 3) k_scalar_batch(Geo g, ScalBatchArgs a)
     if constexpr (TEM) store_row(g, c, nint, own_nb, own_fft, At, a.tvals, a.tdia);
 }
 
+// ------------------------------------- generated-box scalar kernels --
+// a cell with a face on a wall side
+__device__ __forceinline__ bool box_wall(const BoxG &g, int x, int y, int z)
+{
+    return (z == 0 && g.btype[0] == WALL) || (z == g.nz - 1 && g.btype[1] == WALL) || (x == 0 && g.btype[2] == WALL) ||
+           (x == g.nx - 1 && g.btype[3] == WALL) || (y == 0 && g.btype[4] == WALL) ||
+           (y == g.ny - 1 && g.btype[5] == WALL);
+}
+
+// k_scalar for one equation: TYPE = TERBTE, TERBED, or TEMP for the five
+// others (they differ in the face viscosity table only).
+template <int TYPE>
+__global__ void __launch_bounds__(256) k_box_scalar(BoxG g, ScalArgs a)
+{
+    BoxCell q;
+    if (!box_cell(g, q)) return;
+    constexpr bool ed = TYPE == TERBED, te = TYPE == TERBTE;
+    const int c = q.c, N = g.N;
+    const double ev = a.ev;
+    const double pc = a.phi[c];
+    const dv3 gc = ld3(a.gx, a.gy, a.gz, c);
+    double mf[6], pn[6], gn[6];
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+        const double *gr = s < 2 ? a.gz : s < 4 ? a.gx : a.gy;
+        mf[s] = a.mflux[q.f[s]];
+        pn[s] = a.phi[q.nb[s]];
+        gn[s] = gr[q.nb[s]];
+    }
+    double area[3], vol;
+    box_areas(g, q, area, vol);
+    const bool wallcell = (te || ed) && box_wall(g, q.x[0], q.x[1], q.x[2]);
+    double S = 0.0, A = 0.0, ff[6], xo = 0.0;
+    auto fi = [&](auto tag) {
+        using TAG = decltype(tag);
+        constexpr int s = TAG::side, ax = TAG::axis;
+        const BoxFace f = box_face(g, q, area, tag);
+        const double own = ax == 0 ? gc.x : ax == 1 ? gc.y : gc.z;
+        const double d = TAG::high ? own * f.l0 + gn[s] * f.l1 : gn[s] * f.l0 + own * f.l1;
+        const double VisFace = f.vis * (f.area / f.dist);
+        const double fde1 = f.vis * (d * f.area);
+        const double fdi = VisFace * (d * f.dist);
+        double ff0 = -VisFace - dmax(mf[s], 0.0);
+        double ff1 = -VisFace + dmin(mf[s], 0.0);
+        if constexpr (ed) {   // rows of wall cells lose their off-diagonals
+            const bool wn = box_wall(g, q.x[0] + (ax == 0 ? (TAG::high ? 1 : -1) : 0),
+                                     q.x[1] + (ax == 1 ? (TAG::high ? 1 : -1) : 0),
+                                     q.x[2] + (ax == 2 ? (TAG::high ? 1 : -1) : 0));
+            if (TAG::high ? wallcell : wn) ff1 = 0.0;
+            if (TAG::high ? wn : wallcell) ff0 = 0.0;
+        }
+        if constexpr (TAG::high) {
+            S = S + fde1 - fdi;
+            ff[s] = ff1;
+            st_out(&a.ff0[q.f[s]], ff0); st_out(&a.ff1[q.f[s]], ff1);
+        } else {
+            S = S - fde1 + fdi;
+            ff[s] = ff0;
+        }
+        xo += ff[s] * pn[s];
+    };
+    auto fb = [&](int side) {
+        const int f = side == 0 ? q.f[0] : side == 1 ? q.f[1] : side == 2 ? q.f[2] : side == 3 ? q.f[3] : side == 4 ? q.f[4] : q.f[5];
+        const int bt = g.btype[side];
+        const bool last = (f == g.last_face[side]);
+        const dv3 cc = v3(g.cc[0][q.x[0]], g.cc[1][q.x[1]], g.cc[2][q.x[2]]);
+        const dv3 Xpn = ld3(g.fcx, g.fcy, g.fcz, f) - cc;
+        if (bt == INLET) {
+            double Visac = a.inlet_ev;
+            Visac -= ev;
+            Visac = scalar_visac(a.type, ev, Visac);
+            const double VisFace = Visac * g.frlc[f];
+            const double fde = Visac * dot(gc, ld3(g.fnx, g.fny, g.fnz, f));
+            const double fdi = VisFace * dot(gc, Xpn);
+            const double fbc = -VisFace + dmin(a.mflux[f], 0.0);
+            A = A - fbc;
+            S = S - fbc * a.inlet_phi + fde - fdi;
+            if (last) a.phi[N + side] = a.inlet_phi;
+        } else if (bt == OUTLET) {
+            double Visac = ev;
+            Visac -= ev;
+            Visac = scalar_visac(a.type, ev, Visac);
+            const double PhiFace = pc + dot(gc, Xpn);
+            const double VisFace = Visac * g.frlc[f];
+            const double fde = Visac * dot(gc, ld3(g.fnx, g.fny, g.fnz, f));
+            const double fdi = VisFace * dot(gc, Xpn);
+            S = S + fde - fdi;
+            if (last) a.phi[N + side] = PhiFace;
+        } else if (bt == WALL) {
+            if (last && !ed) a.phi[N + side] = pc;
+        }
+    };
+    box_faces(q, fi, fb);
+    const double rho = g.rho;
+    double phic = pc;
+    const double fv = rho * vol * a.rdelta;
+    S += fv * phic;
+    A += fv;
+    if constexpr (te) {
+        const dv3 dUdXp = ld3(a.gUx, a.gUy, a.gUz, c), dVdXp = ld3(a.gVx, a.gVy, a.gVz, c), dWdXp = ld3(a.gWx, a.gWy, a.gWz, c);
+        const double s1 = (dUdXp.x + dUdXp.x) * dUdXp.x + (dUdXp.y + dVdXp.x) * dUdXp.y + (dUdXp.z + dWdXp.x) * dUdXp.z;
+        const double s2 = (dVdXp.x + dUdXp.y) * dVdXp.x + (dVdXp.y + dVdXp.y) * dVdXp.y + (dVdXp.z + dWdXp.y) * dVdXp.z;
+        const double s3 = (dWdXp.x + dUdXp.z) * dWdXp.x + (dWdXp.y + dVdXp.z) * dWdXp.y + (dWdXp.z + dWdXp.z) * dWdXp.z;
+        const double VisT = ev - ev;
+        double TP = VisT * (s1 + s2 + s3);
+        const double Dis = rho * a.ED[c];
+        const double TEc = a.TE[c];
+        S = S + TP * vol;
+        A = A + Dis / (TEc + 0.000000000000000001) * vol;
+        if (wallcell) {
+            // wall faces in ascending id: FRONT, BACK, LEFT, RIGHT, DOWN, UP
+            for (int s = 0; s < 6; s++) {
+                const bool in = s == 0 ? q.in[0] : s == 1 ? q.in[1] : s == 2 ? q.in[2] : s == 3 ? q.in[3] : s == 4 ? q.in[4] : q.in[5];
+                if (in || g.btype[s] != WALL) continue;
+                const int f = s == 0 ? q.f[0] : s == 1 ? q.f[1] : s == 2 ? q.f[2] : s == 3 ? q.f[3] : s == 4 ? q.f[4] : q.f[5];
+                S = S - TP * vol;
+                const dv3 cc = v3(g.cc[0][q.x[0]], g.cc[1][q.x[1]], g.cc[2][q.x[2]]);
+                const dv3 Xpn = ld3(g.fcx, g.fcy, g.fcz, f) - cc;
+                const dv3 Up = v3(a.U[c] - 0., a.V[c] - 0., a.W[c] - 0.);
+                const dv3 n = ld3(g.fnx, g.fny, g.fnz, f);
+                const dv3 nh = n / mag(n);
+                const double dp = dot(Up, nh);
+                const dv3 Ut = Up - nh * dp;
+                const double Uvel = sqrt(dot(Ut, Ut));
+                const double distance_to_face = mag(Xpn);
+                const double rkapdn = 1.0 / (0.419 * distance_to_face);
+                const double Tau_w = ev * Uvel / distance_to_face;
+                const double Utau = sqrt(Tau_w / rho);
+                TP = Tau_w * Utau * rkapdn;
+                if (f == g.last_face[s]) a.TE[N + s] = TEc;
+                S = S + TP * vol;
+                const double DisP = a.cmu75 * sqrt(TEc) * rkapdn;
+                A = A + rho * DisP * vol;
+            }
+        }
+        st_out(&a.TP[c], TP);
+    } else if constexpr (ed) {
+        const double TEc = a.TE[c];
+        const double fact = a.ED[c] / (TEc + 0.000000000000000001) * vol;
+        S = S + 1.44 * fact * a.TP[c];
+        A = A + 1.92 * fact * rho;
+        if (wallcell) {
+            for (int s = 0; s < 6; s++) {
+                const bool in = s == 0 ? q.in[0] : s == 1 ? q.in[1] : s == 2 ? q.in[2] : s == 3 ? q.in[3] : s == 4 ? q.in[4] : q.in[5];
+                if (in || g.btype[s] != WALL) continue;
+                const int f = s == 0 ? q.f[0] : s == 1 ? q.f[1] : s == 2 ? q.f[2] : s == 3 ? q.f[3] : s == 4 ? q.f[4] : q.f[5];
+                const dv3 cc = v3(g.cc[0][q.x[0]], g.cc[1][q.x[1]], g.cc[2][q.x[2]]);
+                const double distance = mag(ld3(g.fcx, g.fcy, g.fcz, f) - cc);
+                const double Dis = a.cmu75 * pow(TEc, 1.5) / (distance * 0.419);
+                phic = Dis;
+                S = Dis;
+                A = 1;
+                if (f == g.last_face[s]) a.ED[N + s] = Dis;
+            }
+        }
+    }
+    A = box_minus_off(q, ff, A);
+    A *= (1. / a.urf);
+    S = S + (1.0 - a.urf) * A * phic;
+    st_out(&a.AV[c], A);
+    st_out(&a.SU[c], S);
+    if (a.r0) st_out(&a.r0[c], S - (A * pc + xo));
+    box_store_row(g, q, ff, A, a.dia);
+}
+
+// k_scalar_batch; tv: the face viscosities of the temperature (g.vis: the
+// passive scalars')
+struct BoxVis { const double *v[3]; };
+template <bool TEM>
+__global__ void __launch_bounds__(256) k_box_scalar_batch(BoxG g, BoxVis tv, ScalBatchArgs a)
+{
+    BoxCell q;
+    if (!box_cell(g, q)) return;
+    const int c = q.c, N = g.N;
+    const double ev = a.ev;
+    double S[SB], A = 0.0, ff[6];
+    double St = 0.0, At = 0.0, fft[6];
+#pragma unroll
+    for (int s = 0; s < SB; s++) S[s] = 0.0;
+    double mf[6];
+#pragma unroll
+    for (int s = 0; s < 6; s++) mf[s] = a.mflux[q.f[s]];
+    double area[3], vol;
+    box_areas(g, q, area, vol);
+    dv3 gs[SB], gt = v3(0.0, 0.0, 0.0);
+    double ps[SB], pt = 0.0;
+#pragma unroll
+    for (int s = 0; s < SB; s++) { gs[s] = ld3(a.gx[s], a.gy[s], a.gz[s], c); ps[s] = a.phi[s][c]; }
+    if constexpr (TEM) { gt = ld3(a.tgx, a.tgy, a.tgz, c); pt = a.tphi[c]; }
+    auto fi = [&](auto tag) {
+        using TAG = decltype(tag);
+        constexpr int s = TAG::side, ax = TAG::axis;
+        const int nb = q.nb[s];
+        const BoxFace f = box_face(g, q, area, tag);
+        const double rl = f.area / f.dist;
+        const double VisFace = f.vis * rl;
+        const double ff0 = -VisFace - dmax(mf[s], 0.0);
+        const double ff1 = -VisFace + dmin(mf[s], 0.0);
+        auto mix = [&](double own, double oth) {
+            return TAG::high ? own * f.l0 + oth * f.l1 : oth * f.l0 + own * f.l1;
+        };
+        if constexpr (TEM) {
+            const double *gr = ax == 0 ? a.tgx : ax == 1 ? a.tgy : a.tgz;
+            const double Vt = tv.v[ax][TAG::high ? q.x[ax] : q.x[ax] - 1];
+            const double d = mix(ax == 0 ? gt.x : ax == 1 ? gt.y : gt.z, gr[nb]);
+            const double VisFaceT = Vt * rl;
+            const double fde1 = Vt * (d * f.area);
+            const double fdi = VisFaceT * (d * f.dist);
+            if constexpr (TAG::high) { St = St + fde1 - fdi; fft[s] = -VisFaceT + dmin(mf[s], 0.0); }
+            else { St = St - fde1 + fdi; fft[s] = -VisFaceT - dmax(mf[s], 0.0); }
+        }
+#pragma unroll
+        for (int k = 0; k < SB; k++) {
+            const double *gr = ax == 0 ? a.gx[k] : ax == 1 ? a.gy[k] : a.gz[k];
+            const double d = mix(ax == 0 ? gs[k].x : ax == 1 ? gs[k].y : gs[k].z, gr[nb]);
+            const double fde1 = f.vis * (d * f.area);
+            const double fdi = VisFace * (d * f.dist);
+            if constexpr (TAG::high) S[k] = S[k] + fde1 - fdi;
+            else S[k] = S[k] - fde1 + fdi;
+        }
+        if constexpr (TAG::high) {
+            ff[s] = ff1;
+            st_out(&a.ff0[q.f[s]], ff0); st_out(&a.ff1[q.f[s]], ff1);
+        } else {
+            ff[s] = ff0;
+        }
+    };
+    auto fb = [&](int side) {
+        const int f = side == 0 ? q.f[0] : side == 1 ? q.f[1] : side == 2 ? q.f[2] : side == 3 ? q.f[3] : side == 4 ? q.f[4] : q.f[5];
+        const int bt = g.btype[side];
+        const bool last = (f == g.last_face[side]);
+        const dv3 cc = v3(g.cc[0][q.x[0]], g.cc[1][q.x[1]], g.cc[2][q.x[2]]);
+        const dv3 Xpn = ld3(g.fcx, g.fcy, g.fcz, f) - cc;
+        const dv3 nrm = ld3(g.fnx, g.fny, g.fnz, f);
+        if (bt == INLET) {
+            const double mfb = a.mflux[f];
+            if constexpr (TEM) {
+                double Vt = a.inlet_ev;
+                Vt -= ev;
+                Vt = scalar_visac(TEMP, ev, Vt);
+                const double VisFaceT = Vt * g.frlc[f];
+                const double fde = Vt * dot(gt, nrm);
+                const double fdi = VisFaceT * dot(gt, Xpn);
+                const double fbc = -VisFaceT + dmin(mfb, 0.0);
+                At = At - fbc;
+                St = St - fbc * a.tinlet + fde - fdi;
+                if (last) a.tphi[N + side] = a.tinlet;
+            }
+            double Visac = a.inlet_ev;
+            Visac -= ev;
+            Visac = scalar_visac(a.type, ev, Visac);
+            const double VisFace = Visac * g.frlc[f];
+            const double fbc = -VisFace + dmin(mfb, 0.0);
+            A = A - fbc;
+#pragma unroll
+            for (int k = 0; k < SB; k++) {
+                const double fde = Visac * dot(gs[k], nrm);
+                const double fdi = VisFace * dot(gs[k], Xpn);
+                S[k] = S[k] - fbc * a.inlet_phi[k] + fde - fdi;
+                if (last) a.phi[k][N + side] = a.inlet_phi[k];
+            }
+        } else if (bt == OUTLET) {
+            if constexpr (TEM) {
+                double Vt = ev;
+                Vt -= ev;
+                Vt = scalar_visac(TEMP, ev, Vt);
+                const double PhiFace = pt + dot(gt, Xpn);
+                const double VisFaceT = Vt * g.frlc[f];
+                const double fde = Vt * dot(gt, nrm);
+                const double fdi = VisFaceT * dot(gt, Xpn);
+                St = St + fde - fdi;
+                if (last) a.tphi[N + side] = PhiFace;
+            }
+            double Visac = ev;
+            Visac -= ev;
+            Visac = scalar_visac(a.type, ev, Visac);
+            const double VisFace = Visac * g.frlc[f];
+#pragma unroll
+            for (int k = 0; k < SB; k++) {
+                const double PhiFace = ps[k] + dot(gs[k], Xpn);
+                const double fde = Visac * dot(gs[k], nrm);
+                const double fdi = VisFace * dot(gs[k], Xpn);
+                S[k] = S[k] + fde - fdi;
+                if (last) a.phi[k][N + side] = PhiFace;
+            }
+        } else if (bt == WALL) {
+            if (last) {
+                if constexpr (TEM) a.tphi[N + side] = pt;
+#pragma unroll
+                for (int k = 0; k < SB; k++) a.phi[k][N + side] = ps[k];
+            }
+        }
+    };
+    box_faces(q, fi, fb);
+    const double fv = g.rho * vol * a.rdelta;
+    if constexpr (TEM) {
+        St += fv * pt;
+        At += fv;
+        At = box_minus_off(q, fft, At);
+        At *= (1. / a.urf);
+        St = St + (1.0 - a.urf) * At * pt;
+        st_out(&a.tS[c], St);
+    }
+#pragma unroll
+    for (int s = 0; s < SB; s++) S[s] += fv * ps[s];
+    A += fv;
+    A = box_minus_off(q, ff, A);
+    A *= (1. / a.urf);
+#pragma unroll
+    for (int s = 0; s < SB; s++) {
+        S[s] = S[s] + (1.0 - a.urf) * A * ps[s];
+        st_out(&a.S[s][c], S[s]);
+    }
+    st_out(&a.AV[c], A);
+    box_store_row(g, q, ff, A, a.dia);
+    if constexpr (TEM) box_store_row(g, q, fft, At, a.tdia);
+}
+
 // FUL, PRO, VARF, VARP (FlowSolver.inl:3243-3260) as one 4-RHS solve; with
 // tem, the temperature equation (:3237-3242) is assembled in the same pass
 // into its own matrix and solved first, as the reference orders them (none of
@@ -1577,13 +2484,21 @@ static void batch_launch(Ctx *c, const ScalBatchArgs &a, bool tem, hipStream_t s
     // (48) read, A (8) written; per face mass flux, lambda, rlencos,
     // normal (48) read; per interior face ff0, ff1 (16) written; per
     // boundary face centre (24) read; one matrix per equation system
-    // (8 nnz each) written
+    // (8 nnz each) written; the box kernel: no cell or interior face geometry,
+    // forder or fother
     const int nsc = SB + (tem ? 1 : 0);
     const Sizes z = sizes_of(c);
-    const double bytes = (40.0 * nsc + 96.0) * z.N + 48.0 * z.F + 16.0 * z.Fi + 24.0 * z.Fb +
-                         8.0 * z.nnz * (tem ? 2 : 1);
+    const bool box = box_on(c) && a.dia && (!tem || a.tdia);
+    const double bytes = (40.0 * nsc + (box ? 8.0 : 96.0)) * z.N + (box ? 8.0 : 48.0) * z.F + 16.0 * z.Fi +
+                         (box ? 56.0 : 24.0) * z.Fb + 8.0 * z.nnz * (tem ? 2 : 1);
     KTimer kt(c, s == c->stream ? MC_KC_SCALAR_BATCH : -1, bytes);
-    if (tem)
+    if (box) {
+        const dim3 gr(walk_blocks(cell_walk(c)));
+        BoxVis tv;
+        for (int k = 0; k < 3; k++) tv.v[k] = c->box.vis[3][k];
+        if (tem) hipLaunchKernelGGL(k_box_scalar_batch<true>, gr, dim3(256), 0, s, box_geo(c, 4), tv, a);
+        else hipLaunchKernelGGL(k_box_scalar_batch<false>, gr, dim3(256), 0, s, box_geo(c, 4), tv, a);
+    } else if (tem)
         hipLaunchKernelGGL(k_scalar_batch<true>, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, s, geo(c), a);
     else
         hipLaunchKernelGGL(k_scalar_batch<false>, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, s, geo(c), a);
@@ -1727,13 +2642,24 @@ int scalar_assemble(Ctx *c, int type, double *r0)
     // reads ED (8) and the velocity gradients (72) and writes TP (8); ED also
     // reads TE, TP (16) and the wall flags (1); per face mass flux, lambda,
     // rlencos, normal (48) read; per interior face ff0, ff1 (16) written; per
-    // boundary face centre (24) read; the matrix entries (8 nnz) written
+    // boundary face centre (24) read; the matrix entries (8 nnz) written.  The
+    // box kernel: no cell or interior face geometry, forder, fother or flags
     const Sizes z = sizes_of(c);
-    double cell = 136.0 + (r0 ? 8.0 : 0.0);
+    const bool box = box_on(c) && a.dia;
+    double cell = (box ? 48.0 : 136.0) + (r0 ? 8.0 : 0.0);
     if (type == TERBTE) cell += 88.0;
-    if (type == TERBED) cell += 17.0;
-    KTimer kt(c, MC_KC_SCALAR_ASM, cell * z.N + 48.0 * z.F + 16.0 * z.Fi + 24.0 * z.Fb + 8.0 * z.nnz);
-    hipLaunchKernelGGL(k_scalar, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, geo(c), a);
+    if (type == TERBED) cell += box ? 16.0 : 17.0;
+    KTimer kt(c, MC_KC_SCALAR_ASM, cell * z.N + (box ? 8.0 : 48.0) * z.F + 16.0 * z.Fi + (box ? 56.0 : 24.0) * z.Fb +
+                                       8.0 * z.nnz);
+    const dim3 gr(walk_blocks(cell_walk(c)));
+    if (!box)
+        hipLaunchKernelGGL(k_scalar, gr, dim3(256), 0, c->stream, geo(c), a);
+    else if (type == TERBTE)
+        hipLaunchKernelGGL(k_box_scalar<TERBTE>, gr, dim3(256), 0, c->stream, box_geo(c, 1), a);
+    else if (type == TERBED)
+        hipLaunchKernelGGL(k_box_scalar<TERBED>, gr, dim3(256), 0, c->stream, box_geo(c, 2), a);
+    else
+        hipLaunchKernelGGL(k_box_scalar<TEMP>, gr, dim3(256), 0, c->stream, box_geo(c, type == TEMP ? 3 : 4), a);
     MC_LAUNCH_CHECK(c);
     return MC_OK;
 }

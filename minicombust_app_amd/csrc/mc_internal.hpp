@@ -143,6 +143,20 @@ struct Ctx {
     double *farea = nullptr, *flam = nullptr, *frlc = nullptr; // [F]
     double *vol = nullptr, *rho = nullptr;                     // [N]
 
+    // geometry of a generated box as per-axis tables (mc_mesh.hip box_tables)
+    struct BoxTables {
+        bool ok = false;             // every stored value is the tables' bit for bit
+        int n[3] = {0, 0, 0};        // cells per axis
+        // per axis: cell centre, cell width, and of the face towards the next
+        // cell its weight lambda, the distance of the two centres and the
+        // face centre's coordinate along the axis
+        double *cc[3] = {}, *w[3] = {}, *lam[3] = {}, *dist[3] = {}, *fc[3] = {};
+        double *ft[3][3] = {};       // [a][b]: coordinate along b of the centres of faces normal to a
+        double *vis[5][3] = {};      // face viscosity along each axis: momentum, TE, ED, TEM, other scalars
+        double zero[3][3] = {};      // [a][b]: the (signed) zero component b of the normals of faces normal to a
+        double rho = 0.0;
+    } box;
+
     // ---- fields ----
     double *phi[NFIELDS] = {};
     double **field_ptrs = nullptr;   // device table: phi, gx, gy, gz of every field
@@ -299,13 +313,9 @@ struct CellWalk {
     int yc = 1;                   // y rows per chunk of the block order
 };
 
-// Cell of thread t (0..255) of brick b in CellWalk order, or -1.
-__device__ __forceinline__ int walk_cell_at(const CellWalk &w, int b, int t)
+// Coordinates and cell of thread t (0..255) of brick b of a box walk, or -1.
+__device__ __forceinline__ int walk_xyz_at(const CellWalk &w, int b, int t, int &x, int &y, int &z)
 {
-    if (w.nx == 0) {
-        const int c = b * 256 + t;
-        return c < w.N ? c : -1;
-    }
     // blocks in chunks of yc consecutive y rows; within a chunk z-slab by
     // z-slab, each slab row by row, each row tile by tile: a cell's x, y and z
     // neighbours are visited a few blocks apart (L2-resident), except across a
@@ -313,12 +323,24 @@ __device__ __forceinline__ int walk_cell_at(const CellWalk &w, int b, int t)
     const int xt = b % w.ntx, r = b / w.ntx;
     const int per = w.yc * w.ntz;
     const int ch = r / per, q = r - ch * per;
-    const int zt = q / w.yc, y = ch * w.yc + (q - zt * w.yc);
+    const int zt = q / w.yc;
+    y = ch * w.yc + (q - zt * w.yc);
     if (y >= w.ny) return -1;
-    const int x = (xt << w.lgtx) + (t & ((1 << w.lgtx) - 1));
-    const int z = zt * (256 >> w.lgtx) + (t >> w.lgtx);
+    x = (xt << w.lgtx) + (t & ((1 << w.lgtx) - 1));
+    z = zt * (256 >> w.lgtx) + (t >> w.lgtx);
     if (x >= w.nx || z >= w.nz) return -1;
     return x + w.nx * (y + w.ny * z);
+}
+
+// Cell of thread t (0..255) of brick b in CellWalk order, or -1.
+__device__ __forceinline__ int walk_cell_at(const CellWalk &w, int b, int t)
+{
+    if (w.nx == 0) {
+        const int c = b * 256 + t;
+        return c < w.N ? c : -1;
+    }
+    int x, y, z;
+    return walk_xyz_at(w, b, t, x, y, z);
 }
 
 __device__ __forceinline__ int walk_cell(const CellWalk &w)
@@ -643,6 +665,7 @@ int noalloc_scratch_init(Ctx *c);   // mc_couple.hip
 int mesh_box_generate(Ctx *c, int64_t m);
 int mesh_from_host(Ctx *c, const mc_mesh_desc *d);
 int mesh_finish(Ctx *c);
+int box_tables(Ctx *c);     // Ctx::box, on a generated box
 int init_fields(Ctx *c);   // constructor fields and boundary slots   // geometry, init, CSR pattern, face orders
 
 // stages (mc_flow.hip)

@@ -570,4 +570,137 @@ int mesh_finish(Ctx *c)
     return MC_OK;
 }
 
+// ------------------------------------------------------- box tables --
+// On a generated box every geometric quantity is a function of one coordinate
+// (centres, weights, distances) or a product of such (areas, volumes), with
+// the same bits wherever that coordinate is the same: per-axis tables of a few
+// hundred values, resident in L1, replace 14 arrays of the cells' and faces'
+// size in the assembly kernels.  The tables are read off one row of cells per
+// axis and then compared with every stored value, bit for bit; a single
+// difference leaves the arrays in use.
+struct TabArgs {
+    int n[3];
+    double *cc[3], *w[3], *lam[3], *dist[3], *fc[3], *ft[3][3], *vis[5][3];
+    const double *C[3], *FC[3], *FN[3], *farea, *flam, *frlc, *vol, *rho;
+    double zero[3][3], rho0;
+    double ev;
+};
+
+// storage position of the face between cell c and the next along axis a
+__device__ __forceinline__ int64_t tab_face(const TabArgs &t, int a, int64_t c)
+{
+    const int64_t N = (int64_t)t.n[0] * t.n[1] * t.n[2];
+    return a == 0 ? c : a == 1 ? N + c : 2 * N + c;
+}
+
+// diffusion coefficients of the scalar equations at a face of weight l0
+// (FlowSolver.inl:2545-2560 with the constant effective viscosity)
+__device__ __forceinline__ double tab_visac(int kind, double ev, double l0)
+{
+    double v = ev * l0 + ev * (1.0 - l0);
+    if (kind == 0) return v;
+    v -= ev;
+    if (kind == 1) return ev + v;
+    if (kind == 2) return ev + v / 1.219;
+    if (kind == 3) return (ev + v / 0.9) / 0.6905;
+    return (ev + v / 0.9) / 0.9;
+}
+
+__global__ void k_tab_fill(TabArgs t, const uint64_t *cells, const double *px, const double *py, const double *pz)
+{
+    const int a = blockIdx.y, i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= t.n[a]) return;
+    const int64_t st[3] = {1, t.n[0], (int64_t)t.n[0] * t.n[1]};
+    const int64_t c = i * st[a];
+    t.cc[a][i] = t.C[a][c];
+    const int corner[3] = {1, 2, 4};
+    dv3 e = v3(px[cells[8 * c + corner[a]]], py[cells[8 * c + corner[a]]], pz[cells[8 * c + corner[a]]]) -
+            v3(px[cells[8 * c]], py[cells[8 * c]], pz[cells[8 * c]]);
+    t.w[a][i] = mag(e);
+    const bool face = i + 1 < t.n[a];
+    const int64_t f = tab_face(t, a, c);
+    t.lam[a][i] = face ? t.flam[f] : 1.0;
+    t.dist[a][i] = face ? t.C[a][c + st[a]] - t.C[a][c] : 0.0;
+    t.fc[a][i] = face ? t.FC[a][f] : 0.0;
+    for (int k = 0; k < 5; k++) t.vis[k][a][i] = face ? tab_visac(k, t.ev, t.flam[f]) : 0.0;
+    // faces normal to b at cell (.., i along a, ..), tangential coordinate a
+    for (int b = 0; b < 3; b++)
+        if (b != a) t.ft[b][a][i] = t.FC[a][tab_face(t, b, c)];
+}
+
+__device__ __forceinline__ bool same(double x, double y) { return __double_as_longlong(x) == __double_as_longlong(y); }
+
+__global__ void k_tab_check(TabArgs t, int *bad)
+{
+    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t N = (int64_t)t.n[0] * t.n[1] * t.n[2];
+    if (c >= N) return;
+    const int x[3] = {(int)(c % t.n[0]), (int)((c / t.n[0]) % t.n[1]), (int)(c / ((int64_t)t.n[0] * t.n[1]))};
+    const double W[3] = {t.w[0][x[0]], t.w[1][x[1]], t.w[2][x[2]]};
+    bool ok = same(t.vol[c], W[0] * W[1] * W[2]) && same(t.rho[c], t.rho0);
+    for (int a = 0; a < 3; a++) ok = ok && same(t.C[a][c], t.cc[a][x[a]]);
+    for (int a = 0; a < 3; a++) {
+        if (x[a] + 1 >= t.n[a]) continue;
+        const int64_t f = tab_face(t, a, c);
+        const double area = W[(a + 1) % 3] * W[(a + 2) % 3];
+        ok = ok && same(t.farea[f], area) && same(t.flam[f], t.lam[a][x[a]]) &&
+             same(t.frlc[f], area / t.dist[a][x[a]]);
+        for (int b = 0; b < 3; b++) {
+            ok = ok && same(t.FN[b][f], b == a ? area : t.zero[a][b]);
+            ok = ok && same(t.FC[b][f], b == a ? t.fc[a][x[a]] : t.ft[a][b][x[b]]);
+        }
+    }
+    if (!ok) *bad = 1;
+}
+
+int box_tables(Ctx *c)
+{
+    if (c->m <= 0 || c->m < 2) return MC_OK;   // two cells at least along every axis
+    MemScope ms(c, MC_MEM_MESH);
+    Ctx::BoxTables &b = c->box;
+    TabArgs t;
+    memset(&t, 0, sizeof(t));
+    b.n[0] = (int)(2 * c->m); b.n[1] = b.n[2] = (int)c->m;
+    const int most = b.n[0];
+    for (int a = 0; a < 3; a++) {
+        double **all[] = {&b.cc[a], &b.w[a], &b.lam[a], &b.dist[a], &b.fc[a], &b.ft[a][(a + 1) % 3],
+                          &b.ft[a][(a + 2) % 3], &b.vis[0][a], &b.vis[1][a], &b.vis[2][a], &b.vis[3][a], &b.vis[4][a]};
+        for (double **p : all) MC_TRY(dalloc(c, p, most));
+    }
+    const double *C[3] = {c->cx, c->cy, c->cz}, *FC[3] = {c->fcx, c->fcy, c->fcz}, *FN[3] = {c->fnx, c->fny, c->fnz};
+    const int64_t N = c->N;
+    for (int a = 0; a < 3; a++) {
+        t.n[a] = b.n[a];
+        t.cc[a] = b.cc[a]; t.w[a] = b.w[a]; t.lam[a] = b.lam[a]; t.dist[a] = b.dist[a]; t.fc[a] = b.fc[a];
+        t.C[a] = C[a]; t.FC[a] = FC[a]; t.FN[a] = FN[a];
+        for (int k = 0; k < 5; k++) t.vis[k][a] = b.vis[k][a];
+        for (int e = 0; e < 3; e++) {
+            t.ft[a][e] = b.ft[a][e];
+            MC_HIP(c, hipMemcpyAsync(&b.zero[a][e], FN[e] + a * N, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+        }
+    }
+    MC_HIP(c, hipMemcpyAsync(&b.rho, c->rho, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    MC_HIP(c, hipStreamSynchronize(c->stream));
+    for (int a = 0; a < 3; a++)
+        for (int e = 0; e < 3; e++) {
+            if (e == a) b.zero[a][e] = 0.0;
+            else if (b.zero[a][e] != 0.0) return MC_OK;
+            t.zero[a][e] = b.zero[a][e];
+        }
+    t.rho0 = b.rho;
+    t.farea = c->farea; t.flam = c->flam; t.frlc = c->frlc; t.vol = c->vol; t.rho = c->rho;
+    t.ev = c->k.ev;
+    int *bad = nullptr;
+    MC_TRY(dalloc(c, &bad, 1));
+    MC_HIP(c, hipMemsetAsync(bad, 0, sizeof(int), c->stream));
+    hipLaunchKernelGGL(k_tab_fill, dim3(div_up(most, 64), 3), dim3(64), 0, c->stream, t, c->cells, c->px, c->py, c->pz);
+    hipLaunchKernelGGL(k_tab_check, dim3(div_up(N, 256)), dim3(256), 0, c->stream, t, bad);
+    MC_LAUNCH_CHECK(c);
+    int h = 1;
+    MC_HIP(c, hipMemcpyAsync(&h, bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    MC_HIP(c, hipStreamSynchronize(c->stream));
+    b.ok = h == 0;
+    return MC_OK;
+}
+
 }  // namespace mc

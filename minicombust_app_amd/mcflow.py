@@ -35,10 +35,10 @@ KC_NAMES = ["grad11", "grad1", "mom_asm", "p_asm", "scalar_asm", "pcg_spmv64", "
             "flux_correct", "mpnn_fwd", "jac64", "jac32", "bicg_spmv", "scalar_batch", "ir_resid", "mpnn_bwd"]
 # kernel symbol (as a profiler lists it) of each single-kernel class (p_asm
 # times two kernels, mc::k_mass_faces then mc::k_mass_rows)
-KC_KERNELS = {"grad11": "mc::k_grad<11, false>", "grad1": "mc::k_grad<1, false>", "mom_asm": "mc::k_momentum",
-              "scalar_asm": "mc::k_scalar(", "pcg_spmv64": "mc::k_pcg_pq<-7, double>",
-              "pcg_spmv32": "mc::k_pcg_pq<7, float>", "flux_correct": "mc::k_flux_correct",
-              "scalar_batch": "mc::k_scalar_batch<true>", "ir_resid": "mc::k_ir_resid<-7>"}
+KC_KERNELS = {"grad11": "mc::k_box_grad<11>", "grad1": "mc::k_box_grad<1>", "mom_asm": "mc::k_box_momentum",
+              "scalar_asm": "mc::k_box_scalar<", "pcg_spmv64": "mc::k_pcg_pq<-7, double>",
+              "pcg_spmv32": "mc::k_pcg_pq<7, float>", "flux_correct": "mc::k_box_flux_correct",
+              "scalar_batch": "mc::k_box_scalar_batch<true>", "ir_resid": "mc::k_ir_resid<-7>"}
 KC_COUNT = len(KC_NAMES)
 # stages of the SIMPLE iteration (MC_ST_*)
 ST_NAMES = ["grad", "vel_flux", "vel_solve", "pres_flux", "pres_solve", "pres_correct", "turb_flux", "turb_solve",
