@@ -1913,9 +1913,9 @@ template <> float *lv_dinv<float>(AmgLevel &L) { return L.dinv32; }
 // (k_jac_first2, k_jac, k_resid_restrict_seq / k_resid_restrict, k_jac_prolong,
 // k_dense_apply) in the same order, so the result is the same.
 // Sizes: LDS holds VT_SUM rows in all; a first level beyond VT_ROWS takes
-// longer on one CU than its launches do on all of them.  Measured: modifier 33
-// mixed (13 launches of the two CSR levels below 9,537 rows into one) 47 us per
-// cycle, ten timesteps 92 -> 82 ms.
+// longer on one CU than its launches do on all of them.  Measured when it also
+// took hierarchies of CSR levels only (now k_csr_tail's): modifier 33 mixed, 13
+// launches of the two levels below 8,985 rows into one, ten timesteps 92 -> 82 ms.
 constexpr int VT_LEVELS = 4, VT_ROWS = 2304, VT_SUM = 4096, TAIL_THREADS = 1024;
 
 template <typename T>
@@ -2116,6 +2116,206 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_vtail(VtArgs<T> a, const KStat
         if (cur != dst) {
             for (int i = tid; i < n; i += TAIL_THREADS) dst[i] = cur[i];
             __syncthreads();
+        }
+    }
+}
+
+// The same cycle where every level left is in CSR storage and small enough for
+// a thread to keep its entries in registers: eight lanes a row, nine rows a
+// thread, the first sixteen entries of a row (the pairwise levels below a box of
+// odd sides have 7 on average and up to 19; the rest is fetched again on each
+// pass).  In k_vtail each of a level's seven passes waits three times for its
+// entries; here they are loaded once on the way down and once on the way up (the
+// last level once), and a pass reads x from LDS only.  It is then bound by LDS and
+// vector instructions of one CU, so the rows' own work is spread: lane l of the
+// eight finishes the thread's row l (every lane has every sum).  x is held as
+// doubles, rounded to T at every store: gathers then need no conversion, which
+// runs at a quarter of the rate.  Modifier 33 mixed (1,124 and 143 rows, dense
+// 73): k_vtail 47 us, this 31; ten timesteps 67.2 -> 62.1 ms.  A thread per row
+// (two rows of sixteen entries) needs the eight partial sums in registers too and
+// spills: 80 us.
+constexpr int CT_ROWS = 1152, CT_NC = 384, CT_SUM = 2048;
+
+template <typename T>
+struct CtRows {
+    static constexpr int R = CT_ROWS / 128, E = 2;
+    static_assert(R == 9, "rows 0 to 7 are finished by the eight lanes, row 8 by lane 0");
+    double v[R][E];
+    unsigned cp[R];      // a row's two columns
+    // bit r: this lane has a first / second entry of row r, the row has more
+    unsigned one, two, longer;
+
+    __device__ __forceinline__ void load(const VtLevel<T> &L, const int *rp)
+    {
+        const int n = L.A.n, lane8 = threadIdx.x & 7, g = threadIdx.x >> 3;
+        one = two = longer = 0;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            cp[r] = 0;
+            v[r][0] = v[r][1] = 0.0;
+            if (128 * r >= n) continue;
+            const int i = min(g + 128 * r, n - 1);
+            const int beg = rp[i], end = rp[i + 1];
+            longer |= (end - beg > 8 * E ? 1u : 0u) << r;
+            const int k0 = beg + lane8, k1 = k0 + 8;
+            const int q0 = k0 < end ? k0 : beg, q1 = k1 < end ? k1 : beg;
+            one |= (k0 < end ? 1u : 0u) << r;
+            two |= (k1 < end ? 1u : 0u) << r;
+            v[r][0] = (double)L.A.csr[q0];
+            v[r][1] = (double)L.A.csr[q1];
+            cp[r] = (unsigned)L.A.col[q0] | (unsigned)L.A.col[q1] << 16;
+        }
+    }
+    // f(r, i, this lane's part of (A src)_i) for every row of the thread
+    template <typename F>
+    __device__ __forceinline__ void parts(const VtLevel<T> &L, const int *rp, const double *src, F f) const
+    {
+        const int n = L.A.n, lane8 = threadIdx.x & 7, g = threadIdx.x >> 3;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if (128 * r >= n) continue;
+            const int i = g + 128 * r;
+            double acc = fma(v[r][0], src[cp[r] & 0xffffu], 0.0);
+            if (!(one >> r & 1)) acc = 0.0;
+            if (two >> r & 1) acc = fma(v[r][1], src[cp[r] >> 16], acc);
+            if (longer >> r & 1) {
+                const int ii = min(i, n - 1);
+                for (int k = rp[ii] + 8 * E + lane8; k < rp[ii + 1]; k += 8)
+                    acc = fma((double)L.A.csr[k], src[L.A.col[k]], acc);
+            }
+            f(r, i, acc);
+        }
+    }
+    // f(i, (A src)_i), each row by one lane
+    template <typename F>
+    __device__ __forceinline__ void rows(const VtLevel<T> &L, const int *rp, const double *src, F f) const
+    {
+        const int n = L.A.n, lane8 = threadIdx.x & 7, g = threadIdx.x >> 3;
+        double mine = 0.0, last = 0.0;
+        parts(L, rp, src, [&](int r, int, double acc) {
+            acc = lane8_sum(acc);
+            if (r == 8) last = acc;
+            else if (lane8 == r) mine = acc;
+        });
+        const int i = g + 128 * lane8;
+        if (i < n) f(i, mine);
+        if (lane8 == 0 && g + 1024 < n) f(g + 1024, last);
+    }
+};
+
+template <typename T>
+__global__ void __launch_bounds__(TAIL_THREADS) k_csr_tail(VtArgs<T> a, const KState *stop)
+{
+    if (stop && stop->all_done) return;
+    __shared__ double xs[CT_SUM], alt[CT_ROWS], pl[CT_ROWS * 8];
+    __shared__ T bl[CT_SUM], dl[CT_SUM];
+    // row pointers, aggregates, their members and the members' ranges
+    __shared__ int rps[CT_SUM + VT_LEVELS];
+    __shared__ unsigned short ag[CT_SUM], am[CT_SUM], ap[CT_SUM + VT_LEVELS];
+    __shared__ double bs[DENSE_MAX], xd[DENSE_MAX], part[TAIL_THREADS / DENSE_MAX][DENSE_MAX];
+    const int tid = threadIdx.x, lane8 = tid & 7, g = tid >> 3, nu = a.nu;
+    for (int l = 0; l < a.nl; l++)
+        for (int i = tid; i <= a.lv[l].A.n; i += TAIL_THREADS) {
+            const VtLevel<T> &L = a.lv[l];
+            rps[L.rpo + i] = L.A.rp[i];
+            if (i <= L.nc) ap[L.rpo + i] = (unsigned short)L.aptr[i];
+            if (i < L.A.n) {
+                dl[L.off + i] = L.dinv[i];
+                ag[L.off + i] = (unsigned short)L.agg[i];
+                am[L.off + i] = (unsigned short)L.amem[i];
+            }
+        }
+    for (int i = tid; i < a.lv[0].A.n; i += TAIL_THREADS) bl[i] = a.b[i];
+    __syncthreads();
+    CtRows<T> M;
+    for (int l = 0; l < a.nl; l++) {
+        const VtLevel<T> &L = a.lv[l];
+        const int n = L.A.n;
+        double *x = xs + L.off;
+        const T *b = bl + L.off;
+        const int *rp = rps + L.rpo;
+        const T *di = dl + L.off;
+        const T w1 = (T)a.w[0], w2 = (T)a.w[nu >= 2 ? 1 : 0];
+        // the buffer from which nu - 1 sweeps end in x
+        double *cur = (nu - 1) & 1 ? alt : x, *oth = (nu - 1) & 1 ? x : alt;
+        for (int i = tid; i < n; i += TAIL_THREADS) cur[i] = (double)vc_first(w1, di[i], b[i]);
+        M.load(L, rp);
+        __syncthreads();
+        for (int k = 1; k < nu; k++) {
+            const T omega = (T)a.w[k];
+            if (k == 1)
+                M.rows(L, rp, cur, [&](int i, double ax) { oth[i] = (double)vc_first2(w1, w2, di[i], b[i], ax); });
+            else
+                M.rows(L, rp, cur,
+                       [&](int i, double ax) { oth[i] = (double)vc_jac((T)cur[i], omega, di[i], b[i], ax); });
+            __syncthreads();
+            double *sw = cur; cur = oth; oth = sw;
+        }
+        M.parts(L, rp, x, [&](int, int i, double acc) {
+            if (i < n) pl[8 * i + lane8] = acc;
+        });
+        __syncthreads();
+        const bool dense = l + 1 == a.nl;
+        T *bc = dense ? nullptr : bl + a.lv[l + 1].off;
+        for (int I0 = 0; I0 < L.nc; I0 += 128) {
+            const int I = min(I0 + g, L.nc - 1);
+            const int t0 = ap[L.rpo + I], cnt = ap[L.rpo + I + 1] - t0;
+            double s = 0.0;
+            for (int t = 0; t < cnt; t++) {
+                const int i = am[L.off + t0 + t];
+                if (lane8 == 0) s += (double)b[i];
+                s -= pl[8 * i + lane8];
+            }
+            s = lane8_sum(s);
+            if (lane8 == 0 && I0 + g < L.nc) { if (dense) bs[I] = (double)(T)s; else bc[I] = (T)s; }
+        }
+        __syncthreads();
+    }
+    {   // dense coarsest level, as k_dense_apply
+        constexpr int PARTS = TAIL_THREADS / DENSE_MAX, PLEN = DENSE_MAX / PARTS;
+        const int nd = a.nd;
+        const int i = tid % DENSE_MAX, p = tid / DENSE_MAX;
+        double sum = 0.0;
+        if (i < nd) {
+            const int j0 = p * PLEN;
+#pragma unroll
+            for (int jj = 0; jj < PLEN; jj++) {
+                const int j = j0 + jj;
+                if (j < nd) sum = fma(a.inv[(size_t)j * nd + i], bs[j], sum);
+            }
+        }
+        part[p][i] = sum;
+        __syncthreads();
+        if (tid < nd) {
+            double y = 0.0;
+#pragma unroll
+            for (int q = 0; q < PARTS; q++) y += part[q][tid];
+            xd[tid] = (double)(T)y;
+        }
+        __syncthreads();
+    }
+    for (int l = a.nl - 1; l >= 0; l--) {
+        const VtLevel<T> &L = a.lv[l];
+        const int n = L.A.n;
+        const double *xc = l + 1 == a.nl ? xd : xs + a.lv[l + 1].off;
+        double *x = xs + L.off;
+        const T *b = bl + L.off;
+        const int *rp = rps + L.rpo;
+        const T *di = dl + L.off;
+        double *cur = nu & 1 ? alt : x, *oth = nu & 1 ? x : alt;
+        for (int i = tid; i < n; i += TAIL_THREADS) cur[i] = (double)vc_prolong((T)x[i], a.cs, (T)xc[ag[L.off + i]]);
+        if (l + 1 != a.nl) M.load(L, rp);   // the last level's entries are still there
+        __syncthreads();
+        for (int k = 0; k < nu; k++) {
+            const T omega = (T)a.w[nu - 1 - k];
+            const bool out = l == 0 && k == nu - 1;
+            M.rows(L, rp, cur, [&](int i, double ax) {
+                const T y = vc_jac((T)cur[i], omega, di[i], b[i], ax);
+                if (out) a.x[i] = y;
+                else oth[i] = (double)y;
+            });
+            __syncthreads();
+            double *sw = cur; cur = oth; oth = sw;
         }
     }
 }
@@ -2698,12 +2898,18 @@ static int vcycle(Ctx *c, size_t l, const T *b, T *x, KState *ks, const KState *
         // small and in seven-diagonal or CSR storage
         const size_t nl = c->amg.size() - 1 - l;
         bool ok = nl <= (size_t)VT_LEVELS && nu <= 8 && L.n <= VT_ROWS;
+        bool csr = true;
         int sum = 0;
         for (size_t k = l; ok && k + 1 < c->amg.size(); k++) {
             const int code = nd_code(level_mat<T>(c->amg[k]));
             sum += c->amg[k].n;
+            csr = csr && code == 0;
             ok = (code == 0 || code == (sizeof(T) == 8 ? -7 : 7)) && sum <= VT_SUM;
         }
+        // CSR levels only: in registers, from the first level that fits
+        // (the larger ones' launches are faster than k_vtail's passes: modifier 41, 2,154
+        // rows, a timestep 7.8 -> 7.0 ms)
+        if (csr) ok = ok && L.n <= CT_ROWS && L.nc <= CT_NC && sum <= CT_SUM;
         if (ok) {
             VtArgs<T> ta;
             memset(&ta, 0, sizeof(ta));
@@ -2725,7 +2931,8 @@ static int vcycle(Ctx *c, size_t l, const T *b, T *x, KState *ks, const KState *
             for (int k = 0; k < 8; k++) ta.w[k] = wts[k];
             MC_TRY(dense_join(c));
             constexpr bool SYM = sizeof(T) == 8;   // FP64 seven-diagonal levels keep the upper diagonals
-            hipLaunchKernelGGL((k_vtail<SYM, T>), dim3(1), dim3(TAIL_THREADS), 0, c->stream, ta, stop);
+            if (csr) hipLaunchKernelGGL(k_csr_tail<T>, dim3(1), dim3(TAIL_THREADS), 0, c->stream, ta, stop);
+            else hipLaunchKernelGGL((k_vtail<SYM, T>), dim3(1), dim3(TAIL_THREADS), 0, c->stream, ta, stop);
             MC_LAUNCH_CHECK(c);
             return MC_OK;
         }
