@@ -69,6 +69,9 @@ struct AmgLevel {
     // members and the Galerkin sums are arithmetic and need no index arrays
     int bx = 0, by = 0, bz = 0;
     int sx = 0, sy = 0, sz = 0;
+    // a matched level that came out as a box halved in every direction (rx > 0:
+    // rx x ry x rz cells, no entry across a row's or plane's end)
+    int rx = 0, ry = 0, rz = 0;
     // aggregation to the next level
     int nc = 0;
     int *agg = nullptr;                       // [n] aggregate id

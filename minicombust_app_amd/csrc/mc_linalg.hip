@@ -1203,6 +1203,34 @@ __global__ void __launch_bounds__(1024) k_dense_inverse(DenseSrc src, double *in
             if (i0 + a < n && j0 + b < n) inv[(size_t)(j0 + b) * n + i0 + a] = m[a][b];
 }
 
+// Pairwise matching on a box of even sides pairs along x, y and z in turn: the
+// aggregates are its 2 x 2 x 2 blocks, numbered in order.  Such a level's transfers
+// need no index arrays (k_box_restrict, k_box_jac_prolong).
+static void regular_level(AmgLevel &L, const HostCSR &A, const std::vector<int> &agg, int nc)
+{
+    if (L.nd != 7 || L.off[4] != 1 || L.off[5] <= 1 || L.off[6] <= L.off[5]) return;
+    const int nx = L.off[5], nxny = L.off[6];
+    for (int d = 0; d < 7; d++)
+        if (L.off[d] != -L.off[6 - d]) return;
+    if (nxny % nx || A.n % nxny) return;
+    const int ny = nxny / nx, nz = A.n / nxny, cx = (nx + 1) >> 1, cy = (ny + 1) >> 1, cz = (nz + 1) >> 1;
+    if (nc != cx * cy * cz) return;
+    int i = 0;
+    for (int z = 0; z < nz; z++)
+        for (int y = 0; y < ny; y++)
+            for (int x = 0; x < nx; x++, i++) {
+                if (agg[i] != (x >> 1) + cx * ((y >> 1) + cy * (z >> 1))) return;
+                for (int k = A.rp[i]; k < A.rp[i + 1]; k++) {   // entries of coordinate neighbours only
+                    const int o = A.col[k] - i;
+                    if ((o == 1 && x + 1 == nx) || (o == -1 && x == 0) || (o == nx && y + 1 == ny) ||
+                        (o == -nx && y == 0))
+                        return;
+                }
+            }
+    L.rx = nx; L.ry = ny; L.rz = nz;
+}
+
+
 static int amg_build(Ctx *c, const double *vals);
 
 // Aggregation-AMG hierarchy from the pressure matrix (host aggregation and
@@ -1241,9 +1269,15 @@ struct BoxDims {
 static BoxDims box_dims(const AmgLevel &L)
 {
     BoxDims b;
-    b.nx = L.bx; b.ny = L.by; b.nz = L.bz; b.n = L.n;
-    b.sx = L.sx; b.sy = L.sy; b.sz = L.sz;
-    b.cx = (L.bx + L.sx) >> L.sx; b.cy = (L.by + L.sy) >> L.sy; b.cz = (L.bz + L.sz) >> L.sz;
+    b.n = L.n;
+    if (L.bx) {
+        b.nx = L.bx; b.ny = L.by; b.nz = L.bz;
+        b.sx = L.sx; b.sy = L.sy; b.sz = L.sz;
+    } else {
+        b.nx = L.rx; b.ny = L.ry; b.nz = L.rz;
+        b.sx = b.sy = b.sz = 1;
+    }
+    b.cx = (b.nx + b.sx) >> b.sx; b.cy = (b.ny + b.sy) >> b.sy; b.cz = (b.nz + b.sz) >> b.sz;
     b.nc = b.cx * b.cy * b.cz;
     return b;
 }
@@ -1510,6 +1544,7 @@ static int amg_build(Ctx *c, const double *vals)
         std::vector<int> gp, gm;
         galerkin(cur, agg, nc, Ac, &gp, &gm);
         L.nc = nc;
+        regular_level(L, cur, agg, nc);
         MC_TRY(dalloc(c, &L.agg, L.n));
         MC_HIP(c, hipMemcpy(L.agg, agg.data(), (size_t)L.n * 4, hipMemcpyHostToDevice));
         {
@@ -2478,6 +2513,39 @@ __global__ void __launch_bounds__(BLOCK) k_box_restrict(BoxWalk w, R resid, T *b
     if (lane8 == 0 && I < b.nc) bc[I] = (T)s;
 }
 
+// The same on a regular matched level, the members added in ascending order as
+// k_restrict does.  A lane per x and coarse y, z: it forms the residuals of its four
+// rows (64 adjacent ones per load), the even lane of a pair adds both lanes' in
+// order.  4,194,304 rows, us: FP64 k_resid 31 + k_restrict 15 -> 32, the FP16 copy 33
+// -> 19 (eight lanes a coarse cell, as above: 44 and 58; a thread a coarse cell: 68
+// and 38).
+template <class R, typename T>
+__global__ void __launch_bounds__(BLOCK) k_reg_restrict(BoxWalk w, R resid, T *bc, const KState *stop)
+{
+    if (stop && stop->all_done) return;
+    const BoxDims &b = w.b;
+    const int t = xcd_block(blockIdx.x, gridDim.x) * BLOCK + threadIdx.x, I = t >> 1;
+    if (I >= b.nc) return;   // both lanes of the pair
+    const int Z = fdiv(I, w.cdxy), q = I - Z * (b.cx * b.cy), Y = fdiv(q, w.cdx), X = q - Y * b.cx;
+    const int x = 2 * X + (t & 1), y = 2 * Y, z = 2 * Z;
+    double r[4], o[4];
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        const bool in = x < b.nx && y + (m & 1) < b.ny && z + (m >> 1) < b.nz;
+        const int i = min(x, b.nx - 1) + b.nx * (min(y + (m & 1), b.ny - 1) + b.ny * min(z + (m >> 1), b.nz - 1));
+        const double v = resid(i);
+        r[m] = in ? v : 0.0;   // adds +0 to a sum that starts at +0
+    }
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+        o[m] = __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(r[m]), 0xB1, 0xf, 0xf, false),
+                                __builtin_amdgcn_update_dpp(0, __double2loint(r[m]), 0xB1, 0xf, 0xf, false));
+    double s = 0.0;
+#pragma unroll
+    for (int m = 0; m < 4; m++) { s += r[m]; s += o[m]; }
+    if (!(t & 1)) bc[I] = (T)s;
+}
+
 // The prolongation and the first post-smoothing sweep in one pass: every
 // value the sweep reads is the prolonged x_j + cs xc[aggregate of j], the
 // aggregate from j's coordinates (no index array), so the prolonged vector is
@@ -2981,23 +3049,32 @@ static int vcycle(Ctx *c, size_t l, const T *b, T *x, KState *ks, const KState *
     T *bc = lv_b<T>(Lc), *xc = lv_x<T>(Lc);
     // below the finest level the residual and the restriction, and the
     // prolongation and the first post-smoothing sweep, share a launch
-    const bool box = L.bx != 0;
+    constexpr int BND = sizeof(T) == 8 ? -7 : 7;   // the box levels' storage (level_mat)
+    const bool reg = L.rx != 0 && nd_code(A) == BND;
+    const bool box = L.bx != 0 || reg;
     const bool fuse = l >= 1 && !half;
-    if (box) {
+    // below the finest level k_reg_restrict's four rows a lane pay from REG_ROWS on
+    // (FP64, us against k_resid_restrict_seq: 65,536 rows 6.6 / 9, 8,192 rows 5.1 / 4)
+    constexpr int REG_ROWS = 32768;
+    if (box && !(reg && fuse && L.n < REG_ROWS)) {
         const BoxWalk w = box_walk(L);
         const dim3 gr(div_up(L.nc, BLOCK / 8));
         bool launched = false;
         if constexpr (sizeof(T) == 4) {
             if (half) {
-                hipLaunchKernelGGL((k_box_restrict<ResidH, float>), gr, dim3(BLOCK), 0, c->stream, w,
-                                   ResidH{H, b, cur}, bc, stop);
+                const ResidH rh{H, b, cur};
+                if (reg) hipLaunchKernelGGL((k_reg_restrict<ResidH, float>), dim3(div_up(2 * L.nc, BLOCK)), dim3(BLOCK), 0,
+                                            c->stream, w, rh, bc, stop);
+                else hipLaunchKernelGGL((k_box_restrict<ResidH, float>), gr, dim3(BLOCK), 0, c->stream, w, rh, bc, stop);
                 launched = true;
             }
         }
         if (!launched) {
-            constexpr int BND = sizeof(T) == 8 ? -7 : 7;   // the box levels' storage (level_mat)
-            hipLaunchKernelGGL((k_box_restrict<ResidDia<BND, T>, T>), gr, dim3(BLOCK), 0, c->stream, w,
-                               (ResidDia<BND, T>{A, b, cur}), bc, stop);
+            using RD = ResidDia<BND, T>;
+            const RD rd{A, b, cur};
+            if (reg) hipLaunchKernelGGL((k_reg_restrict<RD, T>), dim3(div_up(2 * L.nc, BLOCK)), dim3(BLOCK), 0, c->stream,
+                                        w, rd, bc, stop);
+            else hipLaunchKernelGGL((k_box_restrict<RD, T>), gr, dim3(BLOCK), 0, c->stream, w, rd, bc, stop);
         }
     } else if (fuse && A.nd) {
         MC_DISPATCH_ND(nd_code(A), (k_resid_restrict_seq<ND_, T>), dim3(div_up(L.nc, BLOCK / 8)), dim3(BLOCK), 0,
@@ -3044,7 +3121,6 @@ static int vcycle(Ctx *c, size_t l, const T *b, T *x, KState *ks, const KState *
                 }
             }
             if (!launched) {
-                constexpr int BND = sizeof(T) == 8 ? -7 : 7;
                 hipLaunchKernelGGL((k_box_jac_prolong<BND, T>), dim3(g.blocks), dim3(BLOCK), 0, c->stream, pr, A, dinv,
                                    b, dst, om, g.chunk, dotv, c->red, stop);
             }
@@ -3082,8 +3158,8 @@ static int vcycle(Ctx *c, size_t l, const T *b, T *x, KState *ks, const KState *
 // neither written nor read again: M + 2Tn + 4(n + nc + 1) + T nc) and the
 // prolongation is folded into the first post-smoothing sweep (that sweep
 // reads the aggregate ids and the coarse correction, 4n + T nc, and no
-// prolonged vector is written or read).  Box levels do the same on every
-// level and read no aggregate ids.  On the FP16 copy M is its six
+// prolonged vector is written or read).  Box levels and regular matched ones do
+// the same on every level and read no aggregate ids.  On the FP16 copy M is its six
 // off-diagonals (12n) and D the FP32 inverse diagonal; the dense coarsest
 // solve reads its inverse (8 n^2) and b, writes x.
 template <typename T>
@@ -3104,7 +3180,7 @@ static double vcycle_bytes(Ctx *c)
         const double D = half ? 4.0 * n : t * n;
         b += (nu >= 2 ? M : 0.0) + D + 2.0 * t * n;
         b += (double)std::max(0, nu - 2) * (M + D + 3.0 * t * n);
-        if (L.bx) {
+        if (L.bx || (L.rx && nd_code(level_mat<T>(L)) == (sizeof(T) == 8 ? -7 : 7))) {
             b += M + (half ? 8.0 * n : 0.0) + 2.0 * t * n + t * L.nc;
             b += t * L.nc;
         } else if (l >= 1 && !half) {
