@@ -143,12 +143,12 @@ static Sizes sizes_of(const Ctx *c)
 // their sides' places), so the results are the general kernels' bit for bit.
 //
 // m = 128 (4,194,304 cells), general -> box kernels, us: k_grad<11> 570 -> 466,
-// k_grad<1> 120 -> 65, k_momentum 635 -> 390, k_scalar 495 -> 281 (mean of TE
-// and ED), k_scalar_batch<true> beside the ED solve 1200 -> 753, k_mass_faces
-// 487 -> 274, k_mass_rows 274 -> 260, k_flux_correct 282 -> 134,
-// k_cell_correct 145 -> 98.  They move little beyond what they must (momentum:
-// 0.86 GB read and 0.67 written of 0.80 + 0.67) at 3 to 4 TB/s, with up to 44
-// separate streams each.
+// k_grad<1> 120 -> 65, k_momentum 635 -> 390 (341 inside an iteration, without
+// ff0 and ff1), k_scalar 495 -> 281 (mean of TE and ED; 239), k_scalar_batch<true>
+// beside the ED solve 1200 -> 630 to 750, k_mass_faces 487 -> 274 (258),
+// k_mass_rows 274 -> 252, k_flux_correct 282 -> 134, k_cell_correct 145 -> 98.
+// They move little beyond what they must (momentum: 0.86 GB read and 0.67 written
+// of 0.80 + 0.67) at 3 to 4 TB/s, with up to 44 separate streams each.
 struct BoxG {
     int nx, ny, nz, N, nxny;
     const double *cc[3], *w[3], *lam[3], *dist[3], *fc[3], *ft[3][3], *vis[3];
@@ -156,6 +156,7 @@ struct BoxG {
     // boundary faces keep the arrays
     const double *fcx, *fcy, *fcz, *fnx, *fny, *fnz, *farea, *frlc;
     int btype[6], last_face[6];
+    bool lean;   // Ctx::lean: arrays that a later stage of the iteration overwrites unread are not stored
     CellWalk wk;
 };
 
@@ -175,6 +176,7 @@ static BoxG box_geo(const Ctx *c, int vis = 0)
     g.fcx = c->fcx; g.fcy = c->fcy; g.fcz = c->fcz; g.fnx = c->fnx; g.fny = c->fny; g.fnz = c->fnz;
     g.farea = c->farea; g.frlc = c->frlc;
     for (int s = 0; s < 6; s++) { g.btype[s] = c->btype[s]; g.last_face[s] = c->last_face[s]; }
+    g.lean = c->lean;
     g.wk = cell_walk(c);
     return g;
 }
@@ -781,7 +783,7 @@ __global__ void __launch_bounds__(256) k_box_momentum(BoxG g, MomArgs a)
             SV = SV + fvde - fvdi;
             SW = SW + fwde - fwdi;
             ff[s] = ff1;
-            st_out(&a.ff0[q.f[s]], ff0); st_out(&a.ff1[q.f[s]], ff1);
+            if (!g.lean) { st_out(&a.ff0[q.f[s]], ff0); st_out(&a.ff1[q.f[s]], ff1); }
         } else {
             SU = SU - fude + fudi;
             SV = SV - fvde + fvdi;
@@ -908,7 +910,7 @@ static double momentum_bytes(Ctx *c, bool r0)
 {
     const Sizes z = sizes_of(c);
     if (box_on(c))
-        return (160.0 + (r0 ? 24.0 : 0.0)) * z.N + 8.0 * z.F + 16.0 * z.Fi + 64.0 * z.Fb + 8.0 * z.nnz;
+        return (160.0 + (r0 ? 24.0 : 0.0)) * z.N + 8.0 * z.F + (c->lean ? 0.0 : 16.0) * z.Fi + 64.0 * z.Fb + 8.0 * z.nnz;
     return (248.0 + (r0 ? 24.0 : 0.0)) * z.N + 48.0 * z.F + 16.0 * z.Fi + 32.0 * z.Fb + 8.0 * z.nnz;
 }
 
@@ -1262,7 +1264,8 @@ __global__ void __launch_bounds__(256) k_box_mass_faces(BoxG g, MassArgs a)
         double ApV;
         const double m = rhie_chow(f, own, other, ApV);
         st_out(&a.mflux[q.f[s]], m);
-        st_out(&a.ff0[q.f[s]], -ApV); st_out(&a.ff1[q.f[s]], -ApV);
+        st_out(&a.ff0[q.f[s]], -ApV);
+        if (!g.lean) st_out(&a.ff1[q.f[s]], -ApV);
     };
     // any order: the faces are independent
     if (q.in[3]) face(SideTag<3>());
@@ -1300,7 +1303,7 @@ __global__ void __launch_bounds__(256) k_box_mass_rows(BoxG g, const int *row_pt
         AV -= v[s];
     }
     a.SU[c] = S;
-    a.AV[c] = AV;
+    if (!g.lean) a.AV[c] = AV;
     if (!a.into_pressure) return;
     a.Pb[c] = S;
     {   // CSR: ascending columns -z -y -x main +x +y +z
@@ -1474,8 +1477,9 @@ static double mass_bytes(Ctx *c, const MassArgs &a)
 {
     const Sizes z = sizes_of(c);
     const bool box = box_on(c);
-    double b = box ? 136.0 * z.N + 24.0 * z.Fi : 224.0 * z.N + 88.0 * z.Fi;          // faces
-    b += (box ? 28.0 : 72.0) * z.N + 8.0 * z.F + 8.0 * z.Fi + 8.0 * z.nnz;           // rows
+    const bool lean = box && c->lean;
+    double b = box ? 136.0 * z.N + (lean ? 16.0 : 24.0) * z.Fi : 224.0 * z.N + 88.0 * z.Fi;   // faces
+    b += (lean ? 20.0 : box ? 28.0 : 72.0) * z.N + 8.0 * z.F + 8.0 * z.Fi + 8.0 * z.nnz;           // rows
     if (a.pdia) b += 8.0 * (z.N + z.Fi) + 4.0 * z.nnz + 12.0 * z.N;
     if (a.phoff) b += 4.0 * z.N + 4.0 * z.Fi;
     return b;
@@ -1662,7 +1666,7 @@ int calculate_pressure(Ctx *c)
         const bool fresh = simple || c->first_pressure || c->u == nullptr;
         StageTimer ts(c, MC_ST_PRES_SOLVE);
         c->p_zero = false;
-        if (simple) {
+        if (simple && loop > 1) {   // the assembly has stored the first loop's
             MC_HIP(c, hipMemcpyAsync(c->Pb, c->SU, (size_t)N * 8, hipMemcpyDeviceToDevice, c->stream));
         }
         if (fresh || !c->st.p_solves) {
@@ -2183,7 +2187,7 @@ __global__ void __launch_bounds__(256) k_box_scalar(BoxG g, ScalArgs a)
         if constexpr (TAG::high) {
             S = S + fde1 - fdi;
             ff[s] = ff1;
-            st_out(&a.ff0[q.f[s]], ff0); st_out(&a.ff1[q.f[s]], ff1);
+            if (!g.lean) { st_out(&a.ff0[q.f[s]], ff0); st_out(&a.ff1[q.f[s]], ff1); }
         } else {
             S = S - fde1 + fdi;
             ff[s] = ff0;
@@ -2288,7 +2292,7 @@ __global__ void __launch_bounds__(256) k_box_scalar(BoxG g, ScalArgs a)
     A = box_minus_off(q, ff, A);
     A *= (1. / a.urf);
     S = S + (1.0 - a.urf) * A * phic;
-    st_out(&a.AV[c], A);
+    if (!g.lean) st_out(&a.AV[c], A);
     st_out(&a.SU[c], S);
     if (a.r0) st_out(&a.r0[c], S - (A * pc + xo));
     box_store_row(g, q, ff, A, a.dia);
@@ -2646,11 +2650,12 @@ int scalar_assemble(Ctx *c, int type, double *r0)
     // box kernel: no cell or interior face geometry, forder, fother or flags
     const Sizes z = sizes_of(c);
     const bool box = box_on(c) && a.dia;
-    double cell = (box ? 48.0 : 136.0) + (r0 ? 8.0 : 0.0);
+    const bool lean = box && c->lean;
+    double cell = (lean ? 40.0 : box ? 48.0 : 136.0) + (r0 ? 8.0 : 0.0);
     if (type == TERBTE) cell += 88.0;
     if (type == TERBED) cell += box ? 16.0 : 17.0;
-    KTimer kt(c, MC_KC_SCALAR_ASM, cell * z.N + (box ? 8.0 : 48.0) * z.F + 16.0 * z.Fi + (box ? 56.0 : 24.0) * z.Fb +
-                                       8.0 * z.nnz);
+    KTimer kt(c, MC_KC_SCALAR_ASM, cell * z.N + (box ? 8.0 : 48.0) * z.F + (lean ? 0.0 : 16.0) * z.Fi +
+                                       (box ? 56.0 : 24.0) * z.Fb + 8.0 * z.nnz);
     const dim3 gr(walk_blocks(cell_walk(c)));
     if (!box)
         hipLaunchKernelGGL(k_scalar, gr, dim3(256), 0, c->stream, geo(c), a);
@@ -2979,6 +2984,16 @@ int scalar_solve(Ctx *c, int type, bool fork_batch)
 // ============================================================= A17 ==
 int simple_iteration(Ctx *c, int inner)
 {
+    // With the scalars solved, ff0 and ff1 of the momentum and TE / ED assembly, ff1
+    // of the pressure assembly and A_V up to the batched assembly are written again
+    // before anything reads them: the box kernels leave those stores out
+    // (4,194,304 cells, us: momentum 390 -> 341, TE 258 -> 217, ED 305 -> 260,
+    // Rhie-Chow fluxes 274 -> 258).
+    struct Lean {
+        Ctx *c;
+        ~Lean() { c->lean = false; }
+    } lean{c};
+    c->lean = c->opt.solve_scalars != 0;
     {
         StageTimer t(c, MC_ST_GRAD);
         MC_TRY(grad_multi(c, c->opt.limit_grad != 0));   // + limit_phi_gradients, FlowSolver.inl:3197-3198

@@ -159,6 +159,7 @@ struct Ctx {
         double zero[3][3] = {};      // [a][b]: the (signed) zero component b of the normals of faces normal to a
         double rho = 0.0;
     } box;
+    bool lean = false;               // inside a SIMPLE iteration that ends with the scalars' assembly
 
     // ---- fields ----
     double *phi[NFIELDS] = {};
