@@ -145,8 +145,7 @@ static Sizes sizes_of(const Ctx *c)
 // m = 128 (4,194,304 cells), general -> box kernels, us: k_grad<11> 570 -> 466,
 // k_grad<1> 120 -> 65, k_momentum 635 -> 390 (341 inside an iteration, without
 // ff0 and ff1), k_scalar 495 -> 281 (mean of TE and ED; 239), k_scalar_batch<true>
-// beside the ED solve 1200 -> 630 to 750, k_mass_faces 487 -> 274 (258),
-// k_mass_rows 274 -> 252, k_flux_correct 282 -> 134, k_cell_correct 145 -> 98.
+// 840 -> 412, k_mass_faces 487 -> 274 (258), k_mass_rows 274 -> 252, k_flux_correct 282 -> 134, k_cell_correct 145 -> 98.
 // They move little beyond what they must (momentum: 0.86 GB read and 0.67 written
 // of 0.80 + 0.67) at 3 to 4 TB/s, with up to 44 separate streams each.
 struct BoxG {
@@ -1707,8 +1706,10 @@ int calculate_pressure(Ctx *c)
             {
                 // per cell centre, grad PP (48), PP (8), forder and fother (48)
                 // read; per interior face ff0, mass flux, centre, normal (64)
-                // read and mass flux, correction (16) written
-                KTimer kt(c, MC_KC_CORRECT, 104.0 * c->N + 80.0 * (double)(c->F - c->Fb));
+                // read and mass flux, correction (16) written; the box kernel: PP,
+                // ff0, mass flux read, mass flux and correction written
+                const double Fi = (double)(c->F - c->Fb);
+                KTimer kt(c, MC_KC_CORRECT, box_on(c) ? 8.0 * c->N + 32.0 * Fi : 104.0 * c->N + 80.0 * Fi);
                 if (box_on(c))
                     hipLaunchKernelGGL(k_box_flux_correct, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream,
                                        box_geo(c), c->phi[PP], c->gx[PP], c->gy[PP], c->gz[PP], c->ff0, c->mflux,
@@ -2456,10 +2457,7 @@ __global__ void __launch_bounds__(256) k_box_scalar_batch(BoxG g, BoxVis tv, Sca
 // into its own matrix and solved first, as the reference orders them (none of
 // the four reads the temperature, and TEM's assembly reads nothing the TE /
 // ED solves change).
-// The batched pass's arguments.  side = true: it writes the alternate matrix,
-// diagonal and face-coefficient arrays and keeps VARP's right-hand side in
-// srhs[3] (S_U is then the ED system's), so it can run beside the ED solve.
-static ScalBatchArgs batch_args(Ctx *c, bool side)
+static ScalBatchArgs batch_args(Ctx *c)
 {
     static const int types[SB] = {FUEL, PROG, VARFU, VARPR};
     static const int fields[SB] = {FUL, PRO, VARF, VARP};
@@ -2467,13 +2465,13 @@ static ScalBatchArgs batch_args(Ctx *c, bool side)
     for (int s = 0; s < SB; s++) {
         a.phi[s] = c->phi[fields[s]];
         a.gx[s] = c->gx[fields[s]]; a.gy[s] = c->gy[fields[s]]; a.gz[s] = c->gz[fields[s]];
-        a.S[s] = (s == SB - 1 && !side) ? c->SU : c->srhs[s];   // S_phi.U ends holding VARP's, as in the reference
+        a.S[s] = s == SB - 1 ? c->SU : c->srhs[s];   // S_phi.U ends holding VARP's, as in the reference
         a.inlet_phi[s] = (types[s] == FUEL || types[s] == VARFU) ? c->k.gas_ful : 0.0;
     }
     a.mflux = c->mflux;
-    a.ff0 = side ? c->ff0b : c->ff0; a.ff1 = side ? c->ff1b : c->ff1; a.AV = side ? c->AV2 : c->AV;
+    a.ff0 = c->ff0; a.ff1 = c->ff1; a.AV = c->AV;
     a.vals = c->A_vals;
-    a.dia = side ? c->A_dia3 : (double *)fine_dia_of(c, c->A_vals);
+    a.dia = (double *)fine_dia_of(c, c->A_vals);
     a.type = FUEL;
     a.ev = c->k.ev; a.inlet_ev = c->k.inlet_ev; a.rdelta = c->k.rdelta; a.urf = 0.95;
     a.tphi = c->phi[TEM]; a.tgx = c->gx[TEM]; a.tgy = c->gy[TEM]; a.tgz = c->gz[TEM];
@@ -2481,7 +2479,7 @@ static ScalBatchArgs batch_args(Ctx *c, bool side)
     return a;
 }
 
-static void batch_launch(Ctx *c, const ScalBatchArgs &a, bool tem, hipStream_t s)
+static void batch_launch(Ctx *c, const ScalBatchArgs &a, bool tem)
 {
     // per cell and field phi and gradient (32) read and S (8) written;
     // per cell centre (24), volume and density (16), forder and fother
@@ -2495,17 +2493,17 @@ static void batch_launch(Ctx *c, const ScalBatchArgs &a, bool tem, hipStream_t s
     const bool box = box_on(c) && a.dia && (!tem || a.tdia);
     const double bytes = (40.0 * nsc + (box ? 8.0 : 96.0)) * z.N + (box ? 8.0 : 48.0) * z.F + 16.0 * z.Fi +
                          (box ? 56.0 : 24.0) * z.Fb + 8.0 * z.nnz * (tem ? 2 : 1);
-    KTimer kt(c, s == c->stream ? MC_KC_SCALAR_BATCH : -1, bytes);
+    KTimer kt(c, MC_KC_SCALAR_BATCH, bytes);
     if (box) {
         const dim3 gr(walk_blocks(cell_walk(c)));
         BoxVis tv;
         for (int k = 0; k < 3; k++) tv.v[k] = c->box.vis[3][k];
-        if (tem) hipLaunchKernelGGL(k_box_scalar_batch<true>, gr, dim3(256), 0, s, box_geo(c, 4), tv, a);
-        else hipLaunchKernelGGL(k_box_scalar_batch<false>, gr, dim3(256), 0, s, box_geo(c, 4), tv, a);
+        if (tem) hipLaunchKernelGGL(k_box_scalar_batch<true>, gr, dim3(256), 0, c->stream, box_geo(c, 4), tv, a);
+        else hipLaunchKernelGGL(k_box_scalar_batch<false>, gr, dim3(256), 0, c->stream, box_geo(c, 4), tv, a);
     } else if (tem)
-        hipLaunchKernelGGL(k_scalar_batch<true>, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, s, geo(c), a);
+        hipLaunchKernelGGL(k_scalar_batch<true>, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, geo(c), a);
     else
-        hipLaunchKernelGGL(k_scalar_batch<false>, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, s, geo(c), a);
+        hipLaunchKernelGGL(k_scalar_batch<false>, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream, geo(c), a);
 }
 
 // The solves of the batched pass's systems: TEM (its own matrix), then FUL,
@@ -2535,77 +2533,13 @@ static int batch_solves(Ctx *c, const ScalBatchArgs &a, bool tem)
 
 static int batch_solve(Ctx *c, bool tem)
 {
-    const ScalBatchArgs a = batch_args(c, false);
+    const ScalBatchArgs a = batch_args(c);
     {
         StageTimer t(c, MC_ST_SCA_FLUX);
-        batch_launch(c, a, tem, c->stream);
+        batch_launch(c, a, tem);
         MC_LAUNCH_CHECK(c);
     }
     return batch_solves(c, a, tem);
-}
-
-// The batched pass beside the ED solve: it reads nothing the TE / ED solves
-// write (scalar fields and gradients, mass fluxes, geometry) and writes its
-// own arrays, so it can run on the second stream from the end of ED's
-// assembly to the end of ED's solve and repair (not beside an assembly
-// kernel: TE / ED's `k_scalar` keeps the device to itself).  Unused while a
-// stage, the batch kernel or the BiCGStab kernel is timed: their events are
-// on the main stream and would take in the other stream's work.
-static bool batch_beside(const Ctx *c)
-{
-    const unsigned stages = ((1u << MC_ST_COUNT) - 1u) << MC_KC_COUNT;
-    return c->side && c->fine_nd && !(c->profile & (stages | (1u << MC_KC_SCALAR_BATCH) | (1u << MC_KC_BICG)));
-}
-
-// allocated at the first fork; cleared on the main stream, so the fork's
-// event orders the clearing before the batch kernel on the other stream
-static int batch_buffers(Ctx *c)
-{
-    if (c->A_dia3) return MC_OK;
-    {
-        MemScope ms(c, MC_MEM_MATRIX);
-        MC_TRY(dalloc(c, &c->A_dia3, (size_t)c->fine_nd * c->N));   // entries outside the pattern stay zero
-    }
-    {
-        MemScope ms(c, MC_MEM_FIELDS);
-        MC_TRY(dalloc(c, &c->AV2, c->N + 6));   // boundary slots zero, as AV's
-        MC_TRY(dalloc(c, &c->ff0b, c->F));      // boundary faces zero, as ff0's and ff1's
-        MC_TRY(dalloc(c, &c->ff1b, c->F));
-    }
-    MC_HIP(c, hipMemsetAsync(c->A_dia3, 0, (size_t)c->fine_nd * c->N * 8, c->stream));
-    MC_HIP(c, hipMemsetAsync(c->AV2, 0, (size_t)(c->N + 6) * 8, c->stream));
-    MC_HIP(c, hipMemsetAsync(c->ff0b, 0, (size_t)c->F * 8, c->stream));
-    MC_HIP(c, hipMemsetAsync(c->ff1b, 0, (size_t)c->F * 8, c->stream));
-    if (!c->ev_fork) MC_HIP(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
-    if (!c->ev_join) MC_HIP(c, hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
-    return MC_OK;
-}
-
-static int batch_fork(Ctx *c)
-{
-    MC_TRY(batch_buffers(c));
-    MC_HIP(c, hipEventRecord(c->ev_fork, c->stream));
-    MC_HIP(c, hipStreamWaitEvent(c->side, c->ev_fork, 0));
-    batch_launch(c, batch_args(c, true), true, c->side);
-    MC_LAUNCH_CHECK(c);
-    MC_HIP(c, hipEventRecord(c->ev_join, c->side));
-    return MC_OK;
-}
-
-// Join: the alternate arrays hold the batched systems (the last assembled, as
-// in the reference's order) and become the current ones; VARP's right-hand
-// side goes to S_U
-static int batch_join(Ctx *c)
-{
-    MC_HIP(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));
-    std::swap(c->A_dia, c->A_dia3);
-    std::swap(c->AV, c->AV2);
-    std::swap(c->ff0, c->ff0b);
-    std::swap(c->ff1, c->ff1b);
-    const ScalBatchArgs a = batch_args(c, true);
-    MC_TRY(batch_solves(c, a, true));
-    MC_HIP(c, hipMemcpyAsync(c->SU, c->srhs[SB - 1], (size_t)c->N * 8, hipMemcpyDeviceToDevice, c->stream));
-    return MC_OK;
 }
 
 int scalar_batch_solve(Ctx *c) { return batch_solve(c, false); }
@@ -2954,7 +2888,7 @@ int clip_nonneg(Ctx *c, double *phi, int slot)
     return MC_OK;
 }
 
-int scalar_solve(Ctx *c, int type, bool fork_batch)
+int scalar_solve(Ctx *c, int type)
 {
     const int field = scalar_field(type);
     const bool warm = warm_start(c);
@@ -2968,7 +2902,6 @@ int scalar_solve(Ctx *c, int type, bool fork_batch)
         StageTimer t(c, turb ? MC_ST_TURB_FLUX : MC_ST_SCA_FLUX);
         MC_TRY(scalar_assemble(c, type, fused ? c->r0buf[0] : nullptr));
     }
-    if (fork_batch) MC_TRY(batch_fork(c));
     StageTimer ts(c, turb ? MC_ST_TURB_SOLVE : MC_ST_SCA_SOLVE);
     double *b[1] = {c->SU};
     double *x[1] = {c->phi[field]};
@@ -3015,17 +2948,12 @@ int simple_iteration(Ctx *c, int inner)
     MC_TRY(calculate_pressure(c));
     if (c->opt.solve_scalars) {
         MC_TRY(scalar_solve(c, TERBTE));
-        // TEM, then FUL, PRO, VARF, VARP: assembled beside the ED solve when
-        // nothing is being timed
-        const bool beside = batch_beside(c);
-        const int rc = scalar_solve(c, TERBED, beside);
-        if (rc != MC_OK) {
-            // a failed ED solve returns with the batch kernel perhaps still
-            // running: later work on the main stream is ordered after it
-            if (beside && c->ev_join) (void)hipStreamWaitEvent(c->stream, c->ev_join, 0);
-            return rc;
-        }
-        MC_TRY(beside ? batch_join(c) : batch_solve(c, true));
+        MC_TRY(scalar_solve(c, TERBED));
+        // TEM, then FUL, PRO, VARF, VARP.  The assembly ran on a second stream beside
+        // the ED solve while it took 0.84 ms; as k_box_scalar_batch (0.41 ms) it held
+        // up ED's reductions by more than the overlap hid (a timestep, beside / in
+        // order, ms: modifier 64 5.53 / 5.34 mixed, 40 3.97 / 3.87, 128 20.6 / 20.5).
+        MC_TRY(batch_solve(c, true));
     }
     c->st.simple_iterations++;
     c->global_iter++;
