@@ -2920,7 +2920,7 @@ int simple_iteration(Ctx *c, int inner)
     // With the scalars solved, ff0 and ff1 of the momentum and TE / ED assembly, ff1
     // of the pressure assembly and A_V up to the batched assembly are written again
     // before anything reads them: the box kernels leave those stores out
-    // (4,194,304 cells, us: momentum 390 -> 341, TE 258 -> 217, ED 305 -> 260,
+    // (4,194,304 cells, us: momentum 390 -> 341, TE 305 -> 260, ED 258 -> 217,
     // Rhie-Chow fluxes 274 -> 258).
     struct Lean {
         Ctx *c;
