@@ -220,6 +220,7 @@ struct Ctx {
     // ---- AMG ----
     std::vector<AmgLevel> amg;
     bool amg_ready = false;
+    bool amg_box_wanted = false;   // box_wanted() when the hierarchy was built
     int amg_coarse_n = 0;
     double *amg_dense = nullptr;   // [n*n] coarsest (regularised) inverse
     double *amg_work = nullptr;

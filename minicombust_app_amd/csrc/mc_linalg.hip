@@ -1360,12 +1360,18 @@ static int amg_release(Ctx *c)
     return dfree_category(c, MC_MEM_AMG);
 }
 
+// rows up to which a level is the dense coarsest one
+static int amg_coarse_bound(const Ctx *c) { return std::max(8, std::min(c->opt.amg_coarse_max, DENSE_MAX)); }
+
+static bool box_wanted(const Ctx *c);
+
 static int amg_finish_build(Ctx *c, const double *vals)
 {
     const int nco = c->amg.back().n;
     c->amg_coarse_n = nco;
     MC_TRY(dalloc(c, &c->amg_dense, (size_t)nco * nco));
     c->amg_ready = true;
+    c->amg_box_wanted = box_wanted(c);
     c->amg_updates = 0;
     // level 0's diagonal copies were just allocated and zeroed: whatever an
     // earlier pressure assembly wrote went to the hierarchy released above
@@ -1384,14 +1390,23 @@ static int amg_finish_build(Ctx *c, const double *vals)
 // of every solve.
 constexpr double BOX_RTOL = 1e-9;
 
-// *built = false: another tolerance or form (above), not a box pattern, nothing to coarsen, or no positive
-// coupling to choose directions by (the pairwise build then decides)
+// The options' choice.  A hierarchy built for the other one is replaced before
+// the next solve (amg_current), so results depend on the options in force and
+// not on the ones before them.
+static bool box_wanted(const Ctx *c)
+{
+    return c->box_nx && c->fine_nd == 7 && c->N > amg_coarse_bound(c) && c->opt.p_rtol <= BOX_RTOL && !c->opt.limit_grad;
+}
+
+static bool amg_current(const Ctx *c) { return c->amg_ready && c->amg_box_wanted == box_wanted(c); }
+
+// *built = false: not wanted (above), or no positive coupling to choose
+// directions by (the pairwise build then decides)
 static int amg_build_box(Ctx *c, const double *vals, bool *built)
 {
     *built = false;
-    const int coarse_max = std::max(8, std::min(c->opt.amg_coarse_max, DENSE_MAX));
-    if (c->opt.p_rtol > BOX_RTOL || c->opt.limit_grad) return MC_OK;
-    if (!c->box_nx || c->fine_nd != 7 || c->N <= coarse_max) return MC_OK;
+    const int coarse_max = amg_coarse_bound(c);
+    if (!box_wanted(c)) return MC_OK;
     const int nx = c->box_nx, ny = c->box_ny, nz = c->box_nz;
     double st[3];
     {
@@ -1476,7 +1491,7 @@ static int amg_build(Ctx *c, const double *vals)
     MC_HIP(c, hipMemcpyAsync(A.val.data(), vals, (size_t)c->nnz * 8, hipMemcpyDeviceToHost, c->stream));
     MC_HIP(c, hipStreamSynchronize(c->stream));
     MC_TRY(amg_release(c));
-    const int coarse_max = std::max(8, std::min(c->opt.amg_coarse_max, DENSE_MAX));
+    const int coarse_max = amg_coarse_bound(c);
     c->graph_gen++;   // the PCG graphs hold the old levels' buffers
     HostCSR cur = std::move(A);
     bool first = true;
@@ -1593,7 +1608,7 @@ static int box_coarsen(Ctx *c, size_t l)
 
 int amg_update_values(Ctx *c, const double *vals)
 {
-    if (!c->amg_ready) return amg_setup(c, vals);
+    if (!amg_current(c)) return amg_setup(c, vals);
     MC_TRY(dense_join(c));   // the previous inverse still reads the coarsest values
     const double *vf = vals;
     // the pressure assembly wrote level 0's diagonal copies with the values
@@ -3928,7 +3943,7 @@ int pressure_solve(Ctx *c, const double *b, double *x, mc_solve_status *st, doub
     double bn0 = 0.0;
     // a state set through the C-ABI can reach a solve before any assembly
     // built the hierarchy: build it from the stored pressure matrix
-    if (!c->amg_ready) MC_TRY(amg_setup(c, c->PA_vals));
+    if (!amg_current(c)) MC_TRY(amg_setup(c, c->PA_vals));
     // learned = 2: every loop-1 solve starts from the guess; learned = 1: only
     // while its measured saving (iterations x time per iteration) exceeds its
     // cost, re-checking the other choice after 16 solves, then after twice as
