@@ -2914,6 +2914,75 @@ int scalar_solve(Ctx *c, int type)
     return MC_OK;
 }
 
+// The stores a stage's lean assembly left out, from what the stage stored and
+// its solve does not change: ff0 and ff1 of momentum, TE and ED follow from the
+// mass fluxes, A_V of TE and ED is the matrix diagonal; the pressure's ff1 is
+// ff0 and its A_V the (negative) sum over a cell's faces.
+enum { LEAN_MOM = 0, LEAN_TE = 1, LEAN_ED = 2, LEAN_PRES };   // the first three number Ctx::box.vis
+
+template <int STAGE>
+__global__ void __launch_bounds__(256) k_box_lean_restore(BoxG g, const double *mflux, const double *dia, double *ff0,
+                                                          double *ff1, double *AV)
+{
+    BoxCell q;
+    if (!box_cell(g, q)) return;
+    const int c = q.c;
+    if constexpr (STAGE == LEAN_PRES) {
+        double A = 0.0;
+        constexpr int order[6] = {0, 4, 2, 1, 3, 5};   // as k_box_mass_rows
+#pragma unroll
+        for (int k = 0; k < 6; k++) {
+            const int s = order[k];
+            if (!q.in[s]) continue;
+            const double v = ff0[q.f[s]];
+            A -= v;
+            if (s & 1) ff1[q.f[s]] = v;
+        }
+        AV[c] = A;
+    } else {
+        double area[3], vol;
+        box_areas(g, q, area, vol);
+        const bool wall = STAGE == LEAN_ED && box_wall(g, q.x[0], q.x[1], q.x[2]);
+        auto face = [&](auto tag) {
+            using TAG = decltype(tag);
+            constexpr int s = TAG::side, ax = TAG::axis;
+            const BoxFace f = box_face(g, q, area, tag);
+            const double mf = mflux[q.f[s]];
+            const double VisFace = f.vis * (f.area / f.dist);
+            double v0 = -VisFace - dmax(mf, 0.0), v1 = -VisFace + dmin(mf, 0.0);
+            if constexpr (STAGE == LEAN_ED) {
+                if (wall) v1 = 0.0;
+                if (box_wall(g, q.x[0] + (ax == 0), q.x[1] + (ax == 1), q.x[2] + (ax == 2))) v0 = 0.0;
+            }
+            ff0[q.f[s]] = v0;
+            ff1[q.f[s]] = v1;
+        };
+        if (q.in[3]) face(SideTag<3>());
+        if (q.in[5]) face(SideTag<5>());
+        if (q.in[1]) face(SideTag<1>());
+        if constexpr (STAGE != LEAN_MOM) AV[c] = dia[3 * (size_t)g.N + c];
+    }
+}
+
+// rc of a stage's solve, passed on
+static int lean_restore(Ctx *c, int stage, int rc)
+{
+    if (rc != MC_ERR_NOCONV || !c->lean || !box_on(c)) return rc;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(walk_blocks(cell_walk(c))), dim3(256), 0, c->stream,
+                           box_geo(c, stage == LEAN_PRES ? 0 : stage), c->mflux, fine_dia_of(c, c->A_vals), c->ff0,
+                           c->ff1, c->AV);
+    };
+    switch (stage) {
+    case LEAN_MOM: launch(k_box_lean_restore<LEAN_MOM>); break;
+    case LEAN_TE: launch(k_box_lean_restore<LEAN_TE>); break;
+    case LEAN_ED: launch(k_box_lean_restore<LEAN_ED>); break;
+    default: launch(k_box_lean_restore<LEAN_PRES>); break;
+    }
+    MC_LAUNCH_CHECK(c);
+    return rc;
+}
+
 // ============================================================= A17 ==
 int simple_iteration(Ctx *c, int inner)
 {
@@ -2921,7 +2990,8 @@ int simple_iteration(Ctx *c, int inner)
     // of the pressure assembly and A_V up to the batched assembly are written again
     // before anything reads them: the box kernels leave those stores out
     // (4,194,304 cells, us: momentum 390 -> 341, TE 305 -> 260, ED 258 -> 217,
-    // Rhie-Chow fluxes 274 -> 258).
+    // Rhie-Chow fluxes 274 -> 258).  An iteration that ends at a solve that did not
+    // converge makes them up (lean_restore).
     struct Lean {
         Ctx *c;
         ~Lean() { c->lean = false; }
@@ -2943,12 +3013,12 @@ int simple_iteration(Ctx *c, int inner)
     }
     {
         StageTimer t(c, MC_ST_VEL_SOLVE);
-        MC_TRY(momentum_solve(c, true));
+        MC_TRY(lean_restore(c, LEAN_MOM, momentum_solve(c, true)));
     }
-    MC_TRY(calculate_pressure(c));
+    MC_TRY(lean_restore(c, LEAN_PRES, calculate_pressure(c)));
     if (c->opt.solve_scalars) {
-        MC_TRY(scalar_solve(c, TERBTE));
-        MC_TRY(scalar_solve(c, TERBED));
+        MC_TRY(lean_restore(c, LEAN_TE, scalar_solve(c, TERBTE)));
+        MC_TRY(lean_restore(c, LEAN_ED, scalar_solve(c, TERBED)));
         // TEM, then FUL, PRO, VARF, VARP.  The assembly ran on a second stream beside
         // the ED solve while it took 0.84 ms; as k_box_scalar_batch (0.41 ms) it held
         // up ED's reductions by more than the overlap hid (a timestep, beside / in
