@@ -406,6 +406,26 @@ enum { MC_MEM_MESH = 0,   /* topology, geometry, face orders                */
        MC_MEM_COUNT };
 int  mc_ctx_memory(mc_ctx *ctx, int64_t *bytes);
 
+/* ---- inspection ------------------------------------------------------------
+   Which of its forms the context runs, for tests that compare them.  No
+   counterpart in the reference.
+   mc_forms: out[0] = 1 while the assembly takes a generated box's geometry from
+   tables, out[1] = AMG levels built, out[2] / out[3] = the one-workgroup tail
+   the last FP64 / FP32 V-cycle ended in (MC_TAIL_*).
+   mc_amg_level: out[0] = rows, out[1] = stored diagonals (0: CSR), out[2] = its
+   transfers to the next level (MC_LEVEL_*); MC_ERR_ARG beyond the last level. */
+enum { MC_TAIL_NONE = 0, MC_TAIL_DIA, MC_TAIL_MIXED, MC_TAIL_CSR };
+enum { MC_LEVEL_INDEXED = 0, /* through index arrays                          */
+       MC_LEVEL_BOX,         /* halved box level                              */
+       MC_LEVEL_REGULAR };   /* matched level that came out as a halved box   */
+int  mc_forms(mc_ctx *ctx, int64_t *out);
+int  mc_amg_level(mc_ctx *ctx, int level, int64_t *out);
+/* Takes fused passes apart into the passes whose bits they reproduce, until the
+   next call (0, the default: none).                                          */
+enum { MC_PLAIN_TRANSFERS = 1, /* MC_LEVEL_REGULAR levels through index arrays   */
+       MC_PLAIN_FINISH = 2 };  /* every reduction ends in its finishing kernel   */
+int  mc_plain_passes(mc_ctx *ctx, int which);
+
 /* ---- learned pressure-correction initial guess -------------------------- *
  * No counterpart in the reference: its pressure solves start from zero
  * (FlowSolver.inl:2203-2273, gpu/FlowSolver.inl:943-969).  A message-passing

@@ -751,6 +751,37 @@ int mc_ctx_memory(mc_ctx *x, int64_t *bytes)
     return MC_OK;
 }
 
+int mc_forms(mc_ctx *x, int64_t *out)
+{
+    CTX_OR_FAIL
+    if (!out) return MC_ERR_ARG;
+    out[0] = c->box.ok && c->fine_nd == 7;
+    out[1] = (int64_t)c->amg.size();
+    out[2] = c->tail_form[0];
+    out[3] = c->tail_form[1];
+    return MC_OK;
+}
+
+int mc_amg_level(mc_ctx *x, int level, int64_t *out)
+{
+    CTX_OR_FAIL
+    if (!out || level < 0 || level >= (int)c->amg.size()) return MC_ERR_ARG;
+    const AmgLevel &L = c->amg[level];
+    out[0] = L.n;
+    out[1] = L.nd;
+    out[2] = L.bx ? MC_LEVEL_BOX : L.rx ? MC_LEVEL_REGULAR : MC_LEVEL_INDEXED;
+    return MC_OK;
+}
+
+int mc_plain_passes(mc_ctx *x, int which)
+{
+    CTX_OR_FAIL
+    if (which & ~(MC_PLAIN_TRANSFERS | MC_PLAIN_FINISH)) return MC_ERR_ARG;
+    c->plain = which;
+    c->graph_gen++;   // the passes are baked into the PCG graphs
+    return MC_OK;
+}
+
 int mc_copy_probe(mc_ctx *x, int64_t bytes, int reps, double *ms_out)
 {
     CTX_OR_FAIL

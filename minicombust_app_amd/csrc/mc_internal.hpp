@@ -221,6 +221,8 @@ struct Ctx {
     std::vector<AmgLevel> amg;
     bool amg_ready = false;
     bool amg_box_wanted = false;   // box_wanted() when the hierarchy was built
+    int tail_form[2] = {};         // MC_TAIL_* of the last FP64 / FP32 V-cycle
+    int plain = 0;                 // MC_PLAIN_*: passes taken apart for comparison
     int amg_coarse_n = 0;
     double *amg_dense = nullptr;   // [n*n] coarsest (regularised) inverse
     double *amg_work = nullptr;

@@ -75,6 +75,9 @@ static Grid grid_csr(int n)
     return g;
 }
 
+// alpha, omega, rho and beta formed by their consumers (fold_sums)
+static bool fold_on(const Ctx *c, const Grid &g) { return g.blocks <= FOLD_BLOCKS && !(c->plain & MC_PLAIN_FINISH); }
+
 // Device scalars of one Krylov solve (NR <= 4 systems).
 struct KState {
     double rho_old[4], alpha[4], omega[4], rho[4], beta[4];
@@ -793,7 +796,7 @@ static int bicgstab_nr(Ctx *c, const double *vals, double *const *b, double *con
     const Grid g = grid_for(n);
     // short grids: alpha and omega are formed by their consumers (fold_sums);
     // a folding kernel reads one half of the partials buffer and writes the other
-    const bool fold = g.blocks <= FOLD_BLOCKS;
+    const bool fold = fold_on(c, g);
     double *red2 = fold ? c->red + RED_PARTIALS / 2 : c->red;
     if (warm && r0) {
         // the assembly formed r = b - A x0 (same x0, same matrix): it is the r vector
@@ -2958,6 +2961,7 @@ static int tail_launch(Ctx *c, size_t l, const T *b, T *x, int nu, const double 
     else if constexpr (sizeof(T) == 4)
         hipLaunchKernelGGL((k_dia_tail<5, SYM, T>), one, thr, 0, c->stream, ta, stop);
     MC_LAUNCH_CHECK(c);
+    c->tail_form[sizeof(T) == 4] = MC_TAIL_DIA;
     *done = true;
     return MC_OK;
 }
@@ -3017,16 +3021,18 @@ static int vcycle(Ctx *c, size_t l, const T *b, T *x, KState *ks, const KState *
             if (csr) hipLaunchKernelGGL(k_csr_tail<T>, dim3(1), dim3(TAIL_THREADS), 0, c->stream, ta, stop);
             else hipLaunchKernelGGL((k_vtail<SYM, T>), dim3(1), dim3(TAIL_THREADS), 0, c->stream, ta, stop);
             MC_LAUNCH_CHECK(c);
+            c->tail_form[sizeof(T) == 4] = csr ? MC_TAIL_CSR : MC_TAIL_MIXED;
             return MC_OK;
         }
     }
     if (l + 1 == c->amg.size()) {
+        c->tail_form[sizeof(T) == 4] = MC_TAIL_NONE;
         MC_TRY(dense_join(c));
         hipLaunchKernelGGL(k_dense_apply<T>, dim3(1), dim3(1024), 0, c->stream, L.n, c->amg_dense, b, x, stop);
         if (ks) {  // one-level hierarchy: no smoothing sweep carries the (r, z) reduction
             const Grid g = grid_for(L.n);
             hipLaunchKernelGGL(k_rz<T>, dim3(g.blocks), dim3(BLOCK), 0, c->stream, L.n, b, x, ks, c->red, g.chunk);
-            if (g.blocks > FOLD_BLOCKS) launch_finish<1>(c->stream, c->red, g.blocks, EpiRz{ks});
+            if (!fold_on(c, g)) launch_finish<1>(c->stream, c->red, g.blocks, EpiRz{ks});
         }
         return MC_OK;
     }
@@ -3065,7 +3071,7 @@ static int vcycle(Ctx *c, size_t l, const T *b, T *x, KState *ks, const KState *
     // below the finest level the residual and the restriction, and the
     // prolongation and the first post-smoothing sweep, share a launch
     constexpr int BND = sizeof(T) == 8 ? -7 : 7;   // the box levels' storage (level_mat)
-    const bool reg = L.rx != 0 && nd_code(A) == BND;
+    const bool reg = L.rx != 0 && nd_code(A) == BND && !(c->plain & MC_PLAIN_TRANSFERS);
     const bool box = L.bx != 0 || reg;
     const bool fuse = l >= 1 && !half;
     // below the finest level k_reg_restrict's four rows a lane pay from REG_ROWS on
@@ -3153,7 +3159,7 @@ static int vcycle(Ctx *c, size_t l, const T *b, T *x, KState *ks, const KState *
                 MC_DISPATCH_ND(nd_code(A), (k_jac<ND_, T>), dim3(g.blocks), dim3(BLOCK), 0, c->stream, A, dinv, b,
                                cur, dst, (T)wts[nu - 1 - s], g.chunk, dotv, c->red, stop);
         }
-        if (dotv && g.blocks > FOLD_BLOCKS) launch_finish<1>(c->stream, c->red, g.blocks, EpiRz{ks});
+        if (dotv && !fold_on(c, g)) launch_finish<1>(c->stream, c->red, g.blocks, EpiRz{ks});
         oth = cur;
         cur = dst;
     }
@@ -3355,7 +3361,7 @@ static int pcg_iteration(Ctx *c, const Mat<T> &A, const Grid &g, PcgVecs<T> w, T
                          double vbytes, const Pub &pub = Pub())
 {
     const int n = c->N;
-    const bool fold = g.blocks <= FOLD_BLOCKS;   // rho, beta and alpha formed by their consumers (fold_sums)
+    const bool fold = fold_on(c, g);   // rho, beta and alpha formed by their consumers (fold_sums)
     double *red2 = fold ? c->red + RED_PARTIALS / 2 : c->red;
     {
         KTimer kt(c, MC_KC_VCYCLE, c->profile ? vcycle_bytes<T>(c) : 0.0);

@@ -40,6 +40,9 @@ KC_KERNELS = {"grad11": "mc::k_box_grad<11>", "grad1": "mc::k_box_grad<1>", "mom
               "pcg_spmv32": "mc::k_pcg_pq<7, float>", "flux_correct": "mc::k_box_flux_correct",
               "scalar_batch": "mc::k_box_scalar_batch<true>", "ir_resid": "mc::k_ir_resid<-7>"}
 KC_COUNT = len(KC_NAMES)
+TAIL_NONE, TAIL_DIA, TAIL_MIXED, TAIL_CSR = range(4)           # MC_TAIL_*
+LEVEL_INDEXED, LEVEL_BOX, LEVEL_REGULAR = range(3)             # MC_LEVEL_*
+PLAIN_TRANSFERS, PLAIN_FINISH = 1, 2                           # MC_PLAIN_*
 # stages of the SIMPLE iteration (MC_ST_*)
 ST_NAMES = ["grad", "vel_flux", "vel_solve", "pres_flux", "pres_solve", "pres_correct", "turb_flux", "turb_solve",
             "sca_flux", "sca_solve"]
@@ -143,6 +146,9 @@ def lib():
         L.mc_stage_read.argtypes = [P_, C.c_void_p, C.c_void_p]
         L.mc_copy_probe.argtypes = [P_, C.c_int64, C.c_int, C.POINTER(C.c_double)]
         L.mc_ctx_memory.argtypes = [P_, C.c_void_p]
+        L.mc_forms.argtypes = [P_, C.c_void_p]
+        L.mc_amg_level.argtypes = [P_, C.c_int, C.c_void_p]
+        L.mc_plain_passes.argtypes = [P_, C.c_int]
         L.mc_mpnn_nparams.restype = C.c_int64
         L.mc_mpnn_nparams.argtypes = []
         L.mc_mpnn_load.argtypes = [P_, C.c_void_p, C.c_int64]
@@ -394,6 +400,22 @@ class Context:
         s = Stats()
         self._check(self.L.mc_get_stats(self.h, C.byref(s)), "mc_get_stats")
         return {k: getattr(s, k) for k, _ in Stats._fields_}
+
+    def forms(self):
+        """box_tables, amg_levels and the V-cycle tails (TAIL_*) in FP64 and FP32."""
+        v = np.zeros(4, dtype=np.int64)
+        self._check(self.L.mc_forms(self.h, v.ctypes.data), "mc_forms")
+        return dict(zip(("box_tables", "amg_levels", "tail64", "tail32"), v.tolist()))
+
+    def amg_level(self, level):
+        """(rows, stored diagonals or 0 for CSR, transfers LEVEL_*) of an AMG level."""
+        v = np.zeros(3, dtype=np.int64)
+        self._check(self.L.mc_amg_level(self.h, int(level), v.ctypes.data), "mc_amg_level")
+        return tuple(v.tolist())
+
+    def plain_passes(self, which):
+        """Take fused passes apart (PLAIN_TRANSFERS | PLAIN_FINISH; 0: none)."""
+        self._check(self.L.mc_plain_passes(self.h, int(which)), "mc_plain_passes")
 
     def flags(self):
         fp, ts = C.c_int(), C.c_int64()
