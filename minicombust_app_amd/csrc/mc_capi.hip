@@ -622,10 +622,10 @@ int mc_array_set(mc_ctx *x, int id, const void *host, int64_t count)
 {
     CTX_OR_FAIL
     c->pa_dia_fresh = false;   // the AMG fine level is refreshed from whatever the arrays now hold
-    if (id >= MC_ARR_FACE_AREA && id <= MC_ARR_CELL_DENSITY) c->box.ok = false;   // the caller's geometry from here on
     ArrDesc d;
     MC_TRY(describe(c, id, d));
     if (!host || count != d.count) { c->err = "array size mismatch (expected " + std::to_string(d.count) + ")"; return MC_ERR_ARG; }
+    if (id >= MC_ARR_FACE_AREA && id <= MC_ARR_CELL_DENSITY) c->box.ok = false;   // the caller's geometry from here on
     MC_HIP(c, hipStreamSynchronize(c->stream));
     if (d.face) MC_TRY(face_maps(c));
     const int *pos = d.face ? c->h_face_pos.data() : nullptr;

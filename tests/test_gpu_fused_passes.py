@@ -116,3 +116,16 @@ def test_generated_boxes_use_the_tables(m):
     print("box tables m=%d" % m, flush=True)
     with mc.Context(m) as g:
         assert g.forms()["box_tables"] == 1
+
+
+def test_refused_geometry_leaves_the_tables_in_use():
+    """A geometry array set with a wrong count is refused and changes nothing."""
+    print("refused geometry", flush=True)
+    with mc.Context(5) as g:
+        v = g.get(mc.ARR_CELL_DENSITY)
+        for n in (0, g.N - 1, g.N + 1):
+            assert g.L.mc_array_set(g.h, mc.ARR_CELL_DENSITY, v.ctypes.data, n) != mc.MC_OK
+        assert g.L.mc_array_set(g.h, mc.ARR_CELL_DENSITY, None, g.N) != mc.MC_OK
+        assert g.forms()["box_tables"] == 1
+        g.set(mc.ARR_CELL_DENSITY, v)
+        assert g.forms()["box_tables"] == 0
