@@ -1116,9 +1116,14 @@ __global__ void k_level_dia(int n, const int *rp, const int *col, const int *map
 // One CU, a chain of n steps: what counts is a step's length.  Thread t owns
 // the 4 x 4 tile at rows 4 (t / 32), columns 4 (t % 32), so a step needs four
 // values of the pivot row and four of the pivot column (64 bytes of LDS reads
-// a thread; a 1 x 16 strip needs 136), and every thread forms the pivot's
-// reciprocal itself, so one barrier a step suffices (row and column are
-// double-buffered by the step's parity).  128 rows: 240 -> 174 us.
+// a thread; a 1 x 16 strip needs 136), and the half wave that holds the pivot row
+// scales it before it is published, so one barrier a step suffices (row and
+// column are double-buffered by the step's parity).  Four pivots an iteration:
+// the pivot's place in a tile is then a constant and a step is 16 products and
+// no selection of registers (by a running index the selections were most of a
+// step, and the kernel the more slowed by others' waves on its CU).  128 rows
+// with the device idle 235 -> 70 us, beside the learned guess at modifier 128
+// 245 -> 170 us.
 //
 // The matrix: CSR, or a box level's symmetric diagonals (main, +x, +y, +z).
 struct DenseSrc {
@@ -1163,41 +1168,52 @@ __global__ void __launch_bounds__(1024) k_dense_inverse(DenseSrc src, double *in
     const double alpha = (tot / n) / n;
     double m[TQ][TQ];
 #pragma unroll
-    for (int a = 0; a < TQ; a++)
+    for (int a = 0; a < TQ; a++) {
+        const int i = i0 + a;
 #pragma unroll
-        for (int b = 0; b < TQ; b++)
-            m[a][b] = (i0 + a < n && j0 + b < n) ? alpha + dense_src_at(src, i0 + a, j0 + b) : 0.0;
-    for (int k = 0; k < n; k++) {
-        const int buf = k & 1, ka = k - i0, kb = k - j0;
-        if (ka >= 0 && ka < TQ) {
-#pragma unroll
-            for (int a = 0; a < TQ; a++)
-                if (a == ka)
-#pragma unroll
-                    for (int b = 0; b < TQ; b++) rowk[buf][j0 + b] = m[a][b];
+        for (int b = 0; b < TQ; b++) {
+            m[a][b] = (i < n && j0 + b < n) ? alpha : 0.0;
+            if (src.bx && i < n && j0 + b < n) m[a][b] += dense_src_at(src, i, j0 + b);
         }
-        if (kb >= 0 && kb < TQ) {
+        if (!src.bx && i < n)   // a CSR row is read once for its four elements
+            for (int k = src.rp[i]; k < src.rp[i + 1]; k++) {
+                const int jb = src.col[k] - j0;
+                const double v = src.v[k];
 #pragma unroll
-            for (int b = 0; b < TQ; b++)
-                if (b == kb)
-#pragma unroll
-                    for (int a = 0; a < TQ; a++) colk[buf][i0 + a] = m[a][b];
-        }
-        __syncthreads();
-        const double rk = 1.0 / rowk[buf][k];
-        double pr[TQ], pc[TQ];
-#pragma unroll
-        for (int b = 0; b < TQ; b++) pr[b] = ((b == kb) ? 1.0 : rowk[buf][j0 + b]) * rk;
-#pragma unroll
-        for (int a = 0; a < TQ; a++) pc[a] = colk[buf][i0 + a];
-#pragma unroll
-        for (int a = 0; a < TQ; a++)
-#pragma unroll
-            for (int b = 0; b < TQ; b++) {
-                const double mij = (b == kb) ? 0.0 : m[a][b];
-                m[a][b] = (a == ka) ? pr[b] : mij - pc[a] * pr[b];
+                for (int b = 0; b < TQ; b++)
+                    if (b == jb) m[a][b] += v;
             }
     }
+    const int rg = tid >> 5, cg = tid & 31;
+    for (int k0 = 0; k0 < n; k0 += TQ)
+#pragma unroll
+        for (int q = 0; q < TQ; q++) {
+            const int buf = q & 1;
+            if (k0 + q >= n) break;
+            const bool rows = rg == k0 / TQ, cols = cg == k0 / TQ;   // this tile holds row / column k0 + q
+            if (rows) {
+                // the pivot is the value of the half wave's lane k0 / 4
+                const double rk = 1.0 / __shfl(m[q][q], (tid & 32) | (k0 / TQ), 64);
+#pragma unroll
+                for (int b = 0; b < TQ; b++) rowk[buf][j0 + b] = ((cols && b == q) ? 1.0 : m[q][b]) * rk;
+            }
+            if (cols)
+#pragma unroll
+                for (int a = 0; a < TQ; a++) { colk[buf][i0 + a] = m[a][q]; m[a][q] = 0.0; }
+            __syncthreads();
+            double pr[TQ], pc[TQ];
+#pragma unroll
+            for (int b = 0; b < TQ; b++) pr[b] = rowk[buf][j0 + b];
+#pragma unroll
+            for (int a = 0; a < TQ; a++) pc[a] = colk[buf][i0 + a];
+#pragma unroll
+            for (int a = 0; a < TQ; a++)
+#pragma unroll
+                for (int b = 0; b < TQ; b++) m[a][b] = m[a][b] - pc[a] * pr[b];
+            if (rows)
+#pragma unroll
+                for (int b = 0; b < TQ; b++) m[q][b] = pr[b];
+        }
     // stored transposed: k_dense_apply's threads (rows) then read consecutive words
 #pragma unroll
     for (int a = 0; a < TQ; a++)
