@@ -68,7 +68,10 @@ typedef struct mc_options {
     double delta;          /* time step, src/minicombust.cpp:120 (1e-5)            */
     double mom_rtol;       /* BiCGStab rtol, momentum and scalars (PETSc: 1e-5)    */
     int    mom_maxit;
-    double p_rtol;         /* pressure-correction relative residual (1e-8)         */
+    double p_rtol;         /* pressure-correction relative residual (1e-8); 1e-9 and
+                              below without limit_grad, a box mesh's AMG levels are
+                              halved boxes, else matched aggregates (a change builds
+                              the other hierarchy at the next solve)             */
     int    p_maxit;
     int    amg_nu;         /* Jacobi sweeps before and after the coarse correction (3) */
     double amg_omega;      /* Jacobi damping                                       */
@@ -105,9 +108,11 @@ typedef struct mc_options {
                               7-diagonal pressure pattern with an FP16 copy of
                               D^-1 A's off-diagonals (the PCG product and the FP64
                               refinement residual keep the full matrix); 0: FP32 */
-    int    amg_tail;       /* 1: the V-cycle from the first level of at most 2048
-                              rows down runs in one workgroup (same results, fewer
-                              launches); 0: one launch per pass                  */
+    int    amg_tail;       /* 1: the V-cycle's small levels run in one workgroup (same
+                              results, fewer launches): from at most 4096 (FP64) or
+                              5120 (FP32) rows where all are in diagonal storage,
+                              1152 where all are CSR, 2304 for mixtures; 0: one
+                              launch per pass                                    */
     int    p_recycle;      /* 0-4: the last p_recycle loop-1 pressure solutions join
                               the deflation space W of the next loop-1 solve, which
                               starts from the Galerkin projection x0 = W y,
@@ -194,13 +199,14 @@ enum {
 };
 
 /* Kernel classes timed with HIP events when profiling is on.  Every class but
-   MC_KC_VCYCLE is one kernel (fine level for the solver kernels), so its
-   event time is that kernel's launch duration. */
+   MC_KC_VCYCLE and MC_KC_P_ASM (two) is one kernel (fine level for the solver
+   kernels), so its event time is that kernel's launch duration.  Assembly
+   kernels are named in their general form; a generated box runs k_box_*. */
 enum {
     MC_KC_GRAD = 0,      /* k_grad<11>: 11-field LSQ gradient                    */
     MC_KC_GRAD1,         /* k_grad<1>: 1-field LSQ gradient                      */
     MC_KC_MOM_ASM,       /* k_momentum: fluxes + sources + matrix assembly       */
-    MC_KC_P_ASM,         /* k_mass_pressure: Rhie-Chow flux + pressure assembly  */
+    MC_KC_P_ASM,         /* k_mass_faces, k_mass_rows: Rhie-Chow flux + assembly */
     MC_KC_SCALAR_ASM,    /* k_scalar: one scalar's fluxes + sources + assembly   */
     MC_KC_SPMV64,        /* k_pcg_pq<.,double>: fine PCG p-update + SpMV + dot   */
     MC_KC_SPMV32,        /* k_pcg_pq<.,float>: same, FP32 inner PCG              */
@@ -209,7 +215,7 @@ enum {
     MC_KC_MPNN,          /* learned guess: whole forward pass (work = MFMA flops) */
     MC_KC_JAC64,         /* k_jac<.,double>: fine-level Jacobi sweep             */
     MC_KC_JAC32,         /* k_jac<.,float>: fine-level Jacobi sweep              */
-    MC_KC_BICG,          /* k_bi_spmv_v: BiCGStab SpMV + (r0,v) dot              */
+    MC_KC_BICG,          /* k_bi_pv: BiCGStab SpMV + (r0,v) dot                  */
     MC_KC_SCALAR_BATCH,  /* k_scalar_batch: 4 passive scalars assembled at once  */
     MC_KC_IR_RESID,      /* k_ir_resid: FP64 residual of the refinement loop     */
     MC_KC_MPNN_BWD,      /* learned guess: whole backward pass (work = flops)     */

@@ -138,6 +138,8 @@ static Sizes sizes_of(const Ctx *c)
 // component of a normal or of a centre-to-centre vector is nonzero, so only
 // that component of a neighbour's gradient is read: the products left out are
 // signed zeros for finite operands and leave sums that start at +0 unchanged.
+// (A NaN or infinity reaches more cells in the general kernels; a cell's own
+// gradient enters its row with all components in both, so the solve fails in both.)
 // Faces are visited in ascending reference id as everywhere (low z, y, x of
 // interior faces, then the cell's own in side order with low boundary faces at
 // their sides' places), so the results are the general kernels' bit for bit.

@@ -1368,7 +1368,7 @@ static int level_vectors(Ctx *c, AmgLevel &L)
     return MC_OK;
 }
 
-// a hierarchy rebuilt (e.g. after amg_coarse_max changed) first releases the
+// a hierarchy rebuilt (after a change of options) first releases the
 // old one: every allocation charged to MC_MEM_AMG is made by its build
 static int amg_release(Ctx *c)
 {
@@ -2203,6 +2203,9 @@ __global__ void __launch_bounds__(TAIL_THREADS) k_vtail(VtArgs<T> a, const KStat
 // 73): k_vtail 47 us, this 31; ten timesteps 67.2 -> 62.1 ms.  A thread per row
 // (two rows of sixteen entries) needs the eight partial sums in registers too and
 // spills: 80 us.
+// CT_ROWS: nine rows a thread.  CT_SUM: what 160 KB of LDS hold beside the nine
+// rows' partial sums.  CT_NC: aggregates of eight give 144 of 1,152 rows; beyond a
+// third the matching has failed to shrink the level and nothing was measured.
 constexpr int CT_ROWS = 1152, CT_NC = 384, CT_SUM = 2048;
 
 template <typename T>
@@ -2462,7 +2465,8 @@ __global__ void __launch_bounds__(BLOCK) k_resid_h(HMat H, const float *b, const
 }
 
 // ------------------------------------------------- box level passes --
-// n / d for 0 <= n < 2^31 by multiply and shift (d >= 1)
+// n / d for 0 <= n < 2^31 by multiply and shift (d >= 1): Granlund and
+// Montgomery, Division by Invariant Integers using Multiplication, 1994
 struct FastDiv {
     unsigned d, mul, sh;
 };

@@ -19,7 +19,7 @@
 //
 // The edge MLP's second linear layer is applied after the neighbour sum
 // (sum_j W2 r_ij = W2 sum_j r_ij), so every matrix product is node-level: an
-// N x K by K x M product on MFMA (v_mfma_f32_16x16x16_bf16: BF16 operands,
+// N x K by K x M product on MFMA (v_mfma_f32_16x16x32_bf16: BF16 operands,
 // FP32 accumulation).  Edge work is a 64-channel gather; the backward pass
 // turns the scatters into gathers through the reverse-slot map (the graph is
 // symmetric), so nothing uses atomics.  Weight gradients are block partial
