@@ -22,18 +22,18 @@ def _solve(g):
     return x.copy(), st.iterations
 
 
-@pytest.mark.parametrize("psolve", [mc.PSOLVE_FP64, mc.PSOLVE_MIXED])
+@pytest.mark.parametrize("psolve,graph", [(mc.PSOLVE_FP64, 0), (mc.PSOLVE_MIXED, 0), (mc.PSOLVE_FP64, 1)])
 @pytest.mark.parametrize("before,after", [
     (dict(p_rtol=1e-8), dict(p_rtol=1e-10)),
     (dict(p_rtol=1e-10), dict(p_rtol=1e-8)),
     (dict(p_rtol=1e-10, limit_grad=0), dict(p_rtol=1e-10, limit_grad=1)),
     (dict(p_rtol=1e-10, limit_grad=1), dict(p_rtol=1e-10, limit_grad=0)),
 ])
-def test_hierarchy_follows_the_options(before, after, psolve):
-    print("hierarchy %s -> %s psolve=%d" % (before, after, psolve), flush=True)
-    with mc.Context(9, mode=mc.MODE_SIMPLE, psolve=psolve, **after) as g:
+def test_hierarchy_follows_the_options(before, after, psolve, graph):
+    print("hierarchy %s -> %s psolve=%d graph=%d" % (before, after, psolve, graph), flush=True)
+    with mc.Context(9, mode=mc.MODE_SIMPLE, psolve=psolve, pcg_graph=graph, **after) as g:
         want, its = _solve(g)
-    with mc.Context(9, mode=mc.MODE_SIMPLE, psolve=psolve, **before) as g:
+    with mc.Context(9, mode=mc.MODE_SIMPLE, psolve=psolve, pcg_graph=graph, **before) as g:
         _solve(g)
         g.set_options(**after)
         got, n = _solve(g)
