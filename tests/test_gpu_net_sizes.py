@@ -1,0 +1,47 @@
+"""GPU test of the net's training products and their gradient reductions at
+sizes that leave remainders: one 16-row tile (m = 2), a tail of 6 rows (3), two
+workgroups of weight-gradient products (5), many (9), and more rows than one
+tile a wave (34: 78,608 cells, above 65,536).
+
+Bounds as in test_gpu_zlearned.py: the oracle's backward rounds no operand to
+BF16 (about 2^-9 of a value each, some twelve products deep), so a parameter
+block may be off by 6 % of its norm; a lost tile or workgroup is off by more."""
+import numpy as np
+import pytest
+
+from minicombust_app_amd import mcflow as mc
+from oracle import mpnn_ref as mr
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m", [2, 3, 5, 9, 34])
+def test_gradient_sizes(m):
+    print("mpnn gradient m=%d" % m, flush=True)
+    rng = np.random.default_rng(3)
+    w = (mr.init_params(5) + 0.02 * rng.standard_normal(mr.N_PARAMS)).astype(np.float32)
+    with mc.Context(m, mode=mc.MODE_SIMPLE, p_rtol=1e-8) as ctx:
+        ctx.mpnn_load(w)
+        ctx.mpnn_collect(1)
+        ctx.simple_iteration(0)
+        assert ctx.mpnn_dataset_size() == 1
+        f, e, t = ctx.mpnn_pair(0)
+        nb = ctx.get(mc.ARR_CELL_NEIGHBOURS).reshape(ctx.N, 6)
+        nbr = np.where(nb == np.uint64(0xFFFFFFFFFFFFFFFF), -1, nb.astype(np.int64)).astype(np.int64)
+        got, loss = ctx.mpnn_grad(0)
+        again, _ = ctx.mpnn_grad(0)
+    assert np.array_equal(got, again)   # fixed summation order
+    w64 = w.astype(np.float64)
+    y, cache = mr.forward(w64, f, nbr, e, bf16_ops=True)
+    loss_ref, dy = mr.loss_and_dy(y.astype(np.float64), t.astype(np.float64))
+    want = mr.backward(w64, cache, dy)
+    assert abs(loss - loss_ref) <= 2e-2 * abs(loss_ref)
+    at = 0
+    for name, shape in mr.PARAM_SHAPES:
+        n = int(np.prod(shape))
+        a, b = got[at:at + n].astype(np.float64), want[at:at + n]
+        at += n
+        if np.linalg.norm(b) >= 1e-6 * np.linalg.norm(want):
+            rel = np.linalg.norm(a - b) / np.linalg.norm(b)
+            print("  %s %.2e" % (name, rel), flush=True)
+            assert rel <= 6e-2, (name, rel)
