@@ -5,7 +5,8 @@ tile a wave (34: 78,608 cells, above 65,536).
 
 Bounds as in test_gpu_zlearned.py: the oracle's backward rounds no operand to
 BF16 (about 2^-9 of a value each, some twelve products deep), so a parameter
-block may be off by 6 % of its norm; a lost tile or workgroup is off by more."""
+block may be off by 6 % of its norm (8.2e-3 is the largest measured); a lost tile
+or workgroup is off by more."""
 import numpy as np
 import pytest
 
